@@ -51,9 +51,7 @@ size_t chunk_ws_bytes(int B, int T, int H, int K, int V, int dtype, int parts, C
     ws.Gc = static_cast<float*>(take(BH * NT * CH_TOKENS * 4));
   }
   if (parts & WS_STATE) {
-    // states of every hstride-th chunk of each swept sequence (a segment when ns > 1; segments hold whole pairs)
-    const size_t nts = ns > 1 ? NT / ns : NT;
-    ws.hs = take(BH * (size_t)(ns > 1 ? ns : 1) * ((nts + hstride - 1) / hstride) * (size_t)K * V * es);
+    ws.hs = take(BH * ((NT + hstride - 1) / hstride) * (size_t)K * V * es);  // every hstride-th chunk's state
     ws.Rs = take(BH * NT * CH_TOKENS * (size_t)V * es);
   }
   if (parts & WS_GRAD) {
@@ -90,18 +88,48 @@ size_t chunk_ws_bytes(int B, int T, int H, int K, int V, int dtype, int parts, C
   return off;
 }
 
-int segment_count(int B, int T, int H, int K, int V) {
-  (void)K;
-  if (T <= 0 || T % CH_TOKENS) return 1;
-  const int NT = T / CH_TOKENS;
-  const int64_t blocks = (int64_t)(V / 64) * B * H;  // sweep workgroups of the unsegmented problem
-  const int cus = device_cu_count();
-  int ns = 1;
-  // double the segments while the sweeps still fit on the device and each segment keeps >= 16 chunks
-  while (blocks * ns * 2 <= cus && NT % (2 * ns) == 0 && NT / (2 * ns) >= 16) ns *= 2;
-  // the prefix pass and the scan cost about one and a half sweeps of a segment: below four segments they
-  // cost more than the parallelism gains
-  return ns >= 4 ? ns : 1;
+// Time of a segmented (ns > 1) or unsegmented call in microseconds, the forward counted twice (it also runs alone), the
+// kernels that do not depend on the segments left out.  Measured at K = 128 in bf16, a sweep over c chunks takes about
+// 6 + 2.15 c (forward), 6 + 2.4 c (reverse) and 6 + 2.05 c (local reverse) with at most one 32-column workgroup per CU,
+// 6 + 2.9 c, 6 + 3.2 c and 6 + 2.7 c with one 64-column workgroup per CU, and the prefix pass (neither Q nor O) 6 + 1.65 c;
+// workgroups past one per CU run in further rounds.  A step of the scan takes 2.4 at K = 128 and 0.8 at K = 64.
+static float segment_cost(int64_t BH, int NT, int K, int V, int ns, int cps) {
+  const int64_t cus = device_cu_count();
+  auto sweep = [&](int64_t wide, float narrow_us, float wide_us) {  // wide: workgroups of 64 columns
+    if (2 * wide <= cus) return 6.f + narrow_us * cps;
+    return (float)((wide + cus - 1) / cus) * (6.f + wide_us * cps);
+  };
+  const int64_t wv = V / 64, wk = K / 64;
+  float t = 2.f * sweep(BH * wv * ns, 2.15f, 2.9f) + sweep(BH * wv * ns, 2.4f, 3.2f);
+  if (ns > 1) {
+    const float scan = 4.f + (K == 64 ? 0.8f : 2.4f) * (ns - 1);
+    const int64_t live = BH * (wv * (ns - 1) + wk * (ns - 2));  // the prefix pass's workgroups that do any work
+    t += 2.f * (sweep(live, 1.65f, 1.65f) + scan) + sweep(BH * wv * (ns - 1), 2.05f, 2.7f) + scan;
+  }
+  return t;
+}
+
+SegPlan segment_plan(int B, int T, int H, int K, int V) {
+  const int NT = (int)(((int64_t)T + CH_TOKENS - 1) / CH_TOKENS);
+  const int64_t BH = (int64_t)B * H, wide = BH * (V / 64);
+  SegPlan best{1, NT};
+  // Measured (forward / training pair, us): B1 T6007 H8 K128 V256 206 / 471 unsegmented, 110 / 284 in 6 segments; B1
+  // T4096 H1 K128 V128 140 / 282, 63 / 136 in 11; B1 T2048 H16 K128 V256 78 / 203, 70 / 184 in 4 (86 / 220 in 2).
+  // at least four segments (with two or three the prefix pass, half or a third of a sweep, costs what the
+  // parallelism gains) of at least four chunks, no more than the device sweeps at once; whole pairs of chunks, so
+  // that a state kept for every second chunk is one of its segment's own
+  if (NT < 16 || wide <= 0 || wide * 4 > device_cu_count()) return best;
+  float t_best = 0.92f * segment_cost(BH, NT, K, V, 1, NT);  // a predicted gain below 8% is left
+  for (int cps = 4; 4 * cps <= NT + 3; cps += 2) {
+    const int ns = (NT + cps - 1) / cps;
+    if (ns < 4 || wide * ns > device_cu_count()) continue;
+    const float t = segment_cost(BH, NT, K, V, ns, cps);
+    if (t < t_best) {
+      t_best = t;
+      best = SegPlan{ns, cps};
+    }
+  }
+  return best;
 }
 
 int device_cu_count() {
@@ -117,7 +145,7 @@ int device_cu_count() {
 
 bool narrow_sweep_blocks(const ChunkArgs& a, int blocks_per_head) {
   // only when the narrow workgroups all run at once, one per CU (two per CU were measured slower than one wide)
-  return (int64_t)blocks_per_head * a.B * a.H <= (int64_t)device_cu_count();
+  return (int64_t)blocks_per_head * a.B * a.ns * a.H <= (int64_t)device_cu_count();
 }
 
 bool chunk_shape_supported(int K, int V, int dtype) {
@@ -280,7 +308,7 @@ int gdn_chunk_fwd_ws_bytes(int B, int T, int H, int K, int V, int dtype, size_t*
   g_err[0] = 0;
   if (int e = check_common(B, T, H, K, V, dtype)) return e;
   if (!bytes) return fail(GDN_ERR_ARG, "bytes is NULL");
-  *bytes = chunk_ws_bytes(B, T, H, K, V, dtype, WS_FACT | WS_SEGF, nullptr, nullptr, segment_count(B, T, H, K, V), 1);
+  *bytes = chunk_ws_bytes(B, T, H, K, V, dtype, WS_FACT | WS_SEGF, nullptr, nullptr, segment_plan(B, T, H, K, V).ns, 1);
   return GDN_OK;
 }
 
@@ -289,7 +317,7 @@ int gdn_chunk_bwd_ws_bytes(int B, int T, int H, int K, int V, int dtype, size_t*
   if (int e = check_common(B, T, H, K, V, dtype)) return e;
   if (!bytes) return fail(GDN_ERR_ARG, "bytes is NULL");
   *bytes = chunk_ws_bytes(B, T, H, K, V, dtype, WS_FACT | WS_STATE | WS_GRAD | WS_SEGF | WS_SEGB, nullptr, nullptr,
-                          segment_count(B, T, H, K, V), state_stride(V, dtype, false));
+                          segment_plan(B, T, H, K, V).ns, state_stride(V, dtype, false));
   return GDN_OK;
 }
 
@@ -298,7 +326,7 @@ static int stash_sizes(int B, int T, int H, int K, int V, int dtype, bool sepu, 
   g_err[0] = 0;
   if (int e = check_common(B, T, H, K, V, dtype)) return e;
   if (!stash_bytes || !bwd_ws_bytes) return fail(GDN_ERR_ARG, "stash_bytes or bwd_ws_bytes is NULL");
-  const int ns = segment_count(B, T, H, K, V), hs = state_stride(V, dtype, sepu);
+  const int ns = segment_plan(B, T, H, K, V).ns, hs = state_stride(V, dtype, sepu);
   *stash_bytes = chunk_ws_bytes(B, T, H, K, V, dtype, WS_STASH, nullptr, nullptr, ns, hs);
   *bwd_ws_bytes = chunk_ws_bytes(B, T, H, K, V, dtype, WS_GRAD | WS_SEGB, nullptr, nullptr, ns, hs);
   return GDN_OK;
@@ -318,22 +346,20 @@ int gdn_nsgdn_stash_bytes(int B, int T, int H, int K, int V, int dtype, size_t* 
 
 namespace gdn {
 
-// Segmented forward, after the chunk factors of the segmented problem `a` (B*ns sequences of T/ns tokens):
-// the prefix pass (each segment's state from zero -- the first from h0 -- and the transitions of the middle
-// segments), the scan across segments (the state entering each segment), and `a` set up for the main sweep to
-// start every segment from its entering state (it writes hT, from each sequence's last segment).
-static hipError_t seg_forward_prefix(ChunkArgs& a, const float* h0, int B, int ns) {
+// Segmented forward, after the chunk factors: the prefix pass (each segment's state from zero -- the first from h0 --
+// and the transitions of the middle segments), the scan across segments (the state entering each segment), and `a`
+// set up for the main sweep to start every segment from its entering state (it writes hT, from each sequence's last
+// segment).
+static hipError_t seg_forward_prefix(ChunkArgs& a, const float* h0) {
   ChunkArgs p = a;
   p.h0 = h0;
   p.hT = a.ws.sloc;
-  p.ns = ns;
   hipError_t e = timed(ST_PREFIX, a.stream, [&] { return launch_fwd(p, FWD_PREFIX); });
   if (e == hipSuccess)
     e = timed(ST_SEGSCAN, a.stream, [&] {
-      return launch_seg_scan(a.ws.phi, a.ws.sloc, h0, a.ws.sin, nullptr, B, ns, a.H, a.K, a.V, false, a.stream);
+      return launch_seg_scan(a.ws.phi, a.ws.sloc, h0, a.ws.sin, a.B, a.ns, a.H, a.K, a.V, false, a.stream);
     });
   a.h0 = a.ws.sin;
-  a.ns = ns;
   return e;
 }
 
@@ -359,18 +385,19 @@ static int chunk_fwd_impl(const void* q, const void* k, const void* u, const voi
   if (misaligned(q, k, u, v, g, beta, h0, o, hT, ws))
     return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
   ChunkArgs a{};
-  const int ns = segments ? segment_count(B, T, H, K, V) : 1;
+  const SegPlan seg = segments ? segment_plan(B, T, H, K, V) : SegPlan{1, (T + CH_TOKENS - 1) / CH_TOKENS};
   a.hstride = state_stride(V, dtype, u != nullptr);
-  const size_t need = chunk_ws_bytes(B, T, H, K, V, dtype, stash ? WS_STASH : (WS_FACT | WS_SEGF), &a.ws, ws, ns,
+  const size_t need = chunk_ws_bytes(B, T, H, K, V, dtype, stash ? WS_STASH : (WS_FACT | WS_SEGF), &a.ws, ws, seg.ns,
                                      a.hstride);
   if (!ws || ws_bytes < need)
     return fail(GDN_ERR_WORKSPACE, "%s of %zu bytes needed, %zu given", stash ? "stash" : "workspace", need,
                 ws ? ws_bytes : (size_t)0);
   a.q = q; a.k = k; a.u = u; a.v = v; a.g = g; a.beta = beta; a.h0 = h0; a.o = o; a.hT = hT;
-  a.B = B * ns; a.T = T / ns; a.H = H; a.K = K; a.V = V; a.NT = (a.T + CH_TOKENS - 1) / CH_TOKENS;
+  a.B = B; a.T = T; a.H = H; a.K = K; a.V = V; a.NT = (T + CH_TOKENS - 1) / CH_TOKENS;
+  a.ns = seg.ns; a.cps = seg.cps;
   a.scale = scale; a.dtype = dtype; a.stream = st;
   hipError_t e = timed(ST_FACTORS, st, [&] { return launch_factors(a); });
-  if (e == hipSuccess && ns > 1) e = seg_forward_prefix(a, h0, B, ns);
+  if (e == hipSuccess && a.ns > 1) e = seg_forward_prefix(a, h0);
   if (e == hipSuccess)
     e = stash ? timed(ST_FWD_STASH, st, [&] { return launch_fwd(a, FWD_STASH); })
               : timed(ST_FWD, st, [&] { return launch_fwd(a, FWD_OUT); });
@@ -403,33 +430,34 @@ static int chunk_bwd_impl(const void* q, const void* k, const void* u, const voi
   if (misaligned(q, k, u, v, g, beta, h0, dout, dhT, dq, dk, du, dv, dg, dbeta, dh0, stash, ws))
     return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
   ChunkArgs a{};
-  const int ns = segment_count(B, T, H, K, V);  // as the forward that filled the stash chose
+  const SegPlan seg = segment_plan(B, T, H, K, V);  // as the forward that filled the stash chose
   a.hstride = state_stride(V, dtype, u != nullptr);
   if (stashed) {
     // the stash is only read (the kernels take it through the same carve-up as the recompute path's workspace)
-    const size_t sneed = chunk_ws_bytes(B, T, H, K, V, dtype, WS_STASH, &a.ws, const_cast<void*>(stash), ns,
+    const size_t sneed = chunk_ws_bytes(B, T, H, K, V, dtype, WS_STASH, &a.ws, const_cast<void*>(stash), seg.ns,
                                         a.hstride);
     if (!stash || stash_bytes < sneed)
       return fail(GDN_ERR_WORKSPACE, "stash of %zu bytes needed, %zu given", sneed,
                   stash ? stash_bytes : (size_t)0);
   }
   const int parts = stashed ? (WS_GRAD | WS_SEGB) : (WS_FACT | WS_STATE | WS_GRAD | WS_SEGF | WS_SEGB);
-  const size_t need = chunk_ws_bytes(B, T, H, K, V, dtype, parts, &a.ws, ws, ns, a.hstride);
+  const size_t need = chunk_ws_bytes(B, T, H, K, V, dtype, parts, &a.ws, ws, seg.ns, a.hstride);
   if (!ws || ws_bytes < need)
     return fail(GDN_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, ws ? ws_bytes : (size_t)0);
   a.q = q; a.k = k; a.u = u; a.v = v; a.g = g; a.beta = beta; a.h0 = h0;
   a.dout = dout; a.dhT = dhT; a.dq = dq; a.dk = dk; a.du = du; a.dv = dv; a.dg = dg; a.dbeta = dbeta; a.dh0 = dh0;
-  a.B = B * ns; a.T = T / ns; a.H = H; a.K = K; a.V = V; a.NT = (a.T + CH_TOKENS - 1) / CH_TOKENS;
+  a.B = B; a.T = T; a.H = H; a.K = K; a.V = V; a.NT = (T + CH_TOKENS - 1) / CH_TOKENS;
+  a.ns = seg.ns; a.cps = seg.cps;
   a.scale = scale; a.dtype = dtype; a.stream = st;
   hipError_t e = hipSuccess;
   if (!stashed) {
     e = timed(ST_FACTORS, st, [&] { return launch_factors(a); });
     ChunkArgs f = a;
     f.hT = nullptr;
-    if (e == hipSuccess && ns > 1) e = seg_forward_prefix(f, h0, B, ns);
+    if (e == hipSuccess && a.ns > 1) e = seg_forward_prefix(f, h0);
     if (e == hipSuccess) e = timed(ST_BWD_RECOMP, st, [&] { return launch_fwd(f, FWD_RECOMPUTE); });
   }
-  if (e == hipSuccess && ns > 1) {
+  if (e == hipSuccess && a.ns > 1) {
     // local reverse pass (each segment's entering-state gradient from a zero leaving gradient -- the last from
     // dhT; not the first segment's, which only dh0 would need), then the scan backwards across segments: the
     // gradient w.r.t. the state leaving each segment.  The main reverse sweep then writes dh0 from each
@@ -437,14 +465,12 @@ static int chunk_bwd_impl(const void* q, const void* k, const void* u, const voi
     ChunkArgs l = a;
     l.dhT = dhT;
     l.dh0 = a.ws.dsloc;
-    l.ns = ns;
     e = timed(ST_BWD_LOCAL, st, [&] { return launch_bwd_state(l, true); });
     if (e == hipSuccess)
       e = timed(ST_SEGSCAN, st, [&] {
-        return launch_seg_scan(a.ws.phi, a.ws.dsloc, dhT, a.ws.dsend, nullptr, B, ns, H, K, V, true, st);
+        return launch_seg_scan(a.ws.phi, a.ws.dsloc, dhT, a.ws.dsend, B, a.ns, H, K, V, true, st);
       });
     a.dhT = a.ws.dsend;
-    a.ns = ns;
   }
   if (e == hipSuccess) e = timed(ST_BWD_STATE, st, [&] { return launch_bwd_state(a, false); });
   if (e == hipSuccess) e = timed(ST_BWD_INTRA, st, [&] { return launch_bwd_intra(a); });

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
     const float* __restrict__ beta,
     const T* __restrict__ gTm, const T* __restrict__ gP, const float* __restrict__ gGc,
     const float* __restrict__ dhT, float* __restrict__ dh0, T* __restrict__ wsdH, T* __restrict__ wsdY, int T_,
-    int H, int V, int NT, float scale, int ns) {
+    int H, int V, int NT, float scale, int ns, int cps) {
   constexpr int PT = 16 / sizeof(T);
   constexpr int LK = K + PT, LC = CH + PT, LV = BV + PT;
   constexpr int NKH = K / 32;     // row tiles of dS per half
@@ -76,17 +76,20 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
 
   int vb, bh;
   sweep_block(V / BV, gridDim.x * BV / V, vb, bh);
-  const int b = bh / H, h = bh - b * H;
-  const int seg = b % ns;  // segment of sequence b / ns (ns = 1: not segmented)
+  // sequence b, segment seg, head h; the segment's chunks c_first .. c_end - 1 of the sequence (as in the forward sweep)
+  const int bs = bh / H, h = bh - bs * H;
+  const int b = bs / ns, seg = bs - b * ns;
+  const int c_first = seg * cps, c_end = min(NT, c_first + cps);
+  const int64_t seq = (int64_t)b * H + h;
   // The local pass of a segmented sweep (STORE = false) skips each sequence's first segment (its entering-state
   // gradient is the main sweep's dh0) and starts the last from the sequence's dhT, so that its result already
   // carries dhT.  dh0: per swept sequence in the local pass; otherwise, when segmented, only from the first
   // segment of each sequence, at the sequence's index.  dhT: per swept sequence in the main pass.
   if (!STORE && seg == 0) return;  // uniform over the workgroup, before any barrier
   const bool put_dh0 = !STORE || seg == 0;
-  const int64_t dh0_base = (!STORE ? (int64_t)bh : (int64_t)(b / ns) * H + h) * K * V;
+  const int64_t dh0_base = (!STORE ? (int64_t)bh : seq) * K * V;
   const bool use_dhT = dhT && (STORE || seg == ns - 1);
-  const int64_t dhT_base = (STORE ? (int64_t)bh : (int64_t)(b / ns) * H + h) * K * V;
+  const int64_t dhT_base = (STORE ? (int64_t)bh : seq) * K * V;
   const int v0 = vb * BV;
   const int w = wave_id(), l = lane_id();
   const int ws = w & (NSL - 1), hf = w / NSL;  // column slab; half of dS's rows and of the chunk's tokens
@@ -117,7 +120,7 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
     }
   };
   auto prefetch2 = [&](int c) {
-    const int64_t row0 = row0_of(c), cidx = (int64_t)bh * NT + c;
+    const int64_t row0 = row0_of(c), cidx = seq * NT + c;
     const int nv = nvalid_of(c);
     rtm.load(gTm + cidx * CH_TRI_ELEMS, tid);
     rp.load(gP + cidx * CH_TRI_ELEMS, tid);
@@ -135,7 +138,7 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
       dS[t][i] = use_dhT ? dhT[dhT_base + (int64_t)(k0 + 16 * t + acc_row(i)) * V + v0 + c0 + acc_col()] : 0.f;
 
   auto chunk = [&](int c) {
-    const int64_t cidx = (int64_t)bh * NT + c;
+    const int64_t cidx = seq * NT + c;
     rk.store(sK, LK, tid);
     if constexpr (SEPU) ru.store(sU, LK, tid);
     rq.store(sQ, LK, tid);
@@ -149,7 +152,7 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
       sBGn[l] = -pB * gam;
     }
     __syncthreads();
-    if (c > 0) prefetch(c - 1, 1);
+    if (c > c_first) prefetch(c - 1, 1);
 
     // dS leaving the chunk -> dh (fragment layout); partial U dS over this half's rows, for all tokens
     F dSb[NSH];
@@ -179,7 +182,7 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
       for (int e = 0; e < 8; ++e) dOg[ib][e] = from_f<T>(to_f(dOb[ib][e]) * sGam[32 * ib + 8 * (l >> 4) + e]);
     }
     __syncthreads();
-    if (c > 0) prefetch(c - 1, 2);
+    if (c > c_first) prefetch(c - 1, 2);
     // dR (this half's token rows) = diag(exp(G_C - G)) K dS + P^T dO
     f32x4 dR[2];
 #pragma unroll
@@ -196,7 +199,7 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
     const F dRmine = frag_acc2<T>(dR[0], dR[1]);
     xR[w][l] = dRmine;
     __syncthreads();
-    if (c > 0) prefetch2(c - 1);
+    if (c > c_first) prefetch2(c - 1);
     const F dRother = xR[w ^ NSL][l];
     f32x4 Z[2];
 #pragma unroll
@@ -236,9 +239,9 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
   // read by the first chunk's first barrier
   tri_zero_upper<T, STH>(sTm, LC, tid);
   tri_zero_upper<T, STH>(sP, LC, tid);
-  prefetch(NT - 1, 0);
-  prefetch2(NT - 1);
-  for (int c = NT - 1; c >= 0; --c) chunk(c);
+  prefetch(c_end - 1, 0);
+  prefetch2(c_end - 1);
+  for (int c = c_end - 1; c >= c_first; --c) chunk(c);
   if (dh0 && put_dh0) {
 #pragma unroll
     for (int t = 0; t < NKH; ++t)
@@ -742,13 +745,13 @@ __global__ __launch_bounds__(ITH) void bwd_intra_kernel(
 // ---------------------------------------------------------------------------------------------------------
 template <typename T, int K, bool SEPU, int BV>
 static hipError_t bwd_state_bv(const ChunkArgs& a, bool local) {
-  dim3 grid(a.V / BV * a.B * a.H);
+  dim3 grid(a.V / BV * a.B * a.ns * a.H);
   auto go = [&](auto kern) {
     kern<<<grid, state_threads<BV>(), 0, a.stream>>>(
         static_cast<const T*>(a.q), static_cast<const T*>(a.k), static_cast<const T*>(a.u),
         static_cast<const T*>(a.dout), a.beta, static_cast<const T*>(a.ws.Tm), static_cast<const T*>(a.ws.P),
         a.ws.Gc, a.dhT, a.dh0, static_cast<T*>(a.ws.dhs), static_cast<T*>(a.ws.dYs), a.T, a.H, a.V, a.NT,
-        a.scale, a.ns);
+        a.scale, a.ns, a.cps);
     return hipGetLastError();
   };
   return local ? go(bwd_state_kernel<T, K, BV, SEPU, false>) : go(bwd_state_kernel<T, K, BV, SEPU, true>);

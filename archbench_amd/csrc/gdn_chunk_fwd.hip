@@ -43,7 +43,8 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
     const float* __restrict__ beta,
     const float* __restrict__ h0, const T* __restrict__ gTm, const T* __restrict__ gP,
     const float* __restrict__ gGc, T* __restrict__ o, float* __restrict__ hT, float* __restrict__ phi,
-    T* __restrict__ wsH, T* __restrict__ wsR, int T_, int H, int V, int NT, float scale, int ns, int hstride) {
+    T* __restrict__ wsH, T* __restrict__ wsR, int T_, int H, int V, int NT, float scale, int ns, int cps,
+    int hstride) {
   constexpr int PT = 16 / sizeof(T);
   constexpr int LK = K + PT, LC = CH + PT, LV = BV + PT;
   constexpr int NKT = K / 16;  // row tiles of the state slab
@@ -78,12 +79,17 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
   int vb, bh;
   const int NVB = (V + (MODE == 3 ? K : 0)) / BV;  // column blocks per head
   sweep_block(NVB, gridDim.x / NVB, vb, bh);
-  const int b = bh / H, h = bh - b * H;
+  // bh counts the segments of every head: sequence b, segment seg (of ns; ns = 1: not segmented), head h.  The
+  // segment covers the sequence's chunks c_first .. c_end - 1 (cps each, the last segment possibly fewer); chunk c of
+  // the sequence keeps its place in the per-chunk buffers, [B H][NT], whatever the segments
+  const int bs = bh / H, h = bh - bs * H;
+  const int b = bs / ns, seg = bs - b * ns;
+  const int c_first = seg * cps, c_end = min(NT, c_first + cps);
+  const int64_t seq = (int64_t)b * H + h;
   // identity block (MODE 3): columns iv0 .. iv0 + BV - 1 of the transition; v reads nothing (no valid rows)
   const bool ident = MODE == 3 && vb * BV >= V;
   const int iv0 = vb * BV - V;
   const int v0 = ident ? 0 : vb * BV;
-  const int seg = b % ns;  // segment of sequence b / ns (ns = 1: not segmented)
   if constexpr (MODE == 3) {
     if (seg == ns - 1 || (ident && seg == 0)) return;  // uniform over the workgroup, before any barrier
   }
@@ -91,9 +97,9 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
   // segment of each sequence, at the sequence's index.  h0: in MODE 3 the sequence's own, for its first segment
   // only; otherwise per swept sequence (the entering state of every segment).
   const bool put_hT = MODE == 3 || seg == ns - 1;
-  const int64_t hT_base = (MODE == 3 ? (int64_t)bh : (int64_t)(b / ns) * H + h) * K * V;
+  const int64_t hT_base = (MODE == 3 ? (int64_t)bh : seq) * K * V;
   const bool use_h0 = h0 && (MODE != 3 || seg == 0);
-  const int64_t h0_base = (MODE == 3 ? (int64_t)(b / ns) * H + h : (int64_t)bh) * K * V;
+  const int64_t h0_base = (MODE == 3 ? seq : (int64_t)bh) * K * V;
   const int w = wave_id(), l = lane_id();
   const int ws = w & (NSL - 1), hf = w / NSL;        // column slab, token half
   const int c0 = 16 * ws;                             // the slab inside the V block
@@ -117,7 +123,7 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
     rv.load(v + row0 * V + v0, (int64_t)H * V, ident ? 0 : nv, tid);
   };
   auto prefetch2 = [&](int c) {
-    const int64_t row0 = row0_of(c), cidx = (int64_t)bh * NT + c;
+    const int64_t row0 = row0_of(c), cidx = seq * NT + c;
     const int nv = nvalid_of(c);
     rtm.load(gTm + cidx * CH_TRI_ELEMS, tid);
     if constexpr (OUT) rp.load(gP + cidx * CH_TRI_ELEMS, tid);
@@ -161,10 +167,10 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
   };
 
   auto chunk = [&](int c) {
-    const int64_t cidx = (int64_t)bh * NT + c;
+    const int64_t cidx = seq * NT + c;
     to_lds();
     __syncthreads();
-    if (c + 1 < NT) prefetch(c + 1);
+    if (c + 1 < c_end) prefetch(c + 1);
 
     // rows 32 hf .. 32 hf + 31: K S, Q S and Y = diag(beta) (V - diag(gamma) K S); the state's fragments are the
     // wave's own and, for the other half of the K rows, the partner's from xS (written before the last barrier).
@@ -177,7 +183,7 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
     // the state entering every hstride-th chunk goes to the stash (slot c / hstride of the sequence), each wave
     // its own rows; the branch is uniform and the stored values come from registers, not from loads in flight
     const bool keep = (c & (hstride - 1)) == 0;
-    const int64_t hidx = (int64_t)bh * ((NT + hstride - 1) / hstride) + c / hstride;
+    const int64_t hidx = seq * ((NT + hstride - 1) / hstride) + c / hstride;
     if constexpr (SAVE) {
       if (keep) {
 #pragma unroll
@@ -238,7 +244,7 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
     if constexpr (OUT) xR[w][l] = Rbmine;
     if constexpr (SAVE) store_fragblk<T, FWD_NT_STORE>(wsR + cidx * CH * V, CH, hf, cb, ncb, Rbmine);
     __syncthreads();  // R and Rd fragments of both halves exchanged
-    if (c + 1 < NT) prefetch2(c + 1);
+    if (c + 1 < c_end) prefetch2(c + 1);
     const F Rdother = xRd[w ^ NSL][l];
     if constexpr (OUT) {
       const F Rbother = xR[w ^ NSL][l];
@@ -273,9 +279,9 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
   tri_zero_upper<T, FTH>(sTm, LC, tid);
   if constexpr (OUT) tri_zero_upper<T, FTH>(sP, LC, tid);
   publish_state();  // read after the first chunk's first barrier
-  prefetch(0);
-  prefetch2(0);
-  for (int c = 0; c < NT; ++c) chunk(c);
+  prefetch(c_first);
+  prefetch2(c_first);
+  for (int c = c_first; c < c_end; ++c) chunk(c);
   if (ident) {
 #pragma unroll
     for (int t = 0; t < NKH; ++t)
@@ -294,13 +300,13 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
 // ---------------------------------------------------------------------------------------------------------
 template <typename T, int K, int MODE, bool SEPU, int BV>
 static hipError_t fwd_sweep_bv(const ChunkArgs& a) {
-  dim3 grid((a.V + (MODE == 3 ? K : 0)) / BV * a.B * a.H);
+  dim3 grid((a.V + (MODE == 3 ? K : 0)) / BV * a.B * a.ns * a.H);
   fwd_sweep_kernel<T, K, BV, MODE, SEPU><<<grid, fwd_threads<BV>(), 0, a.stream>>>(
       static_cast<const T*>(a.q), static_cast<const T*>(a.k), static_cast<const T*>(a.u),
       static_cast<const T*>(a.v), a.beta, a.h0,
       static_cast<const T*>(a.ws.Tm), static_cast<const T*>(a.ws.P), a.ws.Gc, static_cast<T*>(a.o),
       MODE == 1 ? nullptr : a.hT, a.ws.phi, static_cast<T*>(a.ws.hs), static_cast<T*>(a.ws.Rs), a.T, a.H, a.V,
-      a.NT, a.scale, a.ns, a.hstride);
+      a.NT, a.scale, a.ns, a.cps, a.hstride);
   return hipGetLastError();
 }
 

@@ -43,7 +43,7 @@ struct ChunkWs {
   void* Rs;   // [BH][NT][64][V]    R = U - W S per chunk
   void* dhs;  // [BH][NT][K][V]     dL/d(state leaving each chunk)
   void* dYs;  // [BH][NT][64][V]    dY = Tm^T dL/dR per chunk (the gradient w.r.t. Y, R = Tm Y)
-  // segmented sweeps (WS_SEGF, WS_SEGB; see segment_count), fp32, in the segmented [B*NS, H, ...] layout:
+  // segmented sweeps (WS_SEGF, WS_SEGB; see segment_plan), fp32, one per segment and head, [B][ns][H]:
   float* phi;    // [B*NS][H][K][K]  transition of each segment
   float* sloc;   // [B*NS][H][K][V]  state leaving each segment from a zero entering state
   float* sin;    // [B*NS][H][K][V]  state entering each segment
@@ -73,11 +73,12 @@ struct ChunkArgs {
   float scale;
   int dtype;
   hipStream_t stream;
-  // Segmented sweeps: B counts the segments (B = batch * ns, segment s of sequence b is b * ns + s).  With
-  // ns > 1 the main sweeps write hT only from each sequence's last segment and dh0 only from its first, and the
-  // prefix pass (local reverse pass) starts each sequence's first (last) segment from h0 (dhT), all at the
+  // Segmented sweeps: each sequence's NT chunks are cut into ns segments of cps chunks (the last possibly shorter),
+  // swept in parallel; only the sweeps know of the segments, the per-chunk buffers stay [B * H][NT].  With ns > 1 the
+  // main sweeps take h0 (dhT) per segment, write hT only from each sequence's last segment and dh0 only from its
+  // first, and the prefix pass (local reverse pass) starts each sequence's first (last) segment from h0 (dhT) at the
   // sequence's own index.
-  int ns = 1;
+  int ns = 1, cps = 0;
   int hstride = 1;  // state_stride(): the stash holds the state entering every hstride-th chunk
 };
 
@@ -91,14 +92,14 @@ size_t chunk_ws_bytes(int B, int T, int H, int K, int V, int dtype, int parts, C
                       int hstride);
 
 // Segmented sweeps: when the state sweeps would leave most compute units idle ((V/64) B H workgroups) and the
-// sequence is long, it is cut into NS equal segments of whole chunks, swept in parallel as the problem
-// [B*NS, T/NS, H] (the same memory: a segment of a token-major tensor is contiguous), with the states carried
-// across segments by a prefix pass and a small scan (gdn_segscan.hip).  Returns NS (1: not segmented); a pure
-// function of the shape and the device's CU count, so a forward and its backward agree.
-int segment_count(int B, int T, int H, int K, int V);
+// sequence is long, its chunks are cut into ns segments of cps chunks (the last possibly shorter), swept in parallel,
+// with the states carried across segments by a prefix pass and a small scan (gdn_segscan.hip).  ns = 1: not
+// segmented.  A pure function of the shape and the device's CU count, so a forward and its backward agree.
+struct SegPlan { int ns, cps; };
+SegPlan segment_plan(int B, int T, int H, int K, int V);
 // Carry states (reverse = false) or state gradients (reverse = true) across the segments of every (b, h).
-hipError_t launch_seg_scan(const float* phi, const float* loc, const float* init, float* outs, float* fin, int B,
-                           int NS, int H, int K, int V, bool reverse, hipStream_t stream);
+hipError_t launch_seg_scan(const float* phi, const float* loc, const float* init, float* outs, int B, int NS, int H,
+                           int K, int V, bool reverse, hipStream_t stream);
 bool chunk_shape_supported(int K, int V, int dtype);
 bool step_shape_supported(int K, int V);
 

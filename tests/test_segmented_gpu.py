@@ -126,3 +126,32 @@ def test_segmented_batch_without_states(with_h0, with_dhT):
     errs.update({n: rel_l2(a, b) for n, a, b in zip(NAMES, got, ref)})
     print("[segmented batch] rel-L2 " + ", ".join(f"{n} {e:.2e}" for n, e in errs.items()), flush=True)
     assert all(e <= 1e-2 for e in errs.values()), errs
+
+
+@pytest.mark.parametrize("B,T,H,K,V,dtype", [
+    (1, 1025, 2, 64, 64, torch.bfloat16),    # the last segment is one chunk of one token
+    (1, 1985, 2, 128, 128, torch.bfloat16),  # the last chunk one token; states kept for every second chunk
+    (2, 1601, 1, 64, 64, torch.bfloat16),    # a ragged last chunk; a short last segment
+    (1, 2111, 3, 128, 256, torch.bfloat16),  # every state stored; heads not a multiple of the XCDs
+    (1, 1090, 1, 64, 128, torch.float32),
+])
+def test_segments_of_any_length(B, T, H, K, V, dtype):
+    """A sequence of any length is segmented (the last segment shorter, its last chunk ragged): output, final state
+    and every gradient against the fp64 oracle, at the bars of the equal segments above."""
+    banner(f"segments of any length B={B} T={T} H={H} K={K} V={V} {dtype}")
+    host, dev = device_inputs(B, T, H, K, V, dtype, seed=50, h0_std=0.1, with_do=True)
+    dhT = torch.randn(B, H, K, V, generator=torch.Generator().manual_seed(51)) * 0.1
+    with _lib.StageTimer() as st:
+        o, hT, stash = ops.chunk_fwd_stash(dev.q, dev.k, dev.v, dev.g, dev.beta, dev.h0, 0.7)
+        got = ops.chunk_bwd_stashed(dev.q, dev.k, dev.v, dev.g, dev.beta, dev.h0, dev.do, dhT.cuda(), stash, 0.7)
+    torch.cuda.synchronize()
+    assert {"prefix", "seg_scan", "bwd_local"} <= set(st.result), st.result
+    o_r, hT_r = O.chunk_fwd(host.q, host.k, host.v, host.g, host.beta, 0.7, host.h0)
+    ref = O.chunk_bwd(host.q, host.k, host.v, host.g, host.beta, host.do, 0.7, host.h0, dhT)
+    if dtype == torch.float32:
+        assert_fp32_close("segments of any length", ["o", "hT", *NAMES], [o, hT, *got], [o_r, hT_r, *ref], 1e-4)
+        return
+    errs = {"o": rel_l2(o, o_r), "hT": rel_l2(hT, hT_r)}
+    errs.update({n: rel_l2(a, b) for n, a, b in zip(NAMES, got, ref)})
+    print("[segments of any length] rel-L2 " + ", ".join(f"{n} {e:.2e}" for n, e in errs.items()), flush=True)
+    assert all(e <= 1e-2 for e in errs.values()), errs
