@@ -47,6 +47,9 @@ SIGNATURES = {
     "gdn_short_conv_bwd_ws_bytes": (_i, [_i, _i, _i, _i, ctypes.POINTER(_sz)]),
     "gdn_short_conv_bwd": (_i, [_p, _i64, _p, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _sz, _i, _i, _i, _i, _i, _i,
                                 _p]),
+    "gdn_mixer_stage_fwd": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
+    "gdn_mixer_stage_bwd_ws_bytes": (_i, [_i, _i, _i, _i, _i, ctypes.POINTER(_sz)]),
+    "gdn_mixer_stage_bwd": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i, _i, _i, _i, _i, _p]),
     "gdn_gated_rmsnorm_fwd": (_i, [_p, _p, _i64, _i, _p, _p, _i64, _i, _f, _i, _p]),
     "gdn_gated_rmsnorm_bwd_ws_bytes": (_i, [_i64, _i, ctypes.POINTER(_sz)]),
     "gdn_gated_rmsnorm_bwd": (_i, [_p, _p, _i64, _i, _p, _p, _p, _p, _p, _p, _sz, _i64, _i, _f, _i, _p]),
@@ -195,6 +198,18 @@ def _stash_bytes(B: int, T: int, H: int, K: int, V: int, dtype: torch.dtype, nsg
 def conv_ws_bytes(B: int, T: int, D: int, W: int) -> int:
     out = _sz(0)
     check(load().gdn_short_conv_bwd_ws_bytes(B, T, D, W, ctypes.byref(out)), "gdn_short_conv_bwd_ws_bytes")
+    return out.value
+
+
+def stage_ws_bytes(B: int, T: int, key_dim: int, value_dim: int, W: int) -> int:
+    return _stage_ws_bytes(B, T, key_dim, value_dim, W, _device_index())
+
+
+@functools.lru_cache(maxsize=1024)
+def _stage_ws_bytes(B: int, T: int, key_dim: int, value_dim: int, W: int, dev: int) -> int:
+    out = _sz(0)
+    check(load().gdn_mixer_stage_bwd_ws_bytes(B, T, key_dim, value_dim, W, ctypes.byref(out)),
+          "gdn_mixer_stage_bwd_ws_bytes")
     return out.value
 
 

@@ -620,7 +620,7 @@ int gdn_short_conv_bwd_ws_bytes(int B, int T, int D, int W, size_t* bytes) {
   g_err[0] = 0;
   if (B < 0 || T < 0 || D <= 0 || W <= 0) return fail(GDN_ERR_ARG, "invalid sizes B=%d T=%d D=%d W=%d", B, T, D, W);
   if (!bytes) return fail(GDN_ERR_ARG, "bytes is NULL");
-  *bytes = conv_ws_bytes(B, T, D, W);
+  *bytes = conv_ws_bytes(B, T, {D, 0, 0}, W);
   return GDN_OK;
 }
 
@@ -658,8 +658,8 @@ int gdn_short_conv_fwd(const void* x, int64_t ldx, const float* w, const float* 
   if (state_out && state_out == state_in) return fail(GDN_ERR_ARG, "state_out must not alias state_in");
   if (misaligned(x, w, bias, state_in, y, state_out)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
   ConvArgs a{};
-  a.x = x; a.w = w; a.bias = bias; a.state_in = state_in; a.y = y; a.state_out = state_out;
-  a.B = B; a.T = T; a.D = D; a.ldx = ldx; a.norm_group = norm_group; a.dtype = dtype;
+  a.x = x; a.w = w; a.bias = bias; a.state_in = state_in; a.y[0] = y; a.state_out = state_out;
+  a.B = B; a.T = T; a.n[0] = D; a.normed = 1; a.ldx = ldx; a.norm_group = norm_group; a.dtype = dtype;
   a.stream = static_cast<hipStream_t>(stream);
   const hipError_t e = timed(ST_CONV_FWD, a.stream, [&] { return launch_conv(a, false); });
   if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "short conv forward launch: %s", hipGetErrorString(e));
@@ -686,15 +686,76 @@ int gdn_short_conv_bwd(const void* x, int64_t ldx, const float* w, const float* 
   if (!x || !w || !dy || !dx || !dw) return fail(GDN_ERR_ARG, "null input/output pointer");
   if (misaligned(x, w, bias, state_in, dy, dx, dw, dbias, dstate_in, ws))
     return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
-  const size_t need = conv_ws_bytes(B, T, D, W);
+  const size_t need = conv_ws_bytes(B, T, {D, 0, 0}, W);
   if (!ws || ws_bytes < need)
     return fail(GDN_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, ws ? ws_bytes : (size_t)0);
   ConvArgs a{};
-  a.x = x; a.w = w; a.bias = bias; a.state_in = state_in; a.dy = dy; a.dx = dx; a.dstate_in = dstate_in;
+  a.x = x; a.w = w; a.bias = bias; a.state_in = state_in; a.dy[0] = dy; a.dx = dx; a.dstate_in = dstate_in;
   a.dw = dw; a.dbias = dbias; a.ws = ws;
-  a.B = B; a.T = T; a.D = D; a.ldx = ldx; a.lddx = lddx; a.norm_group = norm_group; a.dtype = dtype; a.stream = st;
+  a.B = B; a.T = T; a.n[0] = D; a.normed = 1; a.ldx = ldx; a.lddx = lddx; a.norm_group = norm_group; a.dtype = dtype; a.stream = st;
   const hipError_t e = timed(ST_CONV_BWD, st, [&] { return launch_conv(a, true); });
   if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "short conv backward launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
+// The mixer's input stage: key_dim columns for q, key_dim for k (both normalised), value_dim for v
+static int stage_check(int B, int T, int key_dim, int value_dim, int W, int norm_group, int dtype) {
+  if (key_dim <= 0 || value_dim <= 0)
+    return fail(GDN_ERR_ARG, "invalid key_dim=%d value_dim=%d", key_dim, value_dim);
+  if ((int64_t)2 * key_dim + value_dim > INT32_MAX / 8) return fail(GDN_ERR_ARG, "too many channels");
+  const int D = 2 * key_dim + value_dim;
+  if (int e = conv_check(B, T, key_dim, D, W, norm_group, dtype, "2 key_dim + value_dim")) return e;
+  return conv_check(B, T, value_dim, D, W, 0, dtype, "2 key_dim + value_dim");
+}
+
+int gdn_mixer_stage_fwd(const void* y, const float* w, void* q, void* k, void* v, int B, int T, int key_dim,
+                        int value_dim, int W, int norm_group, int dtype, void* stream) {
+  g_err[0] = 0;
+  if (int e = stage_check(B, T, key_dim, value_dim, W, norm_group, dtype)) return e;
+  if (B == 0 || T == 0) return GDN_OK;
+  if (!y || !w || !q || !k || !v) return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(y, w, q, k, v)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  ConvArgs a{};
+  a.x = y; a.w = w; a.y[0] = q; a.y[1] = k; a.y[2] = v;
+  a.B = B; a.T = T; a.n[0] = a.n[1] = key_dim; a.n[2] = value_dim; a.normed = 2; a.ldx = 2 * key_dim + value_dim;
+  a.norm_group = norm_group; a.dtype = dtype; a.stream = static_cast<hipStream_t>(stream);
+  const hipError_t e = timed(ST_CONV_FWD, a.stream, [&] { return launch_conv(a, false); });
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "mixer input stage forward launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
+int gdn_mixer_stage_bwd_ws_bytes(int B, int T, int key_dim, int value_dim, int W, size_t* bytes) {
+  g_err[0] = 0;
+  if (B < 0 || T < 0 || key_dim <= 0 || value_dim <= 0 || W <= 0)
+    return fail(GDN_ERR_ARG, "invalid sizes B=%d T=%d key_dim=%d value_dim=%d W=%d", B, T, key_dim, value_dim, W);
+  if (!bytes) return fail(GDN_ERR_ARG, "bytes is NULL");
+  *bytes = conv_ws_bytes(B, T, {key_dim, key_dim, value_dim}, W);
+  return GDN_OK;
+}
+
+int gdn_mixer_stage_bwd(const void* y, const float* w, const void* dq, const void* dk, const void* dv, void* dy,
+                        float* dw, void* ws, size_t ws_bytes, int B, int T, int key_dim, int value_dim, int W,
+                        int norm_group, int dtype, void* stream) {
+  g_err[0] = 0;
+  if (int e = stage_check(B, T, key_dim, value_dim, W, norm_group, dtype)) return e;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int D = 2 * key_dim + value_dim;
+  if (B == 0 || T == 0) {
+    if (copy_or_zero_bytes(nullptr, dw, (size_t)D * W * 4, st) != hipSuccess)
+      return fail(GDN_ERR_LAUNCH, "mixer input stage zero-fill launch failed");
+    return GDN_OK;
+  }
+  if (!y || !w || !dq || !dk || !dv || !dy || !dw) return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(y, w, dq, dk, dv, dy, dw, ws)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  ConvArgs a{};
+  a.x = y; a.w = w; a.dy[0] = dq; a.dy[1] = dk; a.dy[2] = dv; a.dx = dy; a.dw = dw; a.ws = ws;
+  a.B = B; a.T = T; a.n[0] = a.n[1] = key_dim; a.n[2] = value_dim; a.normed = 2; a.ldx = a.lddx = D;
+  a.norm_group = norm_group; a.dtype = dtype; a.stream = st;
+  const size_t need = conv_ws_bytes(B, T, a.n, W);
+  if (!ws || ws_bytes < need)
+    return fail(GDN_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, ws ? ws_bytes : (size_t)0);
+  const hipError_t e = timed(ST_CONV_BWD, st, [&] { return launch_conv(a, true); });
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "mixer input stage backward launch: %s", hipGetErrorString(e));
   return GDN_OK;
 }
 

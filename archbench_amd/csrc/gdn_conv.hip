@@ -9,10 +9,13 @@
 // (= D, or larger to read or write a column slice of a wider tensor in place); w [D, W] fp32 (used rounded to the
 // activation dtype; dw is the fp32 gradient of those rounded taps), bias [D] fp32, conv states
 // [B, D, W-1] in the activation dtype (the previous W-1 inputs, oldest first).
-// Mapping: one wave per (256 channels, 64-token chunk, b); each lane holds 4 consecutive channels, so every token
-// row is one 8-byte (bf16) or 16-byte (fp32) access per lane and a wave covers 512 B / 1 KB contiguous.  The W-1
-// inputs before a chunk are re-read (a (W-1)/64 halo).  A normalisation group of NG channels spans NG/4 lanes and
-// is reduced with lane shuffles.  HBM-bound: x read once, y written once.
+// Mapping: one wave per (256 channels, chunk of 8 to 128 tokens, b); each lane holds 4 consecutive channels, so every
+// token row is one 8-byte (bf16) or 16-byte (fp32) access per lane and a wave covers 512 B / 1 KB contiguous.  The W-1
+// inputs before a chunk are re-read.  A normalisation group of NG channels spans NG/4 lanes and is reduced with lane
+// shuffles.  One launch covers up to three column groups of x (ConvGroups): the mixer's q, k and v, whose three launches
+// of 2 to 8 waves per CU left the memory half idle (B64 T1024 H4: forward 153 -> 96 us, 5.6 TB/s; backward 252 -> 172
+// us, 4.7 TB/s, with the rolling row slots below).  The forward is HBM-bound (x read once, y written once); the backward
+// is near both its HBM and its VALU bound (about 37 issue slots per element, 126 us at that size).
 // Backward: each wave recomputes z for its chunk plus W-1 tokens of look-ahead, forms dz and emits dx with a
 // W-token delay; dw and dbias are summed per wave into a per-chunk partial and reduced over chunks in a fixed
 // order by column_sum_kernel (deterministic, no atomics).
@@ -23,21 +26,22 @@
 
 namespace gdn {
 
-constexpr int CONV_L = 64;  // tokens per wave (the backward without normalisation may take CONV_L_LONG)
-// Tokens per wave of the backward without the normalisation when the grid stays large (at least
-// CONV_LONG_MIN_WAVES_PER_CU waves per CU): each wave's set-up, look-ahead recompute and dw partial are then
-// amortised over twice the tokens (96 -> 86 us at B8 T4096 D2048, 99 -> 91 us at B64 T1024 D1024); on small grids
-// the shorter chunks' parallelism wins (23 against 39 us at B2 T200 D512).  With the normalisation 64 throughout
-// (at the 65m layer's D = 512, 61 against 70 us with 128).
-constexpr int CONV_L_LONG = 128, CONV_LONG_MIN_WAVES_PER_CU = 4;
+// Tokens per wave, a multiple of the rows in flight.  64 on a grid of ordinary size.  The backward takes 128 once that
+// leaves 8 waves per CU: the set-up, the look-ahead recompute and the dw partial of a wave are then amortised over twice
+// the tokens (D = 2048 without normalisation: 94.5 -> 76.6 us at B8 T4096, but 47.8 -> 58.9 at B4 T4000, 4 waves per CU;
+// the 65m mixer's input stage, B64 T1024, 182 -> 172 us).  A small grid is cut finer until it has 10 waves per CU in
+// the forward and 6 in the backward, whose dw partials grow with the cut (input stage, forward / backward at 64, 32, 16
+// and 8 tokens: B6 T777 H8 30.1 / 51.6, 23.9 / 46.0, 22.5 / 52.0, 24.4 / 70.3 us; B2 T1000 H4 20.5 / 37.2, 13.5 / 25.6,
+// 12.4 / 23.4, 9.5 / 23.9 us; B12 T1024 H8, 12 waves per CU at 64 tokens, 42.7 / 74.0, 46.0 / 85.7 us), the backward
+// below 16 tokens only when even that leaves CUs without a wave (B1 T200 H3: 19.0 -> 13.4 us).
+constexpr int CONV_L = 64, CONV_L_LONG = 128, CONV_L_MIN = 8, CONV_L_MIN_BWD = 16;
+constexpr int CONV_LONG_WAVES_PER_CU = 8, CONV_FWD_WAVES_PER_CU = 10, CONV_BWD_WAVES_PER_CU = 6;
 constexpr int CONV_CPL = 4;  // consecutive channels per lane
 constexpr int CONV_CW = 64 * CONV_CPL;  // channels per wave
 constexpr int CONV_WAVES = 4;  // waves per workgroup, on adjacent channel blocks of the same chunk
 constexpr int CONV_UF = 8;  // token rows per load batch, forward
-// token rows of x and of dy per load batch, backward: with the per-group normalisation the smaller batch measured
-// faster (fewer registers in flight beside the group sums' longer chain: 109 -> 102 us at B8 T4096 D2048), without
-// it the larger one (95 against 102 us)
-constexpr int CONV_UB = 8, CONV_UB_NORM = 4;
+constexpr int CONV_UB = 8;  // token rows of x and of dy in flight, backward (4: 180 against 172 us)
+static_assert(CONV_L_MIN % CONV_UB == 0 && CONV_L_MIN_BWD % CONV_UB == 0, "whole batches in every chunk but the last");
 
 // CONV_CPL = 4 consecutive channels of one token row as loaded (8 B in bf16, 16 B in fp32), converted at use so
 // that a whole batch of loads is in flight at once.  The backward reads x and dy and writes dx once each through
@@ -126,36 +130,58 @@ __device__ __forceinline__ void load_window(const T* xl, const T* state_in, int6
   }
 }
 
-// Work items: (part = b * nchunk + chunk, 256-channel block), blocks fastest; wave w of workgroup x takes item
-// x * CONV_WAVES + w, so the waves of a workgroup, each independent, cover adjacent channel blocks of the same
-// token rows (and, when D has fewer than CONV_WAVES blocks, the next chunk's: no wave idles at D = 256 or 512).
-__device__ __forceinline__ bool conv_wave_item(int D, int nparts, int& part, int& cw0) {
-  const int ncb = (D + CONV_CW - 1) / CONV_CW;
-  const int item = (int)blockIdx.x * CONV_WAVES + __builtin_amdgcn_readfirstlane(wave_id());  // uniform: scalar
-  part = item / ncb;
-  cw0 = (item - part * ncb) * CONV_CW;
-  return part < nparts;
-}
-// Forward: grid ceil(B * nchunk * ceil(D / CONV_CW) / CONV_WAVES), CONV_WAVES waves.  Rows are loaded in batches
-// of CONV_UF with the next batch in flight while the current one is computed; the prefetch of the last batch
-// re-reads it (start clamped to t1 - CONV_UF) so every load stays inside the chunk.
+// The channels of x in up to three consecutive column groups (plain convolutions: one), each with a contiguous tensor
+// of its own on the other side (y in the forward, dy in the backward: [B, T, n]); the first `normed` groups are
+// L2-normalised.
+template <typename T>
+struct ConvGroups {
+  T* p[3];
+  int n[3];
+  int normed;
+};
+// Work items: (part = b * nchunk + chunk, 256-channel block of one group), blocks fastest; wave w of workgroup x takes
+// item x * CONV_WAVES + w, so the waves of a workgroup, each independent, cover adjacent channel blocks of the same
+// token rows (and, when there are fewer than CONV_WAVES blocks, the next chunk's: no wave idles).  The whole item is
+// uniform over the wave.
+template <typename T>
+struct ConvItem {
+  int part, b, t0, t1, cw0, xc0, n;  // cw0: first channel inside the group, xc0: the group's first column of x
+  bool norm;
+  T* p;
+  __device__ __forceinline__ bool init(const ConvGroups<T>& g, int Tn, int L, int nchunk, int nparts) {
+    const int nb0 = (g.n[0] + CONV_CW - 1) / CONV_CW, nb1 = nb0 + (g.n[1] + CONV_CW - 1) / CONV_CW;
+    const int ncb = nb1 + (g.n[2] + CONV_CW - 1) / CONV_CW;
+    const int item = (int)blockIdx.x * CONV_WAVES + __builtin_amdgcn_readfirstlane(wave_id());
+    part = item / ncb;
+    const int blk = item - part * ncb, gi = (blk >= nb0) + (blk >= nb1);
+    cw0 = (blk - (gi == 0 ? 0 : gi == 1 ? nb0 : nb1)) * CONV_CW;
+    xc0 = gi == 0 ? 0 : gi == 1 ? g.n[0] : g.n[0] + g.n[1];
+    n = gi == 0 ? g.n[0] : gi == 1 ? g.n[1] : g.n[2];
+    p = gi == 0 ? g.p[0] : gi == 1 ? g.p[1] : g.p[2];
+    norm = gi < g.normed;
+    b = part / nchunk;
+    t0 = (part - b * nchunk) * L;
+    t1 = min(Tn, t0 + L);
+    return part < nparts;
+  }
+};
+// Forward: grid ceil(B * nchunk * blocks / CONV_WAVES), CONV_WAVES waves.  Rows are loaded in batches of CONV_UF with
+// the next batch in flight while the current one is computed; the prefetch of the last batch re-reads it (start clamped
+// to t1 - CONV_UF) so every load stays inside the chunk.  D: all channels (those of w and the states).
 template <typename T, int W, int NG>
-__global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_fwd_kernel(const T* __restrict__ x, const float* __restrict__ w,
-                                                           const float* __restrict__ bias,
-                                                           const T* __restrict__ state_in, T* __restrict__ y,
-                                                           T* __restrict__ state_out, int Tn, int D, int ldx,
-                                                           int nchunk, int nparts) {
+__device__ __forceinline__ void conv_fwd_wave(const ConvItem<T>& it, const T* __restrict__ x,
+                                              const float* __restrict__ w, const float* __restrict__ bias,
+                                              const T* __restrict__ state_in, T* __restrict__ state_out, int Tn, int D,
+                                              int ldx) {
   constexpr int CPL = CONV_CPL, U = CONV_UF;
-  const int l = lane_id();
-  int part, cw0;
-  if (!conv_wave_item(D, nparts, part, cw0)) return;  // past the last item (waves never synchronise)
-  const int c = cw0 + CPL * l;
-  const int b = part / nchunk, ch = part - b * nchunk;
-  const int t0 = ch * CONV_L, t1 = min(Tn, t0 + CONV_L);
-  const bool on = c < D;
-  const int cc = on ? c : 0;  // clamped: lanes past D compute on channel 0 and store nothing
+  const int c = it.cw0 + CPL * lane_id();
+  const int b = it.b, t0 = it.t0, t1 = it.t1;
+  const bool on = c < it.n;
+  const int cg = on ? c : 0;      // channel inside the group; clamped: lanes past it compute on its first channel and
+  const int cc = it.xc0 + cg;     // store nothing.  cc: the same channel of x, w, bias and the states
   const T* xl = x + (int64_t)b * Tn * ldx + cc;  // token t of x at xl + t * ldx
-  T* yl = y + (int64_t)b * Tn * D + cc;
+  const int ldy = it.n;
+  T* yl = it.p + (int64_t)b * Tn * ldy + cg;
   const int64_t srow = ((int64_t)b * D + cc) * (W - 1);
   float wk[CPL][W], bk[CPL];
 #pragma unroll
@@ -183,7 +209,7 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_fwd_kernel(const T*
 #pragma unroll
       for (int j = 0; j < CPL; ++j) yt[j] *= inv;
     }
-    if (on) store4(yl + (int64_t)t * D, yt);
+    if (on) store4(yl + (int64_t)t * ldy, yt);
 #pragma unroll
     for (int i = 0; i + 1 < W - 1; ++i)
 #pragma unroll
@@ -225,40 +251,50 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_fwd_kernel(const T*
   }
 }
 
+// NG: the normalisation group of the groups that have one (0: none has)
+template <typename T, int W, int NG>
+__global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_fwd_kernel(const T* __restrict__ x,
+                                                                        const float* __restrict__ w,
+                                                                        const float* __restrict__ bias,
+                                                                        const T* __restrict__ state_in,
+                                                                        ConvGroups<T> y, T* __restrict__ state_out,
+                                                                        int Tn, int D, int ldx, int L, int nchunk,
+                                                                        int nparts) {
+  ConvItem<T> it;
+  if (!it.init(y, Tn, L, nchunk, nparts)) return;  // past the last item (waves never synchronise)
+  if constexpr (NG > 0) {
+    if (it.norm) return conv_fwd_wave<T, W, NG>(it, x, w, bias, state_in, state_out, Tn, D, ldx);
+  }
+  conv_fwd_wave<T, W, 0>(it, x, w, bias, state_in, state_out, Tn, D, ldx);
+}
+
 // grid and waves as in the forward; partial sums of dw and dbias per (b, chunk) = part.
 // Each wave recomputes z over its chunk plus W-1 tokens of look-ahead, forms dz, and emits dx with a W-1 token
-// delay; rows of x and dy are loaded in double-buffered batches (CONV_UB, or CONV_UB_NORM with the normalisation) as
-// in the forward.
-template <typename T, int W, int NG, int L>
-__global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_bwd_kernel(const T* __restrict__ x, const float* __restrict__ w,
-                                                           const float* __restrict__ bias,
-                                                           const T* __restrict__ state_in,
-                                                           const T* __restrict__ dy, T* __restrict__ dx,
-                                                           T* __restrict__ dstate_in, float* __restrict__ part_out,
-                                                           int Tn, int D, int ldx, int lddx, int nchunk,
-                                                           int nparts) {
-  constexpr int CPL = CONV_CPL, U = NG > 0 ? CONV_UB_NORM : CONV_UB;
-  const int l = lane_id();
-  int part, cw0;
-  if (!conv_wave_item(D, nparts, part, cw0)) return;  // past the last item (waves never synchronise)
-  const int c = cw0 + CPL * l;
-  const int b = part / nchunk, ch = part - b * nchunk;
-  const int t0 = ch * L, t1 = min(Tn, t0 + L);
-  const bool on = c < D;
-  const int cc = on ? c : 0;
+// delay; CONV_UB rows of x and dy are in flight.
+template <typename T, int W, int NG, bool BIAS>
+__device__ __forceinline__ void conv_bwd_wave(const ConvItem<const T>& it, const T* __restrict__ x,
+                                              const float* __restrict__ w, const float* __restrict__ bias,
+                                              const T* __restrict__ state_in, T* __restrict__ dx,
+                                              T* __restrict__ dstate_in, float* __restrict__ part_out, int ldp,
+                                              int Tn, int D, int ldx, int lddx) {
+  constexpr int CPL = CONV_CPL, U = CONV_UB;
+  const int c = it.cw0 + CPL * lane_id();
+  const int b = it.b, t0 = it.t0, t1 = it.t1;
+  const bool on = c < it.n;
+  const int cg = on ? c : 0, cc = it.xc0 + cg;  // as in the forward
   const T* xl = x + (int64_t)b * Tn * ldx + cc;
   const int64_t srow = ((int64_t)b * D + cc) * (W - 1);
-  // the batch element's rows of x ([Tn] rows ldx apart), dy and dx ([Tn][D]) as buffer resources (uniform base,
-  // 32-bit offsets: the host keeps Tn * ldx * sizeof(T) under 2 GiB); token t, this lane's channels at byte
-  // offset xoff(t) in x and boff(t) in dy and dx
-  const int64_t bbase = (int64_t)b * Tn * D;
-  const int bbytes = Tn * D * (int)sizeof(T);
+  // the batch element's rows of x ([Tn] rows ldx apart), dy ([Tn][n]) and dx (rows lddx apart) as buffer resources
+  // (uniform base, 32-bit offsets: the host keeps Tn * ldx * sizeof(T) under 2 GiB); token t, this lane's channels at
+  // byte offset xoff(t) in x, boff(t) in dy and dxoff(t) in dx
+  const int ldy = it.n;
   const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(x + (int64_t)b * Tn * ldx), 0,
                                                     Tn * ldx * (int)sizeof(T), BUF_RSRC_WORD3);
-  const auto rdy = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(dy + bbase), 0, bbytes, BUF_RSRC_WORD3);
+  const auto rdy = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(it.p + (int64_t)b * Tn * ldy), 0,
+                                                     Tn * ldy * (int)sizeof(T), BUF_RSRC_WORD3);
   const auto rdx = __builtin_amdgcn_make_buffer_rsrc(dx + (int64_t)b * Tn * lddx, 0, Tn * lddx * (int)sizeof(T),
                                                      BUF_RSRC_WORD3);
-  auto boff = [&](int t) { return (t * D + cc) * (int)sizeof(T); };
+  auto boff = [&](int t) { return (t * ldy + cg) * (int)sizeof(T); };
   auto xoff = [&](int t) { return (t * ldx + cc) * (int)sizeof(T); };
   auto dxoff = [&](int t) { return (t * lddx + cc) * (int)sizeof(T); };
   float wk[CPL][W], bk[CPL];
@@ -266,7 +302,7 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_bwd_kernel(const T*
   for (int j = 0; j < CPL; ++j) {
 #pragma unroll
     for (int i = 0; i < W; ++i) wk[j][i] = act_round<T>(w[(cc + j) * W + i]);
-    bk[j] = bias ? bias[cc + j] : 0.f;
+    bk[j] = BIAS && bias ? bias[cc + j] : 0.f;
   }
   float win[W - 1][CPL], dzw[W - 1][CPL], dwa[CPL][W], dba[CPL];
   load_window<T, W>(xl, state_in, srow, ldx, t0, win);
@@ -331,7 +367,7 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_bwd_kernel(const T*
     if constexpr (decltype(own)::value) {
 #pragma unroll
       for (int j = 0; j < CPL; ++j) {
-        dba[j] += dz[j];
+        if constexpr (BIAS) dba[j] += dz[j];
         dwa[j][W - 1] += dz[j] * xs[j];
 #pragma unroll
         for (int i = 0; i < W - 1; ++i) dwa[j][i] += dz[j] * win[i][j];
@@ -353,44 +389,37 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_bwd_kernel(const T*
   };
   using Own = std::true_type;
   using LookAhead = std::false_type;
-  const int nfull = (t1 - t0) / U;
+  // Rows U tokens ahead, one register slot per row modulo U, reloaded as soon as it is consumed (a second set of slots
+  // for the next batch took 32 more registers, one wave per SIMD fewer).  Loads past the sequence's end read its last row.
+  Row4<T> bx[U], bd[U];
+  auto load = [&](int u, int t) {
+    const int tc = min(t, Tn - 1);
+    bx[u].load_buf_nt(rx, xoff(tc));
+    bd[u].load_buf_nt(rdy, boff(tc));
+  };
+#pragma unroll
+  for (int u = 0; u < U; ++u) load(u, t0 + u);
   int s = t0;
-  if (nfull > 0) {
-    Row4<T> bx[U], bd[U];
+  for (const int full = t0 + (t1 - t0) / U * U; s < full; s += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      bx[u].load_buf_nt(rx, xoff(t0 + u));
-      bd[u].load_buf_nt(rdy, boff(t0 + u));
-    }
-    for (int n = 0; n < nfull; ++n, s += U) {
-      Row4<T> cx[U], cd[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        cx[u] = bx[u];
-        cd[u] = bd[u];
-      }
-      const int sn = min(s + U, t1 - U);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        bx[u].load_buf_nt(rx, xoff(sn + u));
-        bd[u].load_buf_nt(rdy, boff(sn + u));
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) step(s + u, cx[u], cd[u], Own{});
+      const Row4<T> cx = bx[u], cd = bd[u];
+      load(u, s + u + U);
+      step(s + u, cx, cd, Own{});
     }
   }
-  for (; s < t1; ++s) {
-    Row4<T> xr, dr;
-    xr.load_buf_nt(rx, xoff(s));
-    dr.load_buf_nt(rdy, boff(s));
-    step(s, xr, dr, Own{});
-  }
-  const int send = min(Tn, t1 + W - 1);
-  for (; s < send; ++s) {
-    Row4<T> xr, dr;
-    xr.load_buf_nt(rx, xoff(s));
-    dr.load_buf_nt(rdy, boff(s));
-    step(s, xr, dr, LookAhead{});
+  // Only the sequence's last chunk can hold a partial batch (the host keeps chunks whole multiples of U), only the
+  // others look ahead; either way the rows are in the slots already.
+  if (t1 == Tn) {
+#pragma unroll
+    for (int u = 0; u < U - 1; ++u)
+      if (s + u < t1) step(s + u, bx[u], bd[u], Own{});
+    s = t1;
+  } else {
+#pragma unroll
+    for (int u = 0; u < W - 1; ++u)
+      if (t1 + u < Tn) step(t1 + u, bx[u], bd[u], LookAhead{});
+    s = min(Tn, t1 + W - 1);
   }
   // past the sequence end dz = 0: flush the remaining dx of the chunk's tail (and of the state when Tn is short)
   for (; s < t1 + W - 1; ++s) {
@@ -404,77 +433,117 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_bwd_kernel(const T*
     for (int j = 0; j < CPL; ++j) dzw[W - 2][j] = 0.f;
   }
   if (on) {
-    float* row = part_out + (int64_t)part * (D * W + D);  // [dw (D x W) | dbias (D)] of this (b, chunk)
+    float* row = part_out + (int64_t)it.part * ldp;  // [dw (D x W) | dbias (D) if wanted] of this (b, chunk)
 #pragma unroll
     for (int j = 0; j < CPL; ++j) {
 #pragma unroll
       for (int i = 0; i < W; ++i) row[(cc + j) * W + i] = dwa[j][i];
-      row[D * W + cc + j] = dba[j];
+      if constexpr (BIAS) row[D * W + cc + j] = dba[j];
     }
   }
 }
 
+// BIAS: there is a bias or its gradient is wanted
+template <typename T, int W, int NG, bool BIAS>
+__global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_bwd_kernel(const T* __restrict__ x,
+                                                                        const float* __restrict__ w,
+                                                                        const float* __restrict__ bias,
+                                                                        const T* __restrict__ state_in,
+                                                                        ConvGroups<const T> dy, T* __restrict__ dx,
+                                                                        T* __restrict__ dstate_in,
+                                                                        float* __restrict__ part_out, int ldp, int Tn,
+                                                                        int D, int ldx, int lddx, int L, int nchunk,
+                                                                        int nparts) {
+  ConvItem<const T> it;
+  if (!it.init(dy, Tn, L, nchunk, nparts)) return;  // past the last item (waves never synchronise)
+  if constexpr (NG > 0) {
+    if (it.norm)
+      return conv_bwd_wave<T, W, NG, BIAS>(it, x, w, bias, state_in, dx, dstate_in, part_out, ldp, Tn, D, ldx, lddx);
+  }
+  conv_bwd_wave<T, W, 0, BIAS>(it, x, w, bias, state_in, dx, dstate_in, part_out, ldp, Tn, D, ldx, lddx);
+}
+
 // ---------------------------------------------------------------------------------------------------------
-size_t conv_ws_bytes(int B, int T, int D, int W) {
-  // partial rows of the backward: one per (b, chunk of CONV_L or CONV_L_LONG tokens), at most this many
-  const size_t nparts = (size_t)B * ((T + CONV_L - 1) / CONV_L);
+static int conv_blocks(const int (&n)[3]) {
+  int ncb = 0;
+  for (int i = 0; i < 3; ++i) ncb += (n[i] + CONV_CW - 1) / CONV_CW;
+  return ncb;
+}
+
+// tokens per wave (see CONV_L)
+static int conv_len(int B, int T, int ncb, bool backward) {
+  const int64_t cus = device_cu_count();
+  auto waves = [&](int L) { return (int64_t)ncb * B * ((T + L - 1) / L); };
+  if (backward && waves(CONV_L_LONG) >= CONV_LONG_WAVES_PER_CU * cus) return CONV_L_LONG;
+  int L = CONV_L;
+  while (L > (backward ? CONV_L_MIN_BWD : CONV_L_MIN) &&
+         waves(L) < (backward ? CONV_BWD_WAVES_PER_CU : CONV_FWD_WAVES_PER_CU) * cus)
+    L /= 2;
+  return backward && waves(L) < cus ? CONV_L_MIN : L;
+}
+
+size_t conv_ws_bytes(int B, int T, const int (&n)[3], int W) {
+  // partial rows of the backward: one per (b, chunk)
+  const int D = n[0] + n[1] + n[2];
+  const int L = conv_len(B, T, conv_blocks(n), true);
+  const size_t nparts = (size_t)B * ((T + L - 1) / L);
   return (nparts * (size_t)(D * W + D) * 4 + 255) & ~size_t(255);
 }
 
-bool conv_shape_supported(int D, int W, int norm_group) {
-  return D > 0 && D % CONV_CPL == 0 && W == 4 &&
-         (norm_group == 0 || ((norm_group == 64 || norm_group == 128 || norm_group == 256) && D % norm_group == 0));
+static bool conv_width_ok(int n, int norm_group) {
+  return n > 0 && n % CONV_CPL == 0 &&
+         (norm_group == 0 || ((norm_group == 64 || norm_group == 128 || norm_group == 256) && n % norm_group == 0));
 }
+bool conv_shape_supported(int D, int W, int norm_group) { return W == 4 && conv_width_ok(D, norm_group); }
 
 // workgroups for every (part, 256-channel block) item, CONV_WAVES items each
-static dim3 conv_grid(int D, int nparts) {
-  const int64_t items = (int64_t)(D + CONV_CW - 1) / CONV_CW * nparts;
-  return dim3((unsigned)((items + CONV_WAVES - 1) / CONV_WAVES));
+static dim3 conv_grid(int ncb, int nparts) {
+  return dim3((unsigned)(((int64_t)ncb * nparts + CONV_WAVES - 1) / CONV_WAVES));
 }
 
 template <typename T, int NG>
 static hipError_t conv_fwd_k(const ConvArgs& a) {
-  const int nchunk = (a.T + CONV_L - 1) / CONV_L;
-  const int nparts = a.B * nchunk;
-  conv_silu_fwd_kernel<T, 4, NG><<<conv_grid(a.D, nparts), 64 * CONV_WAVES, 0, a.stream>>>(
-      static_cast<const T*>(a.x), a.w, a.bias, static_cast<const T*>(a.state_in), static_cast<T*>(a.y),
-      static_cast<T*>(a.state_out), a.T, a.D, (int)a.ldx, nchunk, nparts);
+  const int ncb = conv_blocks(a.n), D = a.n[0] + a.n[1] + a.n[2];
+  const int L = conv_len(a.B, a.T, ncb, false), nchunk = (a.T + L - 1) / L, nparts = a.B * nchunk;
+  ConvGroups<T> g;
+  for (int i = 0; i < 3; ++i) g.p[i] = static_cast<T*>(a.y[i]), g.n[i] = a.n[i];
+  g.normed = NG > 0 ? a.normed : 0;
+  conv_silu_fwd_kernel<T, 4, NG><<<conv_grid(ncb, nparts), 64 * CONV_WAVES, 0, a.stream>>>(
+      static_cast<const T*>(a.x), a.w, a.bias, static_cast<const T*>(a.state_in), g, static_cast<T*>(a.state_out),
+      a.T, D, (int)a.ldx, L, nchunk, nparts);
   return hipGetLastError();
 }
 
-template <typename T, int NG, int L>
-static hipError_t conv_bwd_len(const ConvArgs& a) {
-  const int nchunk = (a.T + L - 1) / L;
-  const int nparts = a.B * nchunk;
+template <typename T, int NG, bool BIAS>
+static hipError_t conv_bwd_k(const ConvArgs& a) {
+  const int ncb = conv_blocks(a.n), D = a.n[0] + a.n[1] + a.n[2];
+  const int L = conv_len(a.B, a.T, ncb, true), nchunk = (a.T + L - 1) / L, nparts = a.B * nchunk;
+  ConvGroups<const T> g;
+  for (int i = 0; i < 3; ++i) g.p[i] = static_cast<const T*>(a.dy[i]), g.n[i] = a.n[i];
+  g.normed = NG > 0 ? a.normed : 0;
   float* part = static_cast<float*>(a.ws);
-  conv_silu_bwd_kernel<T, 4, NG, L><<<conv_grid(a.D, nparts), 64 * CONV_WAVES, 0, a.stream>>>(
-      static_cast<const T*>(a.x), a.w, a.bias, static_cast<const T*>(a.state_in), static_cast<const T*>(a.dy),
-      static_cast<T*>(a.dx), static_cast<T*>(a.dstate_in), part, a.T, a.D, (int)a.ldx, (int)a.lddx, nchunk,
-      nparts);
+  const int ldp = D * 4 + (BIAS ? D : 0);
+  conv_silu_bwd_kernel<T, 4, NG, BIAS><<<conv_grid(ncb, nparts), 64 * CONV_WAVES, 0, a.stream>>>(
+      static_cast<const T*>(a.x), a.w, a.bias, static_cast<const T*>(a.state_in), g, static_cast<T*>(a.dx),
+      static_cast<T*>(a.dstate_in), part, ldp, a.T, D, (int)a.ldx, (int)a.lddx, L, nchunk, nparts);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return launch_column_sum(part, nparts, a.D * 4 + a.D, ColumnOut{{a.dw, a.dbias, nullptr}, {a.D * 4, a.D, 0}},
-                           a.stream);
+  return launch_column_sum(part, nparts, ldp, ColumnOut{{a.dw, a.dbias, nullptr}, {D * 4, ldp - D * 4, 0}}, a.stream);
 }
 
 template <typename T, int NG>
-static hipError_t conv_bwd_k(const ConvArgs& a) {
-  if constexpr (NG == 0) {
-    const int64_t long_waves =
-        (int64_t)((a.D + CONV_CW - 1) / CONV_CW) * a.B * ((a.T + CONV_L_LONG - 1) / CONV_L_LONG);
-    if (long_waves >= (int64_t)CONV_LONG_MIN_WAVES_PER_CU * device_cu_count())
-      return conv_bwd_len<T, NG, CONV_L_LONG>(a);
-  }
-  return conv_bwd_len<T, NG, CONV_L>(a);
+static hipError_t conv_k(const ConvArgs& a, bool backward) {
+  if (!backward) return conv_fwd_k<T, NG>(a);
+  return a.bias || a.dbias ? conv_bwd_k<T, NG, true>(a) : conv_bwd_k<T, NG, false>(a);
 }
 
 template <typename T>
 static hipError_t conv_dispatch(const ConvArgs& a, bool backward) {
   switch (a.norm_group) {
-    case 0: return backward ? conv_bwd_k<T, 0>(a) : conv_fwd_k<T, 0>(a);
-    case 64: return backward ? conv_bwd_k<T, 64>(a) : conv_fwd_k<T, 64>(a);
-    case 128: return backward ? conv_bwd_k<T, 128>(a) : conv_fwd_k<T, 128>(a);
-    case 256: return backward ? conv_bwd_k<T, 256>(a) : conv_fwd_k<T, 256>(a);
+    case 0: return conv_k<T, 0>(a, backward);
+    case 64: return conv_k<T, 64>(a, backward);
+    case 128: return conv_k<T, 128>(a, backward);
+    case 256: return conv_k<T, 256>(a, backward);
   }
   return hipErrorInvalidValue;
 }

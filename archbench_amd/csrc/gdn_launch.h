@@ -103,24 +103,26 @@ hipError_t launch_seg_scan(const float* phi, const float* loc, const float* init
 bool chunk_shape_supported(int K, int V, int dtype);
 bool step_shape_supported(int K, int V);
 
-// Short causal convolution + SiLU (+ per-group L2 normalisation), gdn_conv.hip.
+// Short causal convolution + SiLU (+ per-group L2 normalisation), gdn_conv.hip.  The channels of x are up to three
+// consecutive column groups of n[i] channels (n[1] = n[2] = 0: one), each with its own contiguous [B, T, n[i]] tensor
+// for y and dy; the first `normed` groups are normalised.  D = n[0] + n[1] + n[2].
 struct ConvArgs {
   const void* x;          // [B, T] rows of D channels, ldx elements apart (ldx >= D)
   const float* w;         // [D, W]
   const float* bias;      // [D] or null
   const void* state_in;   // [B, D, W-1] or null (zeros)
-  void* y;                // [B, T, D] (forward)
+  void* y[3];             // [B, T, n[i]] (forward)
   void* state_out;        // [B, D, W-1] or null (forward)
-  const void* dy;         // backward
+  const void* dy[3];      // backward
   void* dx;               // [B, T] rows of D channels, lddx elements apart
   void* dstate_in;        // or null
   float *dw, *dbias;      // dbias may be null
   void* ws;
-  int B, T, D, norm_group, dtype;
+  int B, T, n[3], normed, norm_group, dtype;
   int64_t ldx, lddx;  // row strides of x and dx (>= D)
   hipStream_t stream;
 };
-size_t conv_ws_bytes(int B, int T, int D, int W);
+size_t conv_ws_bytes(int B, int T, const int (&n)[3], int W);
 bool conv_shape_supported(int D, int W, int norm_group);
 hipError_t launch_conv(const ConvArgs& a, bool backward);
 

@@ -659,34 +659,21 @@ def short_conv_bwd(x: Tensor, w: Tensor, bias: Optional[Tensor], state: Optional
     """(dx, dw [D,W] fp32, dbias [D] fp32, dstate [B,D,W-1]); dbias / dstate are zeros-shaped if not needed."""
     _require_gpu(x, w, bias, state, dy)
     B, T, D, W = _conv_shapes(x, w, bias, state)
-    dx = x.new_empty(B, T, D)
-    dw, db, dstate = _conv_bwd_launch(x, w, bias, state, dy, dx, D, norm_group)
-    return dx, dw, db, dstate
-
-
-def _conv_bwd_launch(x: Tensor, w: Tensor, bias: Optional[Tensor], state: Optional[Tensor], dy: Tensor, dx: Tensor,
-                     lddx: int, norm_group: int, dw: Optional[Tensor] = None) -> tuple[Tensor, Tensor, Tensor]:
-    """The conv backward into dx, whose tokens lie lddx elements apart (dx may be a column slice of a wider
-    gradient), and into dw when given (contiguous fp32 [D, W], e.g. a row slice of a larger weight gradient);
-    returns (dw, dbias, dstate)."""
-    B, T, D, W = _conv_shapes(x, w, bias, state)
     lib = _lib.load()
     dy = _arg(dy, x.dtype)
+    dx = x.new_empty(B, T, D)
     x, ldx = _token_rows(x)
     w, bias, state = _arg(w, torch.float32), _arg(bias, torch.float32), _arg(state, x.dtype)
-    if dw is None:
-        dw = torch.empty(D, W, dtype=torch.float32, device=x.device)
-    elif dw.shape != (D, W) or dw.dtype != torch.float32 or not dw.is_contiguous() or dw.data_ptr() % 16:
-        raise ValueError(f"dw must be a contiguous 16-byte aligned fp32 [{D}, {W}] tensor")
+    dw = torch.empty(D, W, dtype=torch.float32, device=x.device)
     db = torch.empty(D, dtype=torch.float32, device=x.device)
     dstate = torch.empty(B, D, W - 1, dtype=x.dtype, device=x.device)
     ws = _lib.workspace(x.device, _lib.conv_ws_bytes(B, T, D, W))
     rc = lib.gdn_short_conv_bwd(_lib.ptr(x), ldx, _lib.ptr(w), _lib.ptr(bias), _lib.ptr(state), _lib.ptr(dy),
-                                _lib.ptr(dx), lddx, _lib.ptr(dw), _lib.ptr(db), _lib.ptr(dstate), _lib.ptr(ws),
+                                _lib.ptr(dx), D, _lib.ptr(dw), _lib.ptr(db), _lib.ptr(dstate), _lib.ptr(ws),
                                 ws.numel(), B, T, D, W, int(norm_group), _lib.dtype_code(x.dtype),
                                 _lib.stream_ptr(x.device))
     _lib.check(rc, "gdn_short_conv_bwd")
-    return dw, db, dstate
+    return dx, dw, db, dstate
 
 
 @short_conv_bwd.register_fake
@@ -729,16 +716,16 @@ short_conv.register_autograd(_conv_backward, setup_context=_conv_setup)
 
 # The mixer's input stage in one op: q, k and v convolved straight out of the q/k/v input projection's output y
 # [B, T, 2 key_dim + value_dim] (its column groups, read in place), with one weight [2 key_dim + value_dim, W] for
-# the three convolutions (q's rows, then k's, then v's).  The backward writes dq, dk, dv's input gradients into the
-# column slices of one dy and the three weight gradients into the row slices of one dw, so no gradient of a split
-# or of a concatenation costs a pass (the conv backward takes dx's row stride).
+# the three convolutions (q's rows, then k's, then v's), in one launch.  The backward, one launch and the sum of its
+# partial weight gradients, writes the three input gradients into the column groups of one dy and the weight gradients
+# into one dw, so no gradient of a split or of a concatenation costs a pass.
 def _stage_dims(y: Tensor, w: Tensor, key_dim: int, value_dim: int):
     n = 2 * key_dim + value_dim
     if y.dim() != 3 or y.shape[-1] != n:
         raise ValueError(f"y must be [B, T, 2 key_dim + value_dim = {n}], got {tuple(y.shape)}")
     if w.dim() != 2 or w.shape[0] != n:
         raise ValueError(f"w must be [2 key_dim + value_dim = {n}, W], got {tuple(w.shape)}")
-    return (0, key_dim), (key_dim, key_dim), (2 * key_dim, value_dim)
+    return y.shape[0], y.shape[1], n, w.shape[1]
 
 
 @torch.library.custom_op("archbench_amd::mixer_input_stage", mutates_args=())
@@ -747,10 +734,14 @@ def mixer_input_stage(y: Tensor, w: Tensor, key_dim: int, value_dim: int,
     """(q, k, v): silu(causal conv(.)) of y's q, k and v columns (q and k L2-normalised per norm_group channels;
     conv weights fp32, used rounded to y's dtype; no bias, no state)."""
     _require_gpu(y, w)
-    cols = _stage_dims(y, w, key_dim, value_dim)
-    w = _arg(w, torch.float32)
-    return tuple(short_conv(y[..., c0:c0 + d], w[c0:c0 + d], None, None, ng)[0]
-                 for (c0, d), ng in zip(cols, (norm_group, norm_group, 0)))
+    B, T, _, W = _stage_dims(y, w, key_dim, value_dim)
+    lib = _lib.load()
+    y, w = _arg(y), _arg(w, torch.float32)
+    q, k, v = y.new_empty(B, T, key_dim), y.new_empty(B, T, key_dim), y.new_empty(B, T, value_dim)
+    rc = lib.gdn_mixer_stage_fwd(_lib.ptr(y), _lib.ptr(w), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, T, key_dim,
+                                 value_dim, W, int(norm_group), _lib.dtype_code(y.dtype), _lib.stream_ptr(y.device))
+    _lib.check(rc, "gdn_mixer_stage_fwd")
+    return q, k, v
 
 
 @mixer_input_stage.register_fake
@@ -764,13 +755,20 @@ def mixer_input_stage_bwd(y: Tensor, w: Tensor, dq: Tensor, dk: Tensor, dv: Tens
                           norm_group: int) -> tuple[Tensor, Tensor]:
     """(dy, dw): the three conv backwards written into dy's column slices and dw's row slices (dw fp32)."""
     _require_gpu(y, w, dq, dk, dv)
-    cols = _stage_dims(y, w, key_dim, value_dim)
-    w = _arg(w, torch.float32)
-    B, T, L = y.shape
-    dy = y.new_empty(B, T, L)
-    dw = torch.empty(w.shape, dtype=torch.float32, device=w.device)
-    for (c0, d), g, ng in zip(cols, (dq, dk, dv), (norm_group, norm_group, 0)):
-        _conv_bwd_launch(y[..., c0:c0 + d], w[c0:c0 + d], None, None, g, dy[..., c0:c0 + d], L, ng, dw[c0:c0 + d])
+    B, T, D, W = _stage_dims(y, w, key_dim, value_dim)
+    for n, g, d in (("dq", dq, key_dim), ("dk", dk, key_dim), ("dv", dv, value_dim)):
+        if tuple(g.shape) != (B, T, d):
+            raise ValueError(f"{n} must be [B, T, {d}] = {(B, T, d)}, got {tuple(g.shape)}")
+    lib = _lib.load()
+    y, w = _arg(y), _arg(w, torch.float32)
+    dq, dk, dv = _arg(dq, y.dtype), _arg(dk, y.dtype), _arg(dv, y.dtype)
+    dy = torch.empty_like(y)
+    dw = torch.empty(D, W, dtype=torch.float32, device=w.device)
+    ws = _lib.workspace(y.device, _lib.stage_ws_bytes(B, T, key_dim, value_dim, W))
+    rc = lib.gdn_mixer_stage_bwd(_lib.ptr(y), _lib.ptr(w), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(dy),
+                                 _lib.ptr(dw), _lib.ptr(ws), ws.numel(), B, T, key_dim, value_dim, W,
+                                 int(norm_group), _lib.dtype_code(y.dtype), _lib.stream_ptr(y.device))
+    _lib.check(rc, "gdn_mixer_stage_bwd")
     return dy, dw
 
 

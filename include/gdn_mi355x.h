@@ -157,6 +157,17 @@ int gdn_short_conv_bwd(const void* x, int64_t ldx, const float* w, const float* 
                        const void* dy, void* dx, int64_t lddx, float* dw, float* dbias, void* dstate_in, void* ws,
                        size_t ws_bytes, int B, int T, int D, int W, int norm_group, int dtype, void* stream);
 
+/* The mixer's input stage: the three short convolutions above (no bias, no state) in one launch each way.  y
+ * [B, T, 2 key_dim + value_dim] holds q's, k's and v's channels (a fused input projection's output), w
+ * [2 key_dim + value_dim, W] their taps in the same order; q, k [B, T, key_dim] (normalised per norm_group channels)
+ * and v [B, T, value_dim] are written, or their gradients read and dy, dw written. */
+int gdn_mixer_stage_fwd(const void* y, const float* w, void* q, void* k, void* v, int B, int T, int key_dim,
+                        int value_dim, int W, int norm_group, int dtype, void* stream);
+int gdn_mixer_stage_bwd_ws_bytes(int B, int T, int key_dim, int value_dim, int W, size_t* bytes);
+int gdn_mixer_stage_bwd(const void* y, const float* w, const void* dq, const void* dk, const void* dv, void* dy,
+                        float* dw, void* ws, size_t ws_bytes, int B, int T, int key_dim, int value_dim, int W,
+                        int norm_group, int dtype, void* stream);
+
 /* Gated RMSNorm of the op's output, per row of `dim` channels (one head of one token):
  *   y = x * rsqrt(mean(x^2) + eps) * weight * silu(gate)
  * Replaces the output normalisation of the mixer: fla's FusedRMSNormGated in GatedDeltaNet and the reference's

@@ -228,8 +228,8 @@ def test_conv_taps_rounded_to_activation_dtype():
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_conv_backward_long_chunks_match_oracle(dtype):
-    """Without normalisation a large grid takes the backward's 128-token waves (at least four waves per CU): a
-    ragged last chunk (T = 4000 = 31 * 128 + 32), bias and conv state, against the oracle."""
+    """A large grid's backward without normalisation, over many chunks per sequence: a ragged last chunk (T = 4000 =
+    62 * 64 + 32 = 31 * 128 + 32), bias and conv state, against the oracle."""
     B, T, D = 4, 4000, 2048
     waves_long = (D // 256) * B * -(-T // 128)
     if waves_long < 4 * torch.cuda.get_device_properties(0).multi_processor_count:
@@ -244,3 +244,34 @@ def test_conv_backward_long_chunks_match_oracle(dtype):
     _check(dw, dw_ref, dtype, "dw")
     _check(db, db_ref, dtype, "dbias")
     _check(dst, dst_ref, dtype, "dstate")
+
+
+@pytest.mark.parametrize("B,T,kd,vd,ng", [
+    (1, 5, 64, 128, 64),       # shorter than a batch of rows
+    (2, 8, 128, 256, 128),     # one whole batch
+    (1, 203, 384, 768, 128),   # 8-token waves, half-empty channel blocks, a ragged end
+    (3, 1003, 384, 512, 128),  # 8-token waves forward, 16 backward
+    (6, 777, 512, 1024, 256),  # 32-token waves in the backward
+    (12, 1021, 1024, 512, 64),   # 64-token waves
+    (16, 2050, 1024, 2048, 128),  # 128-token waves in the backward, two tokens past the last
+])
+def test_mixer_input_stage_chunk_lengths(B, T, kd, vd, ng):
+    """The stage at the token-chunk lengths its grid rule picks, forward and backward, on one normalisation group of
+    each of its column groups (the convolutions are depthwise) at the ends of their column ranges against the oracle."""
+    banner(f"mixer input stage chunk lengths B={B} T={T} kd={kd} vd={vd} ng={ng}")
+    gen = torch.Generator("cuda").manual_seed(13)
+    L = 2 * kd + vd
+    y = torch.randn(B, T, L, device="cuda", generator=gen).bfloat16()
+    w = (torch.randn(L, W, device="cuda", generator=gen) * 0.5).bfloat16().float()
+    grads = [torch.randn(B, T, d, device="cuda", generator=gen).bfloat16() for d in (kd, kd, vd)]
+    outs = ops.mixer_input_stage(y, w, kd, vd, ng)
+    dy, dw = ops.mixer_input_stage_bwd(y, w, *grads, kd, vd, ng)
+    torch.cuda.synchronize()
+    for g0, d, norm, o, gr in zip((0, kd, 2 * kd), (kd, kd, vd), (ng, ng, 0), outs, grads):
+        c0 = d - 64 if not norm else d - norm
+        cols = slice(g0 + c0, g0 + d)
+        xs, ws, gs = y[..., cols].float().cpu(), w[cols].cpu(), gr[..., c0:].float().cpu()
+        _check(o[..., c0:], CO.short_conv_fwd(xs, ws, None, None, norm)[0], torch.bfloat16, "y")
+        dx_ref, dw_ref, _, _ = CO.short_conv_bwd(xs, ws, None, None, gs, norm)
+        _check(dy[..., cols], dx_ref, torch.bfloat16, "dx")
+        _check(dw[cols], dw_ref, torch.bfloat16, "dw")
