@@ -875,6 +875,37 @@ int gdn_cross_entropy_fwd_bwd(void* logits, const int64_t* target, float* loss, 
   return GDN_OK;
 }
 
+// elementwise passes: a grid of 2048-element workgroups
+static int stream_check(int64_t n, int dtype) {
+  if (dtype != DT_F32 && dtype != DT_BF16) return fail(GDN_ERR_ARG, "dtype code %d is not GDN_DTYPE_F32/BF16", dtype);
+  if (n < 0 || n > (int64_t)INT32_MAX * 2048) return fail(GDN_ERR_ARG, "invalid n=%lld", (long long)n);
+  return GDN_OK;
+}
+
+int gdn_scale(const void* x, const float* s, void* y, int64_t n, int dtype, void* stream) {
+  g_err[0] = 0;
+  if (int e = stream_check(n, dtype)) return e;
+  if (n == 0) return GDN_OK;
+  if (!x || !s || !y) return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(x, y)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  const hipError_t e = launch_scale(x, s, y, n, dtype, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "scale launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
+int gdn_sum_parts(const float* part, int nparts, void* out, int64_t n, int dtype, void* stream) {
+  g_err[0] = 0;
+  if (int e = stream_check(n, dtype)) return e;
+  if (nparts < 1 || n % 8 != 0) return fail(GDN_ERR_ARG, "nparts=%d must be >= 1 and n=%lld a multiple of 8", nparts,
+                                            (long long)n);
+  if (n == 0) return GDN_OK;
+  if (!part || !out) return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(part, out)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  const hipError_t e = launch_sum_parts(part, nparts, out, n, dtype, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "sum of parts launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
 static int write_dir_check(int B, int T, int H, int K, int n_steps, int dtype) {
   if (dtype != DT_F32 && dtype != DT_BF16) return fail(GDN_ERR_ARG, "dtype code %d is not GDN_DTYPE_F32/BF16", dtype);
   if (B < 0 || T < 0 || H <= 0 || K <= 0) return fail(GDN_ERR_ARG, "invalid sizes B=%d T=%d H=%d K=%d", B, T, H, K);

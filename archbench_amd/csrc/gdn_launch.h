@@ -193,6 +193,9 @@ struct CeArgs {
 };
 bool ce_shape_supported(int V, int64_t ld);
 hipError_t launch_ce(const CeArgs& a);
+// y = *s x over n elements; out = sum over nparts of part[p][n] (n a multiple of 8), rounded to dtype
+hipError_t launch_scale(const void* x, const float* s, void* y, int64_t n, int dtype, hipStream_t st);
+hipError_t launch_sum_parts(const float* part, int nparts, void* out, int64_t n, int dtype, hipStream_t st);
 
 // Write direction of the n-step family (gdn_writedir.hip): k [B,T,H,K] -> u, and the backward.
 struct WriteDirArgs {

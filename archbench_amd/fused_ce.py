@@ -2,13 +2,13 @@
 
 Same interface and arithmetic as archbench/fused_ce.py:20-57 (``fused_linear_cross_entropy(x, target, weight,
 num_chunks=8, ignore_index=-100)`` -> mean token cross-entropy; the forward computes every gradient and the
-backward only scales them).  Per chunk of rows: logits = x W^T and the two gradient products dx = dlogits W,
-dW += dlogits^T x (fp32 accumulation) are plain library GEMMs (hipBLASLt through torch.mm / addmm); between them
-one HIP kernel (``ops.cross_entropy_fwd_bwd_``) computes each row's loss and overwrites the logits with
-dloss * (softmax - onehot), reading and writing the chunk once.  With 288 GB of HBM a chunk of 2048 rows x 50304
-classes (206 MB in bf16) is cheap to hold, so the logits are kept rather than recomputed -- and even one chunk
-for 32768 tokens (3.3 GB): with ``num_chunks=1`` the weight gradient comes straight out of one bf16-output GEMM
-instead of fp32 accumulation across chunks, the fastest configuration on MI355X.
+backward only scales them).  Per pass of rows: logits = x W^T and the two gradient products dx = dlogits W,
+dW += dlogits^T x (fp32 accumulation) are plain library GEMMs (hipBLASLt through torch); between them one HIP kernel
+(``ops.cross_entropy_fwd_bwd_``) computes each row's loss and overwrites the logits with
+dloss * (softmax - onehot), reading and writing the chunk once.  ``num_chunks`` bounds the memory: a pass takes the
+rows of one chunk and as many more as fit in the room that the accumulation in place saves (_rows_per_pass).  With
+288 GB of HBM even one chunk for 32768 tokens (3.3 GB of logits) is cheap to hold; with one pass the weight gradient
+comes straight out of one GEMM in the weight's dtype, the fastest configuration on MI355X.
 """
 
 from __future__ import annotations
@@ -27,38 +27,83 @@ def fused_ce_available() -> bool:
     return True
 
 
+_TILE = 256  # rows and columns of the GEMMs' output tiles
+
+
+def _rows_per_pass(N: int, num_chunks: int, d: int, es: int) -> int:
+    """Rows per pass: a chunk's ceil(N / num_chunks), plus what fits in the memory a second fp32 copy of dW [V, d] would
+    take (an accumulation out of place held one): two thirds of it as logits [rows, V] of es bytes, the last third left
+    for dx's partial products (_dx_split).  Every pass reads and writes dW once and runs products of its rows' size:
+    N = 8192, d = 1024, V = 50304 in eight passes of 1024 rows took 6.2 ms (dx on 80 of 256 CUs, 72 us a pass copying
+    dW), in four of 2048 3.3 ms."""
+    C = -(-N // num_chunks)
+    if C >= N:
+        return max(N, 1)
+    most = C + 8 * d // (3 * es)
+    rows = -(-N // -(-N // most))
+    return min(most, -(-rows // _TILE) * _TILE, N)
+
+
+def _dx_split(rows: int, d: int, V: int) -> int:
+    """Parts of the contraction over V in dx = dlogits W: as one product it has rows/256 x d/256 output tiles for 256
+    CUs (rows 2048, d 1024: 32, 308 us); in S parts, batched and summed in fp32, S times as many (S = 8: 197 us).  The
+    parts hold whole 16-byte pieces of a row and take at most a third of dW's fp32 size."""
+    if rows == 0:
+        return 1
+    tiles = -(-rows // _TILE) * -(-d // _TILE)
+    S = min(256 // tiles, V // (3 * rows), 16)
+    while S > 1 and V % (8 * S):
+        S -= 1
+    return max(S, 1)
+
+
+def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> None:
+    """out [rows, d] = dlogits [rows, V] W [V, d]."""
+    rows, V = dlogits.shape
+    d = weight.shape[1]
+    # 16-byte rows throughout; not under an autocast that would change a dtype
+    split = dlogits.dtype == weight.dtype == out.dtype == torch.bfloat16 and d % 8 == 0 and weight.is_contiguous()
+    S = _dx_split(rows, d, V) if split else 1
+    if S == 1:
+        out.copy_(dlogits @ weight)
+        return
+    parts = torch.bmm(dlogits.view(rows, S, V // S).transpose(0, 1), weight.view(S, V // S, d),
+                      out_dtype=torch.float32)
+    ops.sum_parts_(parts, out)
+
+
 class _FusedLinearCE(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, target, weight, num_chunks: int, ignore_index: int):
-        N, _ = x.shape
-        C = -(-N // num_chunks)
+        N, d = x.shape
+        C = _rows_per_pass(N, num_chunks, d, x.element_size())
         total = target.ne(ignore_index).sum().clamp_min(1)
         dloss = total.float().reciprocal().reshape(1)  # device scalar: no host sync
         loss_rows = torch.empty(N, device=x.device, dtype=torch.float32)
         dx = torch.empty_like(x)
-        if C >= N:
-            # one chunk: dW needs no accumulation across chunks, so the GEMM writes it in the weight's dtype
-            # directly (fp32 accumulation inside, one rounding -- where the chunked path rounds at the end)
-            logits = x @ weight.t()
-            loss_rows = ops.cross_entropy_fwd_bwd_(logits, target, dloss, ignore_index)[0]
-            dx = logits @ weight
-            dw = logits.t() @ x
-        else:
-            dw = torch.zeros(weight.shape, device=x.device, dtype=torch.float32)
-            for s in range(0, N, C):
-                e = min(s + C, N)
-                c_x = x[s:e]
-                logits = c_x @ weight.t()
-                loss_rows[s:e] = ops.cross_entropy_fwd_bwd_(logits, target[s:e], dloss, ignore_index)[0]
-                dx[s:e] = logits @ weight
-                dw = torch.addmm(dw, logits.t(), c_x, out_dtype=torch.float32)
+        dw = None
+        for s in range(0, max(N, 1), C):
+            e = min(s + C, N)
+            c_x = x[s:e]
+            logits = c_x @ weight.t()
+            loss_rows[s:e] = ops.cross_entropy_fwd_bwd_(logits, target[s:e], dloss, ignore_index)[0]
+            _dx(logits, weight, dx[s:e])
+            if C >= N:
+                # one pass: dW needs no accumulation across passes, so the GEMM writes it in the weight's dtype
+                # directly (fp32 accumulation inside, one rounding -- where several passes round at the end)
+                dw = logits.t() @ c_x
+            elif dw is None:
+                dw = torch.mm(logits.t(), c_x, out_dtype=torch.float32)
+            else:  # in place
+                torch.addmm(dw, logits.t(), c_x, out_dtype=torch.float32, out=dw)
+            del logits
         ctx.save_for_backward(dx, dw.to(weight.dtype))
         return loss_rows.sum() / total
 
     @staticmethod
     def backward(ctx, dout):
         dx, dw = ctx.saved_tensors
-        return dx * dout, None, dw * dout, None, None
+        return ops.scaled(dx, dout), None, ops.scaled(dw, dout), None, None
 
 
 def fused_linear_cross_entropy(x, target, weight, num_chunks: int = 8, ignore_index: int = -100):

@@ -1123,6 +1123,55 @@ def _(logits, target, dloss, ignore_index):
     return logits.new_empty(N, dtype=torch.float32), logits.new_empty(N, dtype=torch.float32)
 
 
+@torch.library.custom_op("archbench_amd::scaled", mutates_args=())
+def scaled(x: Tensor, s: Tensor) -> Tensor:
+    """s x for a device scalar s (one element), in x's dtype with the product in fp32."""
+    _require_gpu(x, s)
+    if s.numel() != 1:
+        raise ValueError(f"s must hold one element, got {tuple(s.shape)}")
+    x, s = _arg(x), s.float()
+    y = torch.empty_like(x)
+    rc = _lib.load().gdn_scale(_lib.ptr(x), _lib.ptr(s), _lib.ptr(y), x.numel(), _lib.dtype_code(x.dtype),
+                               _lib.stream_ptr(x.device))
+    _lib.check(rc, "gdn_scale")
+    return y
+
+
+@scaled.register_fake
+def _(x, s):
+    return torch.empty_like(x)
+
+
+def _scaled_setup(ctx, inputs, output):
+    ctx.save_for_backward(*inputs)
+
+
+def _scaled_backward(ctx, dy):
+    x, s = ctx.saved_tensors
+    return scaled(dy, s), (dy.float() * x.float()).sum().reshape(s.shape).to(s.dtype)
+
+
+scaled.register_autograd(_scaled_backward, setup_context=_scaled_setup)
+
+
+@torch.library.custom_op("archbench_amd::sum_parts_", mutates_args=("out",))
+def sum_parts_(parts: Tensor, out: Tensor) -> None:
+    """out (contiguous, bf16 or fp32) <- the sum over parts' first dimension (fp32, contiguous), rounded once."""
+    _require_gpu(parts, out)
+    if parts.dtype != torch.float32 or parts.shape[1:] != out.shape or not (parts.is_contiguous()
+                                                                           and out.is_contiguous()):
+        raise ValueError(f"parts must be contiguous fp32 [S, *out.shape], got {parts.dtype} {tuple(parts.shape)} for "
+                         f"{tuple(out.shape)}")
+    rc = _lib.load().gdn_sum_parts(_lib.ptr(parts), parts.shape[0], _lib.ptr(out), out.numel(),
+                                   _lib.dtype_code(out.dtype), _lib.stream_ptr(out.device))
+    _lib.check(rc, "gdn_sum_parts")
+
+
+@sum_parts_.register_fake
+def _(parts, out):
+    return None
+
+
 # ------------------------------------------------------------------------------------------------- decode step
 @torch.library.custom_op("archbench_amd::gdn_recurrent_step", mutates_args=("state",))
 def _recurrent_step(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state: Tensor,

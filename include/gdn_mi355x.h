@@ -222,6 +222,11 @@ int gdn_gates_bwd(const void* a, const void* b, int64_t lda, const float* A_log,
 int gdn_cross_entropy_fwd_bwd(void* logits, const int64_t* target, float* loss, float* lse, const float* dloss,
                               int64_t N, int V, int64_t ld, int64_t ignore_index, int dtype, void* stream);
 
+/* The streaming passes around the fused loss's matrix products: y = *s x (s a device scalar) over n elements of dtype,
+ * and out = sum over p < nparts of part[p * n + i] (fp32, p ascending), rounded once to dtype (n a multiple of 8). */
+int gdn_scale(const void* x, const float* s, void* y, int64_t n, int dtype, void* stream);
+int gdn_sum_parts(const float* part, int nparts, void* out, int64_t n, int dtype, void* stream);
+
 /* Write direction of the n-step family: per token row of K channels (one head of one token), with p the previous
  * token's key in the same sequence (zero at t = 0),
  *   u_1 = beta k,  u_{i+1} = u_i - lam beta (p . u_i) (p - (p . k) k)   for i < n_steps.

@@ -65,3 +65,46 @@ def test_fused_linear_ce_matches_oracle(num_chunks, V):
     assert rel_l2(xd.grad.reshape(-1, H), dx_r) <= 1e-2
     assert rel_l2(wd.grad, dw_r) <= 1e-2
     assert wd.grad.shape == w.shape and xd.grad.shape == x.shape
+
+
+@pytest.mark.parametrize("N,H,V,num_chunks", [
+    (700, 256, 4096, 8),   # two passes, the second ragged; dx in two parts
+    (1100, 128, 8192, 8),  # four passes; dx in eight parts
+    (257, 64, 1000, 4),    # a vocabulary that allows no parts
+    (90, 512, 16384, 1),   # one pass; dx in sixteen parts
+])
+def test_fused_linear_ce_passes_and_parts(N, H, V, num_chunks):
+    """The rows per pass, the accumulation of dW across passes and the parts of dx against the oracle."""
+    rows = fused_ce._rows_per_pass(N, num_chunks, H, 2)
+    banner(f"fused linear CE N={N} H={H} V={V}: {rows} rows per pass, {fused_ce._dx_split(rows, H, V)} parts")
+    gen = torch.Generator().manual_seed(N)
+    x = torch.randn(1, N, H, generator=gen).bfloat16()
+    w = (torch.randn(V, H, generator=gen) * 0.05).bfloat16()
+    t = torch.randint(0, V, (1, N), generator=gen)
+    t[0, ::9] = -100
+    xd, wd = x.cuda().requires_grad_(), w.cuda().requires_grad_()
+    loss = fused_ce.fused_linear_cross_entropy(xd, t.cuda(), wd, num_chunks=num_chunks)
+    (3.0 * loss).backward()
+    l_r, dx_r, dw_r = CE.linear_ce(x.float().reshape(-1, H), t.reshape(-1), w.float())
+    assert abs(loss.item() - l_r.item()) <= 1e-3 * abs(l_r.item())
+    assert rel_l2(xd.grad.reshape(-1, H), 3.0 * dx_r) <= 1e-2
+    assert rel_l2(wd.grad, 3.0 * dw_r) <= 1e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("n,S", [(1, 1), (8, 3), (1001, 2), (4096, 16)])
+def test_scale_and_sum_of_parts(dtype, n, S):
+    """ops.scaled equals the product in fp32 rounded once, ops.sum_parts_ the ordered fp32 sum rounded once, exactly."""
+    banner(f"scaled / sum of parts n={n} S={S} {dtype}")
+    gen = torch.Generator("cuda").manual_seed(n)
+    x = torch.randn(n, device="cuda", generator=gen).to(dtype)
+    s = torch.tensor(0.37, device="cuda")
+    assert torch.equal(ops.scaled(x, s), (x.float() * s).to(dtype))
+    if n % 8 == 0:
+        parts = torch.randn(S, n, device="cuda", generator=gen)
+        ref = torch.zeros(n, device="cuda")
+        for p in parts:
+            ref += p
+        out = torch.empty(n, device="cuda", dtype=dtype)
+        ops.sum_parts_(parts, out)
+        assert torch.equal(out, ref.to(dtype))
