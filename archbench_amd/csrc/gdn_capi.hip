@@ -951,7 +951,7 @@ int gdn_write_direction_bwd(const void* k, const float* beta, const float* lam, 
 static int token_scan_check(int B, int T, int H, int K, int V) {
   if (B < 0 || T < 0 || H <= 0 || V <= 0) return fail(GDN_ERR_ARG, "invalid sizes B=%d T=%d H=%d V=%d", B, T, H, V);
   if (!token_scan_supported(K)) return fail(GDN_ERR_SHAPE, "token scan not compiled for K=%d (K in {64, 128})", K);
-  if ((int64_t)B * H * ((V + 63) / 64) > INT32_MAX) return fail(GDN_ERR_ARG, "grid too large");
+  if ((int64_t)B * H * ((V + 31) / 32) > INT32_MAX) return fail(GDN_ERR_ARG, "grid too large");
   return GDN_OK;
 }
 
@@ -960,10 +960,10 @@ int gdn_token_scan_sizes(int B, int T, int H, int K, int V, size_t* st_bytes, si
   g_err[0] = 0;
   if (int e = token_scan_check(B, T, H, K, V)) return e;
   if (!st_bytes || !scratch_bytes || !n_partials) return fail(GDN_ERR_ARG, "null output pointer");
-  const size_t NB = (size_t)(V + 63) / 64, NCH = (size_t)(T + token_scan_ct() - 1) / token_scan_ct();
+  const size_t NCH = (size_t)(T + token_scan_ct() - 1) / token_scan_ct();
   *st_bytes = (size_t)B * H * NCH * K * V * 4;
-  *scratch_bytes = (size_t)B * H * NB * token_scan_scratch_floats(K) * 4;
-  *n_partials = (int)NB;
+  *scratch_bytes = token_scan_scratch_floats(B, T, H, K, V) * 4;
+  *n_partials = token_scan_row_blocks(B, T, H, K, V);
   return GDN_OK;
 }
 
@@ -997,7 +997,7 @@ int gdn_token_scan_bwd(const float* q, const float* k, const float* u, const flo
   if ((int64_t)B * T == 0) return GDN_OK;
   if (!q || !k || !u || !la || !r || !st || !dy || !dv || !dq_part || !du_part || !dk_part || !dla_part || !scratch)
     return fail(GDN_ERR_ARG, "null input/output pointer");
-  if (misaligned(q, k, u, dhT, dh0)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  if (misaligned(q, k, u, dhT, dh0, dq_part, du_part, dk_part, scratch)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
   if (st_bytes < need_st) return fail(GDN_ERR_WORKSPACE, "checkpoint buffer %zu bytes, need %zu", st_bytes, need_st);
   if (scratch_bytes < need_sc)
     return fail(GDN_ERR_WORKSPACE, "scratch %zu bytes, need %zu", scratch_bytes, need_sc);

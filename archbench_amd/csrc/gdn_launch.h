@@ -224,7 +224,9 @@ struct TokenScanArgs {
 };
 bool token_scan_supported(int K);
 int token_scan_ct();
-size_t token_scan_scratch_floats(int K);  // backward scratch per (b, h, 64-row block)
+// the backward's row blocks per head (its partial rows per token) and its scratch
+int token_scan_row_blocks(int B, int T, int H, int K, int V);
+size_t token_scan_scratch_floats(int B, int T, int H, int K, int V);
 hipError_t launch_token_scan(const TokenScanArgs& a, bool backward);
 
 // Compute units of the current device (cached per device; 256 if the query fails).

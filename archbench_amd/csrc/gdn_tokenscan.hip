@@ -2,35 +2,51 @@
 // "triton" / "ref" scan (archbench/layers/nsgdn.py:80-154, ops :162-216; the recurrence of nsgdn_ref, :408-417).
 // Per token t of a (b, h) sequence, with the state S [V, K] fp32 from zero (or from an initial state):
 //     S <- e^{la_t} S;   r_t = v_t - S k_t;   S <- S + r_t u_t^T;   y_t = S q_t.
-// Rows of S are independent given the token stream.  A workgroup of eight waves owns 64 rows; eight lanes share a
-// row, lane part l & 7 holding K / 8 of its entries in registers, so a row's dot products (S k, S q, G u) are a
-// partial sum per lane and three DPP steps inside the 8-lane group.  k, u, q of a token are workgroup-uniform and
-// reach the lanes through LDS, staged a block of tokens at a time (double-buffered: the next block is staged while
-// one computes, one barrier per block).  Every CT tokens the forward stores S (the checkpoint the backward restarts
-// from) in [K][V] order.
+// Rows of S are independent given the token stream.  Sixteen lanes (one DPP row) share RL rows of S, lane part
+// p = l & 15 holding K / 16 entries of each in registers, so a row's dot products (S k, S q, G u) are a partial sum per
+// lane and four DPP steps.  k, u, q of a token are workgroup-uniform and reach the lanes through LDS, staged a block of
+// tokens at a time (double-buffered: the next block is staged while one computes, one barrier per block).  A row's
+// per-token scalars (v; r and dy in the backward) are loaded once per block, one token per lane, and broadcast inside
+// the DPP row (row_newbcast); e^{la} is computed by one lane per token and read with readlane; a block's results are
+// kept by the lane of their token and leave in one store.  So the chain from token to token is a handful of
+// arithmetic steps: no load, store, transcendental or branch stands in it.
+// Every CT tokens the forward stores S (the checkpoint the backward restarts from) in [K][V] order.
 // The backward walks the checkpoints in reverse and each chunk in groups of four tokens, last first: it recomputes
 // a group's states forward from the state entering the group (stored by a forward pass over the chunk from its
 // checkpoint), keeping e^{la} S before each token's update in registers and accumulating dq = sum_rows S_t^T dy_t,
 // then runs the group's tokens backward with the state gradient G [V, K] in registers beside S:
 //     G += dy_t q_t^T;  dv_t = G u_t;  du_t = sum_rows G r_t;  G -= dv_t k_t^T;
 //     dk_t = -sum_rows (e^{la} S_{t-1}) dv_t;  dla_t = sum (G o e^{la} S_{t-1});  G <- e^{la_t} G.
-// Sums over rows are a reduce-scatter over the wave's 8 rows (lane swaps and DPP, no LDS crossbar), then over the
-// eight waves through LDS (a fixed order, no atomics), then over a head's V / 64 workgroups through partial rows that
-// the host adds.
+// Sums over rows are formed over a lane's own rows, then a reduce-scatter over the wave's four row groups (lane swaps,
+// no LDS crossbar), then over the waves through LDS (a fixed order, no atomics), then over a head's workgroups through
+// partial rows that are added afterwards.
+// Bound: the forward by that chain (per token at K = 128 about 0.24 us: two dot products and row sums, the update and
+// the reads between them) until a SIMD holds two waves or more, the backward by its arithmetic (its row sums over
+// the state's rows included) at one or two waves per SIMD.  Against eight lanes per row with the token's loads, stores,
+// expf and LDS row sums in the chain: B4 T1024 H4 K128 V256 forward 507 -> 241 us, backward 1916 -> 908 us.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
+#include <utility>
 
 #include "gdn_common.h"
 #include "gdn_launch.h"
 
 namespace gdn {
 
-constexpr int TS_CT = 32;                    // tokens between checkpoints
-constexpr int TS_GS = 4;                     // tokens per group of the backward (decayed states held in registers)
-constexpr int TS_ROWS = 64;                  // state rows per workgroup
-constexpr int TS_LB = 3;                     // log2 of the lanes per row (16 lanes: slower, spills)
-constexpr int TS_LPR = 1 << TS_LB;           // lanes per row
-constexpr int TS_THREADS = TS_LPR * TS_ROWS;
-constexpr int TS_WAVES = TS_THREADS / 64;    // each wave holds 64 / TS_LPR rows
+constexpr int TS_CT = 32;   // tokens between checkpoints
+constexpr int TS_GS = 4;    // tokens per group of the backward (decayed states held in registers)
+constexpr int TS_TB = 8;    // tokens per block of the forward
+constexpr int TS_LPR = 16;  // lanes per row: one DPP row
+static_assert(TS_CT % TS_TB == 0, "checkpoints fall on block starts");
+
+// A workgroup's share of the state: RL rows per lane, four row groups per wave
+template <int RL_, int WAVES_>
+struct TsShape {
+  static constexpr int RL = RL_, WAVES = WAVES_, THREADS = 64 * WAVES, WROWS = 4 * RL, ROWS = WROWS * WAVES;
+  static_assert(RL == 1 || RL == 2, "a group's row scalars fit the sixteen lanes of a row");
+  static_assert((WAVES & (WAVES - 1)) == 0, "the waves' sums are added as a binary tree");
+};
 
 // The block / group barrier orders LDS only (the staged vectors and the row sums): __syncthreads() would also wait
 // for every global load in flight, the next block's included, and so expose a memory latency per barrier.
@@ -39,286 +55,377 @@ __device__ __forceinline__ void ts_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
-// A zero the compiler cannot see through, added to a workgroup-uniform index so that the load is a vector load: a
-// scalar load would be waited for at the next barrier (scalar loads and LDS share one wait counter).
-__device__ __forceinline__ int ts_vector_zero() {
-  int z;
-  asm volatile("v_mov_b32 %0, 0" : "=v"(z));
-  return z;
+
+// f(integral_constant<0>), ..., f(integral_constant<N - 1>): DPP and readlane patterns need constant indexes
+template <typename F, int... I>
+__device__ __forceinline__ void ts_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void ts_for(F&& f) {
+  ts_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// sum over the lanes of a row, left in each of them: quad_perm [1,0,3,2], [2,3,0,1], then row_half_mirror (lane
-// p <- 7 - p) adds the other quad of an 8-lane group and row_mirror (p <- 15 - p) the other half of a 16-lane row
-__device__ __forceinline__ float ts_row_sum(float x) {
-  x = dpp_sum_step<0x4e>(dpp_sum_step<0xb1>(x));
-  if constexpr (TS_LB >= 3) x = dpp_sum_step<0x141>(x);
-  if constexpr (TS_LB >= 4) x = dpp_sum_step<0x140>(x);
+// lane I's value of each 16-lane row, in every lane of the row (row_newbcast:I)
+template <int I>
+__device__ __forceinline__ float ts_row_bcast(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x150 + I, 0xf, 0xf, true));
+}
+template <int I>
+__device__ __forceinline__ float ts_lane(float x) {  // lane I's value, uniform over the wave
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), I));
+}
+
+// `x` is kept as computed here: a select on a lane index would otherwise sink x's last steps under an exec-mask branch
+__device__ __forceinline__ float ts_pin(float x) {
+  asm volatile("" : "+v"(x));
   return x;
 }
 
-// Reduce-scatter over a wave's 64 / TS_LPR rows: N values per lane (its part's local columns), summed over the lanes
-// that share l & (TS_LPR - 1) (lane bits TS_LB .. 5).  With R = N TS_LPR / 64, lane l ends with the sums of local
-// columns m + R (l >> TS_LB), m < R, in a[0 .. R).  Each round pairs lanes that differ in one bit and hold the same column set: one keeps the lower
-// half of its set, the other the upper half, and each adds what its partner sends.
+// Reduce-scatter over a wave's four row groups: N values per lane (its part's columns, already summed over the lane's
+// rows), summed over the lanes that share l & 15.  With R = N / 4, lane l ends with the sums of columns
+// m + R (l >> 4), m < R, in a[0 .. R).  Each round pairs lanes that differ in one bit and hold the same column set: one
+// keeps the lower half of its set, the other the upper half, and each adds what its partner sends
+// (v_permlane32_swap of (a[m], a[m + N/2]) gives the lower half-wave its partner's a[m] and the upper half its partner's
+// a[m + N/2], each keeping its own in the other result, so one add finishes the round; v_permlane16_swap likewise
+// between even and odd 16-lane rows).
 template <int N>
-__device__ __forceinline__ void ts_rows_rs(float (&a)[N], int l) {
-  // bit 5: v_permlane32_swap of (a[m], a[m + N/2]) gives the lower half-wave its partner's a[m] and the upper half
-  // its partner's a[m + N/2] (each keeps its own in the other result), so one add finishes the round
+__device__ __forceinline__ void ts_rows_rs(float (&a)[N]) {
 #pragma unroll
   for (int m = 0; m < N / 2; ++m) {
     const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[m]), __float_as_uint(a[m + N / 2]), false, false);
     a[m] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
   }
-  if constexpr (TS_LB > 4) return;
-  // bit 4: the same with v_permlane16_swap between even and odd 16-lane rows
 #pragma unroll
   for (int m = 0; m < N / 4; ++m) {
     const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[m]), __float_as_uint(a[m + N / 4]), false, false);
     a[m] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
   }
-  if constexpr (TS_LB > 3) return;
-  // bit 3: row_ror:8 pairs lanes p and p ^ 8 of a 16-lane row
-  const int b3 = (l >> 3) & 1;
+}
+
+// Row sums of RL values at once (left in every lane of the row): a DPP step may read its source only two instructions
+// after it was written, so each of the four steps is followed by a quarter of the RL * N independent instructions that
+// `fill` issues (fill(j), j < N: at least two per step) instead of idling; the scheduling barriers keep them there.
+template <int RL, int N, typename F>
+__device__ __forceinline__ void ts_row_sums(float (&d)[RL], F&& fill) {
+  ts_for<4>([&](auto S) {
+    constexpr int s = decltype(S)::value, CTRL = s == 0 ? 0xb1 : s == 1 ? 0x4e : s == 2 ? 0x141 : 0x140;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int m = 0; m < N / 8; ++m) {
-    const float keep = b3 ? a[m + N / 8] : a[m], send = b3 ? a[m] : a[m + N / 8];
-    a[m] = keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), 0x128, 0xf, 0xf, true));
+    for (int i = 0; i < RL; ++i) d[i] = dpp_sum_step<CTRL>(d[i]);
+#pragma unroll
+    for (int j = s * N / 4; j < (s + 1) * N / 4; ++j) fill(j);
+  });
+  __builtin_amdgcn_sched_barrier(0);
+}
+// One round of a reduce-scatter over a row's lanes: a[0 .. 2N) -> a[0 .. N); the lane whose bit is clear keeps a[k] and
+// sends a[k + N] to its partner under CTRL, which has the bit set and does the reverse.
+template <int N, int CTRL>
+__device__ __forceinline__ void ts_lane_rs(float* a, bool hi) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const float keep = hi ? a[k + N] : a[k], send = hi ? a[k] : a[k + N];
+    a[k] = keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), CTRL, 0xf, 0xf, true));
   }
 }
 
-// A token's k, u, q in LDS: per vector eight blocks of K / 8 floats, each padded by 4 so that the eight lanes of a
-// row (one per block) read different banks with 16-byte reads.  Piece p < 3 K / 4 of a token (or one of the K / 4
-// pieces of u alone) is one float4, loaded into a register well ahead of its token and stored here before it.
+// sum of a lane's products, in four chains
+template <int N>
+__device__ __forceinline__ float ts_dot(const float (&a)[N], const float (&b)[N]) {
+  float d[4] = {a[0] * b[0], a[1] * b[1], a[2] * b[2], a[3] * b[3]};
+#pragma unroll
+  for (int j = 4; j < N; ++j) d[j & 3] = fmaf(a[j], b[j], d[j & 3]);
+  return (d[0] + d[1]) + (d[2] + d[3]);
+}
+
+// A token's k, u, q in LDS: per vector sixteen parts of K / 16 floats, padded so that the lanes of a row (one per part)
+// read different banks with 16-byte reads (K = 64: one piece each, contiguous).  Piece p < 3 K / 4 of a token is one
+// float4, loaded into a register well ahead of its token and stored here before it.
 template <int K>
 struct TokStage {
-  static constexpr int KQ = K / TS_LPR, K4 = K / 4, LD = KQ + 4, VEC = TS_LPR * LD, SIZE = 3 * VEC;
-  static __device__ __forceinline__ void load(const float* kp, const float* up, const float* qp, int64_t t, int tid,
-                                              bool kq, f32x4& x) {  // tid: the piece
-    const int vec = tid / K4, e4 = tid - vec * K4;
-    if (kq ? tid < 3 * K4 : vec == 1) {
-      const float* src = vec == 0 ? kp : vec == 1 ? up : qp;
-      x = *reinterpret_cast<const f32x4*>(src + t * K + 4 * e4);
-    }
+  static constexpr int KQ = K / TS_LPR, K4 = K / 4, LD = KQ == 4 ? 4 : KQ + 4, VEC = TS_LPR * LD, SIZE = 3 * VEC;
+  static constexpr int PER = 3 * K4;  // pieces per token
+  static_assert(KQ % 4 == 0, "a lane's part of a vector is read in 16-byte pieces");
+  static __device__ __forceinline__ f32x4 load(const float* kp, const float* up, const float* qp, int64_t t, int piece) {
+    const int vec = piece / K4, e4 = piece - vec * K4;
+    const float* src = vec == 0 ? kp : vec == 1 ? up : qp;
+    return *reinterpret_cast<const f32x4*>(src + t * K + 4 * e4);
   }
-  static __device__ __forceinline__ void stage(float* sv, int tid, bool kq, const f32x4& x) {
-    const int vec = tid / K4, c = 4 * (tid - vec * K4), qd = c / KQ;
-    if (kq ? tid < 3 * K4 : vec == 1) *reinterpret_cast<f32x4*>(sv + vec * VEC + qd * LD + c - qd * KQ) = x;
+  static __device__ __forceinline__ void stage(float* sv, int piece, const f32x4& x) {
+    const int vec = piece / K4, c = 4 * (piece - vec * K4), qd = c / KQ;
+    *reinterpret_cast<f32x4*>(sv + vec * VEC + qd * LD + c - qd * KQ) = x;
+  }
+  // this lane's part of staged vector vec
+  static __device__ __forceinline__ void read(const float* sv, int vec, int part, float (&o)[KQ]) {
+    const f32x4* p = reinterpret_cast<const f32x4*>(sv + vec * VEC + part * LD);
+#pragma unroll
+    for (int m = 0; m < KQ / 4; ++m) {
+      const f32x4 t = p[m];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[4 * m + e] = t[e];
+    }
   }
 };
 
-// this lane's quarter of a staged vector, as KQ floats through 16-byte LDS reads
-template <int KQ>
-__device__ __forceinline__ void ts_read(const float* p, float (&o)[KQ]) {
-#pragma unroll
-  for (int m = 0; m < KQ / 4; ++m) {
-    const f32x4 t = reinterpret_cast<const f32x4*>(p)[m];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[4 * m + e] = t[e];
-  }
-}
-
-// Tokens per block of the forward: a block's k, u, q are staged through LDS together (loaded a block ahead), so the
-// workgroup meets at one barrier per block and its waves run through the block's tokens unsynchronised.
-constexpr int TS_TB = 8;
-static_assert(TS_CT % TS_TB == 0, "checkpoints fall on block starts");
-
-// grid B * H * NB (NB = ceil(V / 64)) workgroups of TS_THREADS (512) threads: workgroup x -> (b h, row block vb)
-template <int K>
-__global__ __launch_bounds__(TS_THREADS) void token_scan_fwd_kernel(
+// grid B * H * NB (NB = ceil(V / ROWS)) workgroups: workgroup x -> (b h, row block vb).  Tokens past the end of the
+// sequence in the last block are identity tokens (zero vectors, v = 0, la = 0), which leave S as it is; nothing is
+// stored for them.
+template <int K, typename SH>
+__global__ __launch_bounds__(SH::THREADS) void token_scan_fwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ u, const float* __restrict__ v,
     const float* __restrict__ la, const float* __restrict__ h0, float* __restrict__ y, float* __restrict__ r,
     float* __restrict__ st, float* __restrict__ hT, int T_, int H, int V, int NCH, int NB) {
   using TS = TokStage<K>;
-  constexpr int KQ = TS::KQ, PER = 3 * TS::K4, NL = (TS_TB * PER + TS_THREADS - 1) / TS_THREADS;
+  constexpr int KQ = TS::KQ, RL = SH::RL, NL = (TS_TB * TS::PER + SH::THREADS - 1) / SH::THREADS;
   __shared__ __attribute__((aligned(16))) float sv[2][TS_TB][TS::SIZE];
-  const int tid = threadIdx.x, l = lane_id(), qd = l & (TS_LPR - 1);
+  const int tid = threadIdx.x, l = lane_id(), p = l & 15;
   const int pid = blockIdx.x, bh = pid / NB, vb = pid - bh * NB;
   const int b = bh / H, h = bh - b * H;
-  const int vi = vb * TS_ROWS + (tid >> TS_LB);
-  const bool on = vi < V;
-  const int vc = on ? vi : V - 1;  // rows past V compute on row V-1 and store nothing
-  // states [B, H, K, V] (fla's layout): entry (row vi, column qd KQ + j) at cb + j V
-  const int64_t cb = (int64_t)bh * K * V + (int64_t)qd * KQ * V + vi;
-  float S[KQ];
+  const int v0 = vb * SH::ROWS + wave_id() * SH::WROWS + (l >> 4) * RL;  // this lane's rows v0 .. v0 + RL - 1
+  // states [B, H, K, V] (fla's layout): entry (row v0 + i, column p KQ + j) at cb + j V + i
+  const int64_t cb = (int64_t)bh * K * V + (int64_t)p * KQ * V + v0;
+  float S[RL][KQ];
 #pragma unroll
-  for (int j = 0; j < KQ; ++j) S[j] = h0 && on ? h0[cb + (int64_t)j * V] : 0.f;
-  float* stb = st + (int64_t)bh * NCH * K * V + (int64_t)qd * KQ * V + vi;
+  for (int i = 0; i < RL; ++i)
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) S[i][j] = h0 && v0 + i < V ? h0[cb + (int64_t)j * V + i] : 0.f;
+  float* stb = st + (int64_t)bh * NCH * K * V;  // uniform; this lane's entries at st_off + j V + i of a checkpoint
+  const int64_t st_off = (int64_t)p * KQ * V + v0;
   const int64_t tok_first = (int64_t)b * T_ * H + h;
-  // block t0's vectors: thread piece e < TS_TB * PER is float4 e % PER (k, u, q in order) of token t0 + e / PER
+  // block t0's row scalars: this lane loads v of token p >> 1 for its row (RL = 2: row p & 1), and la of that token; the
+  // block's vectors: piece e < TB * PER is float4 e % PER of token t0 + e / PER
+  const int ti = p >> 1, vs = v0 + (RL == 2 ? p & 1 : 0);
   f32x4 xr[NL];
-  float vn[TS_TB], ln[TS_TB];  // the next block's v (this row) and la, loaded a block ahead
-  const int zv = ts_vector_zero();
+  float vn = 0.f, ln = 0.f;
   auto load_block = [&](int t0) {
 #pragma unroll
     for (int m = 0; m < NL; ++m) {
-      const int e = tid + m * TS_THREADS, i = e / PER, rem = e - i * PER;
-      if (e < TS_TB * PER && t0 + i < T_) TS::load(k, u, q, tok_first + (int64_t)(t0 + i) * H, rem, true, xr[m]);
+      const int e = tid + m * SH::THREADS, i = e / TS::PER;
+      xr[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (e < TS_TB * TS::PER && t0 + i < T_)
+        xr[m] = TS::load(k, u, q, tok_first + (int64_t)(t0 + i) * H, e - i * TS::PER);
     }
-#pragma unroll
-    for (int i = 0; i < TS_TB; ++i) {
-      const int64_t tk = tok_first + (int64_t)min(t0 + i, T_ - 1) * H;
-      vn[i] = v[tk * V + vc];
-      ln[i] = la[tk + zv];
-    }
+    const bool in = t0 + ti < T_;
+    const int64_t tk = tok_first + (int64_t)(t0 + ti) * H;
+    vn = in && vs < V ? v[tk * V + vs] : 0.f;
+    ln = in ? la[tk] : 0.f;
   };
   auto stage_block = [&](float (*dst)[TS::SIZE]) {
 #pragma unroll
     for (int m = 0; m < NL; ++m) {
-      const int e = tid + m * TS_THREADS, i = e / PER, rem = e - i * PER;
-      if (e < TS_TB * PER) TS::stage(dst[i], rem, true, xr[m]);
+      const int e = tid + m * SH::THREADS, i = e / TS::PER;
+      if (e < TS_TB * TS::PER) TS::stage(dst[i], e - i * TS::PER, xr[m]);
     }
   };
-  float vcur[TS_TB], lcur[TS_TB];
   load_block(0);  // T_ >= 1 here (the host returns before launching an empty scan)
   stage_block(sv[0]);
-#pragma unroll
-  for (int i = 0; i < TS_TB; ++i) vcur[i] = vn[i], lcur[i] = ln[i];
+  float vc = vn, ac = expf(ln);
   if (TS_TB < T_) load_block(TS_TB);
   ts_barrier();
   for (int t0 = 0, blk = 0; t0 < T_; t0 += TS_TB, ++blk) {
-    if (t0 % TS_CT == 0 && on) {
+    if (t0 % TS_CT == 0) {
       const int64_t c = t0 / TS_CT;
 #pragma unroll
-      for (int j = 0; j < KQ; ++j) stb[(c * K + j) * V] = S[j];
+      for (int i = 0; i < RL; ++i)
+        if (v0 + i < V) {
+#pragma unroll
+          for (int j = 0; j < KQ; ++j) stb[c * K * V + (int64_t)j * V + (st_off + i)] = S[i][j];
+        }
     }
+    const float(*sb)[TS::SIZE] = sv[blk & 1];
+    float rout[RL] = {}, ypart[RL][TS_TB];  // lane 2 i + 1: r of token i; this lane's part of each token's y
+    // the next token's vectors are read from LDS before this token's arithmetic, so their latency is off the chain
+    float vec[2][3][KQ];
+    auto read3 = [&](int i, float (&d)[3][KQ]) {
+      TS::read(sb[i], 0, p, d[0]);
+      TS::read(sb[i], 1, p, d[1]);
+      TS::read(sb[i], 2, p, d[2]);
+    };
+    read3(0, vec[0]);
+    ts_for<TS_TB>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i + 1 < TS_TB) read3(i + 1, vec[(i + 1) & 1]);
+      const auto& kk = vec[i & 1][0];
+      const auto& uu = vec[i & 1][1];
+      const auto& qq = vec[i & 1][2];
+      const float a = ts_lane<2 * i>(ac);
+      float d[RL], vr[RL];
+      ts_for<RL>([&](auto RI) {
+        constexpr int rr = decltype(RI)::value;
+        d[rr] = ts_dot(S[rr], kk);
+        vr[rr] = ts_row_bcast<2 * i + (RL == 2 ? rr : 0)>(vc);
+      });
+      // r = v - a (S k), with the decay of S in the gaps of the row sum
+      ts_row_sums<RL, KQ>(d, [&](int j) {
 #pragma unroll
-    for (int i = 0; i < TS_TB; ++i) {
-      if (t0 + i >= T_) break;
-      const int64_t tok = tok_first + (int64_t)(t0 + i) * H;
-      const float a = expf(lcur[i]);
-      const float* sk = sv[blk & 1][i] + qd * TS::LD;
-      float kk[KQ];
-      ts_read<KQ>(sk, kk);
-      float d[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int rr = 0; rr < RL; ++rr) S[rr][j] *= a;
+      });
 #pragma unroll
-      for (int j = 0; j < KQ; ++j) {
-        S[j] *= a;
-        d[j & 3] = fmaf(S[j], kk[j], d[j & 3]);
+      for (int rr = 0; rr < RL; ++rr) {
+        const float res = fmaf(-a, d[rr], vr[rr]);
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) S[rr][j] = fmaf(res, uu[j], S[rr][j]);
+        rout[rr] = p == 2 * i + 1 ? res : rout[rr];
+        ypart[rr][i] = ts_dot(S[rr], qq);
       }
-      const float rr = vcur[i] - ts_row_sum((d[0] + d[1]) + (d[2] + d[3]));
-      float uu[KQ], qq[KQ];
-      ts_read<KQ>(sk + TS::VEC, uu);
-      ts_read<KQ>(sk + 2 * TS::VEC, qq);
-      float e[4] = {0.f, 0.f, 0.f, 0.f};
+    });
+    // y: the block's eight partials reduce-scattered over the row's lanes (bits 3, 2, 1 of p select the token, bit 0 is
+    // summed), so lane p ends with token p >> 1's
+    static_assert(TS_TB == 8, "three rounds scatter the block's tokens");
+    float out[RL];
 #pragma unroll
-      for (int j = 0; j < KQ; ++j) {
-        S[j] = fmaf(rr, uu[j], S[j]);
-        e[j & 3] = fmaf(S[j], qq[j], e[j & 3]);
-      }
-      const float yy = ts_row_sum((e[0] + e[1]) + (e[2] + e[3]));
-      if (on && qd == 0) r[tok * V + vi] = rr;
-      if (on && qd == 1) y[tok * V + vi] = yy;
+    for (int i = 0; i < RL; ++i) {
+      float* a = ypart[i];
+      ts_lane_rs<4, 0x140>(a, p & 8);
+      ts_lane_rs<2, 0x141>(a, p & 4);
+      ts_lane_rs<1, 0x4e>(a, p & 2);
+      const float yy = ts_pin(dpp_sum_step<0xb1>(a[0]));
+      out[i] = p & 1 ? rout[i] : yy;
     }
-    if (t0 + TS_TB < T_) {  // stage the next block (loaded a block ago), load the one after it
-      stage_block(sv[(blk + 1) & 1]);
+    if (t0 + TS_TB < T_) {  // stage the next block (loaded a block ago); before the stores below, whose way to memory
+      stage_block(sv[(blk + 1) & 1]);  // the wait for these loads would otherwise include
+      vc = vn;
+      ac = expf(ln);
+    }
+    if (t0 + ti < T_) {
+      const int64_t tok = tok_first + (int64_t)(t0 + ti) * H;
+      float* dst = (p & 1 ? r : y) + tok * V + v0;
 #pragma unroll
-      for (int i = 0; i < TS_TB; ++i) vcur[i] = vn[i], lcur[i] = ln[i];
-      if (t0 + 2 * TS_TB < T_) load_block(t0 + 2 * TS_TB);
+      for (int i = 0; i < RL; ++i)
+        if (v0 + i < V) dst[i] = out[i];
     }
+    if (t0 + 2 * TS_TB < T_) load_block(t0 + 2 * TS_TB);
     ts_barrier();  // the block's vectors read by every lane; the next block's staged
   }
-  if (hT && on) {
+  if (hT) {
 #pragma unroll
-    for (int j = 0; j < KQ; ++j) hT[cb + (int64_t)j * V] = S[j];
+    for (int i = 0; i < RL; ++i)
+      if (v0 + i < V) {
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) hT[cb + (int64_t)j * V + i] = S[i][j];
+      }
   }
 }
 
 // The row sums of a group's steps: each wave's column sums (after ts_rows_rs) and its dla go to LDS slots of their
-// own (vector, token), and after the group's barrier the eight waves are added in a fixed order and stored as the
+// own (vector, token), and after the group's barrier the waves are added in a fixed order and stored as the
 // workgroup's partial rows (double-buffered by group parity).
-template <int K>
+template <int K, typename SH>
 struct TokSums {
-  float col[2][3][TS_GS][TS_WAVES][K];  // [parity][dq, du, dk][token][wave][column]
-  float sca[2][TS_GS][TS_WAVES];        // [parity][token][wave]: dla
-  // this wave's reduce-scattered sums of local columns (part l & (TS_LPR - 1)) into slot (vec, i)
-  template <int KQ>
+  static constexpr int KQ = K / TS_LPR, R = KQ / 4;
+  float col[2][3][TS_GS][SH::WAVES][K];  // [parity][dq, du, dk][token][wave][column]
+  float sca[2][SH::WAVES][TS_GS];        // [parity][wave][token]: dla
+  // this wave's reduce-scattered sums into slot (vec, i)
   __device__ __forceinline__ void put(int par, int vec, int i, const float (&a)[KQ], int l) {
-    constexpr int R = KQ * TS_LPR / 64;
-    const int w = wave_id(), c0 = (l & (TS_LPR - 1)) * KQ + R * (l >> TS_LB);
+    float* d = &col[par][vec][i][wave_id()][(l & 15) * KQ + R * (l >> 4)];
 #pragma unroll
-    for (int m = 0; m < R; ++m) col[par][vec][i][w][c0 + m] = a[m];
+    for (int m = 0; m < R; ++m) d[m] = a[m];
   }
   // the waves' values added as a pairwise tree (a fixed order)
-  template <typename F>
-  static __device__ __forceinline__ float tree(F&& x) {
-    float a[TS_WAVES];
+  template <typename X, typename F>
+  static __device__ __forceinline__ X tree(F&& x) {
+    X a[SH::WAVES];
 #pragma unroll
-    for (int w = 0; w < TS_WAVES; ++w) a[w] = x(w);
+    for (int w = 0; w < SH::WAVES; ++w) a[w] = x(w);
 #pragma unroll
-    for (int h = TS_WAVES / 2; h >= 1; h /= 2) {
+    for (int h = SH::WAVES / 2; h >= 1; h /= 2) {
 #pragma unroll
       for (int w = 0; w < h; ++w) a[w] = a[2 * w] + a[2 * w + 1];
     }
     return a[0];
   }
-  __device__ __forceinline__ float col_sum(int par, int vec, int i, int c) const {
-    return tree([&](int w) { return col[par][vec][i][w][c]; });
+  __device__ __forceinline__ f32x4 col_sum4(int par, int vec, int i, int c) const {
+    return tree<f32x4>([&](int w) { return *reinterpret_cast<const f32x4*>(&col[par][vec][i][w][c]); });
   }
   __device__ __forceinline__ float sca_sum(int par, int i) const {
-    return tree([&](int w) { return sca[par][i][w]; });
+    return tree<float>([&](int w) { return sca[par][w][i]; });
   }
 };
-static_assert(TS_LB >= 3 && TS_LB <= 4, "row sums and reduce-scatter rounds cover 8 or 16 lanes per row");
 
-// Partials: gqp, gup, gkp [NB][B*T*H][K], glap [NB][B*T*H]; sc [B*H*NB][TS_CT / TS_GS][K / TS_LPR][TS_THREADS] scratch of
+// Partials: gqp, gup, gkp [NB][B*T*H][K], glap [NB][B*T*H]; sc [B*H*NB][TS_CT / TS_GS][THREADS][RL K / 16] scratch of
 // the chunk's group-start states.
 // Per chunk (last first), in groups of TS_GS tokens: a forward pass from the checkpoint stores the state entering each
 // group but the first and last (the last stays in registers); then, group by group from the last, the group's tokens
 // are recomputed forward from its start state with each decayed state e^{la} S_{t-1} kept in registers (and dq
 // accumulated), and walked backward.  A short last group is padded with identity tokens (la = 0, zero vectors and
-// row values), which change neither S nor G, and whose sums are not stored.  Both passes stage a group's vectors
-// through LDS (and load its row values) a group ahead: one barrier per group.
-template <int K>
-__global__ __launch_bounds__(TS_THREADS) void token_scan_bwd_kernel(
+// row values), which change neither S nor G, and whose sums are not stored.  The forward pass has the chunk's u in LDS
+// at once; the groups' vectors are staged (and their row values loaded) a group ahead: one barrier per group.
+template <int K, typename SH>
+__global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void token_scan_bwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ u, const float* __restrict__ la,
     const float* __restrict__ r, const float* __restrict__ st, const float* __restrict__ gy,
     const float* __restrict__ dhT, float* __restrict__ gv, float* __restrict__ gqp, float* __restrict__ gup,
     float* __restrict__ gkp, float* __restrict__ glap, float* __restrict__ dh0, float* __restrict__ sc, int T_, int H,
     int V, int NCH, int NB, int64_t ntok) {
   using TS = TokStage<K>;
-  constexpr int KQ = TS::KQ, NGS = TS_CT / TS_GS, PER = 3 * TS::K4;
-  static_assert(TS_GS * PER <= TS_THREADS, "one piece of a group's vectors per thread");
+  constexpr int KQ = TS::KQ, RL = SH::RL, THREADS = SH::THREADS, NGS = TS_CT / TS_GS;
+  constexpr int NL = (TS_GS * TS::PER + THREADS - 1) / THREADS;
   __shared__ __attribute__((aligned(16))) float sv[2][TS_GS][TS::SIZE];
-  __shared__ TokSums<K> sums;
-  const int tid = threadIdx.x, l = lane_id(), qd = l & (TS_LPR - 1);
+  __shared__ __attribute__((aligned(16))) TokSums<K, SH> sums;
+  const int tid = threadIdx.x, l = lane_id(), p = l & 15;
   const int pid = blockIdx.x, bh = pid / NB, vb = pid - bh * NB;
   const int b = bh / H, h = bh - b * H;
-  const int vi = vb * TS_ROWS + (tid >> TS_LB);
-  const bool on = vi < V;
-  const float* stb = st + (int64_t)bh * NCH * K * V + (int64_t)qd * KQ * V + vi;
-  float* scw = sc + (int64_t)pid * NGS * KQ * TS_THREADS + tid;
+  const int v0 = vb * SH::ROWS + wave_id() * SH::WROWS + (l >> 4) * RL;  // this lane's rows, as in the forward
+  // uniform bases and 32-bit lane offsets: per-lane 64-bit addresses of the unrolled accesses would fill the registers
+  const float* stb = st + (int64_t)bh * NCH * K * V;
+  const int64_t st_off = (int64_t)p * KQ * V + v0;
+  constexpr int SV = RL * KQ / 4;  // 16-byte pieces of this lane's state
+  f32x4* scw = reinterpret_cast<f32x4*>(sc + (int64_t)pid * NGS * RL * KQ * THREADS);
+  const unsigned sc_off = (unsigned)tid * SV;
+  auto put_state = [&](int g, const float (&X)[RL][KQ]) {
+#pragma unroll
+    for (int m = 0; m < SV; ++m) {
+      const int i = 4 * m / KQ, j = 4 * m % KQ;
+      scw[(unsigned)(g * THREADS * SV) + (sc_off + m)] = f32x4{X[i][j], X[i][j + 1], X[i][j + 2], X[i][j + 3]};
+    }
+  };
+  auto get_state = [&](int g, float (&X)[RL][KQ]) {
+#pragma unroll
+    for (int m = 0; m < SV; ++m) {
+      const int i = 4 * m / KQ, j = 4 * m % KQ;
+      const f32x4 t = scw[(unsigned)(g * THREADS * SV) + (sc_off + m)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) X[i][j + e] = t[e];
+    }
+  };
   float* const gout[3] = {gqp + (int64_t)vb * ntok * K, gup + (int64_t)vb * ntok * K, gkp + (int64_t)vb * ntok * K};
   float* gl_b = glap + (int64_t)vb * ntok;
-  const int zv = ts_vector_zero();
-  const int pi = tid / PER, prem = tid - pi * PER;  // this thread's piece of a group's vectors: token pi, piece prem
-  f32x4 xr;                                         // ... of the next group, loaded a group ahead
-  float nla[TS_GS], nr[TS_GS], ngy[TS_GS];          // the next group's row values
-  float cla[TS_GS], cr[TS_GS], cgy[TS_GS];          // the current group's
-  // a group's tokens tok_at(i), i < TS_GS (tok < 0: an identity token); kq: k, q and dy too (else u and r alone)
-  auto load_grp = [&](auto&& tok_at, bool kq) {
-    if (pi < TS_GS) {
-      const int64_t tk = tok_at(pi);
-      if (tk >= 0) TS::load(k, u, q, tk, prem, kq, xr);
-      else xr = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+  f32x4 xr[NL];  // this thread's pieces of the next group's vectors (piece e: token e / PER), loaded a group ahead
+  // The group's row scalars, one token per lane: lane p holds r of token p & 3 and row p >> 2 for p < 4 RL, dy likewise
+  // for the next 4 RL lanes; and la of token l & 3
+  const int ti = p & 3, si = p >> 2, srow = v0 + (RL == 2 ? si & 1 : 0);
+  const float* sp = (RL == 2 ? si >= 2 : (si & 1)) ? gy : r;
+  float xn, ln, xc, ac;
+  auto load_grp = [&](auto&& tok_at) {  // tok_at(i): token i of the group (< 0: an identity token)
 #pragma unroll
-    for (int i = 0; i < TS_GS; ++i) {
-      const int64_t tk = tok_at(i);
-      nla[i] = tk >= 0 ? la[tk + zv] : 0.f;
-      nr[i] = tk >= 0 && on ? r[tk * V + vi] : 0.f;
-      ngy[i] = tk >= 0 && on && kq ? gy[tk * V + vi] : 0.f;
+    for (int m = 0; m < NL; ++m) {
+      const int e = tid + m * THREADS, pi = e / TS::PER;
+      xr[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (e < TS_GS * TS::PER) {
+        const int64_t tk = tok_at(pi);
+        if (tk >= 0) xr[m] = TS::load(k, u, q, tk, e - pi * TS::PER);
+      }
     }
+    const int64_t tk = tok_at(ti);
+    xn = tk >= 0 && srow < V ? sp[tk * V + srow] : 0.f;
+    ln = tk >= 0 ? la[tk] : 0.f;
   };
-  auto stage_grp = [&](int buf, bool kq) {
-    if (pi < TS_GS) TS::stage(sv[buf][pi], prem, kq, xr);
+  auto stage_grp = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < TS_GS; ++i) cla[i] = nla[i], cr[i] = nr[i], cgy[i] = ngy[i];
+    for (int m = 0; m < NL; ++m) {
+      const int e = tid + m * THREADS, pi = e / TS::PER;
+      if (e < TS_GS * TS::PER) TS::stage(sv[buf][pi], e - pi * TS::PER, xr[m]);
+    }
+    xc = xn;
+    ac = expf(ln);
   };
   int par = 0;  // parity of the group: sv[par & 1] holds its vectors, sums[par & 1] takes its row sums
-  const int64_t cb = (int64_t)bh * K * V + (int64_t)qd * KQ * V + vi;  // [B, H, K, V] states, as in the forward
-  float G[KQ], S[KQ];
+  const int64_t cb = (int64_t)bh * K * V + (int64_t)p * KQ * V + v0;  // [B, H, K, V] states, as in the forward
+  float G[RL][KQ], S[RL][KQ];
 #pragma unroll
-  for (int j = 0; j < KQ; ++j) G[j] = dhT && on ? dhT[cb + (int64_t)j * V] : 0.f;
+  for (int i = 0; i < RL; ++i)
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) G[i][j] = dhT && v0 + i < V ? dhT[cb + (int64_t)j * V + i] : 0.f;
   for (int c = NCH - 1; c >= 0; --c) {
     const int n = min(TS_CT, T_ - c * TS_CT), ng = (n + TS_GS - 1) / TS_GS;
     const int64_t tok0 = ((int64_t)b * T_ + (int64_t)c * TS_CT) * H + h;
@@ -326,44 +433,75 @@ __global__ __launch_bounds__(TS_THREADS) void token_scan_bwd_kernel(
       const int t = g * TS_GS + i;
       return t < n ? tok0 + (int64_t)t * H : -1;
     };
+    auto load_state = [&](float (&X)[RL][KQ]) {  // the chunk's checkpoint
 #pragma unroll
-    for (int j = 0; j < KQ; ++j) S[j] = on ? stb[((int64_t)c * K + j) * V] : 0.f;
-    // forward from the checkpoint to the last group's start, storing the start states of groups 1 .. ng - 2
+      for (int i = 0; i < RL; ++i)
+#pragma unroll
+        for (int j = 0; j < KQ; ++j)
+          X[i][j] = v0 + i < V ? stb[(int64_t)c * K * V + (int64_t)j * V + (st_off + i)] : 0.f;
+    };
+    load_state(S);
+    // forward from the checkpoint to the last group's start, storing the start states of groups 1 .. ng - 2: the chunk's
+    // u staged whole (over the row sums, which are free between chunks), so no barrier stands between its groups
     if (ng > 1) {
-      load_grp([&](int i) { return tok_in(0, i); }, false);
-      stage_grp(par & 1, false);
-      if (ng > 2) load_grp([&](int i) { return tok_in(1, i); }, false);
-      ts_barrier();
-      for (int g = 0; g < ng - 1; ++g, ++par) {
-        const int p = par & 1;
-        if (g > 0) {
+      constexpr int NU = (TS_CT * TS::K4 + THREADS - 1) / THREADS;
+      f32x4 xu[NU];
+      float rc[RL][2], a32;
 #pragma unroll
-          for (int j = 0; j < KQ; ++j) scw[((int64_t)g * KQ + j) * TS_THREADS] = S[j];
-        }
-#pragma unroll
-        for (int i = 0; i < TS_GS; ++i) {
-          float uu[KQ];
-          ts_read<KQ>(sv[p][i] + TS::VEC + qd * TS::LD, uu);
-          const float a = expf(cla[i]);
-#pragma unroll
-          for (int j = 0; j < KQ; ++j) S[j] = fmaf(cr[i], uu[j], S[j] * a);
-        }
-        if (g + 1 < ng - 1) {
-          stage_grp((par + 1) & 1, false);
-          if (g + 2 < ng - 1) load_grp([&](int i) { return tok_in(g + 2, i); }, false);
-        }
-        ts_barrier();
+      for (int m = 0; m < NU; ++m) {
+        const int e = tid + m * THREADS, t = e / TS::K4;
+        xu[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (t < n) xu[m] = *reinterpret_cast<const f32x4*>(u + (tok0 + (int64_t)t * H) * K + 4 * (e - t * TS::K4));
       }
-    }
-    // groups last to first: TS_GS forward steps (tokens 0 .. TS_GS - 1 of the group), then TS_GS backward steps
-    auto flush = [&](int g, int pb) {  // the group's row sums, from LDS slots of parity pb
 #pragma unroll
-      for (int m = 0; m < (3 * TS_GS * K + TS_THREADS - 1) / TS_THREADS; ++m) {
-        const int o = tid + m * TS_THREADS;
-        if (o < 3 * TS_GS * K) {
-          const int vec = o / (TS_GS * K), rem = o - vec * TS_GS * K, i = rem / K, cc = rem - i * K;
+      for (int i = 0; i < RL; ++i)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          rc[i][m] = p + 16 * m < n && v0 + i < V ? r[(tok0 + (int64_t)(p + 16 * m) * H) * V + v0 + i] : 0.f;
+      a32 = (l & 31) < n ? la[tok0 + (int64_t)(l & 31) * H] : 0.f;
+      ts_barrier();  // the previous chunk's last row sums read
+      float* su = &sums.col[0][0][0][0][0];
+      static_assert(sizeof(sums.col) >= TS_CT * TS::VEC * 4, "the chunk's u fits over the row sums");
+#pragma unroll
+      for (int m = 0; m < NU; ++m) {
+        const int e = tid + m * THREADS, t = e / TS::K4, cc = 4 * (e - t * TS::K4), qd = cc / KQ;
+        if (t < TS_CT) *reinterpret_cast<f32x4*>(su + t * TS::VEC + qd * TS::LD + cc - qd * KQ) = xu[m];
+      }
+      a32 = expf(a32);
+      ts_barrier();
+      ts_for<NGS - 1>([&](auto GI) {
+        constexpr int g = decltype(GI)::value;
+        __builtin_amdgcn_sched_barrier(0);  // one group's reads at a time (registers)
+        if (g < ng - 1) {
+          if (g > 0) put_state(g, S);
+          float uu[TS_GS][KQ];
+#pragma unroll
+          for (int i = 0; i < TS_GS; ++i) TS::read(su + (g * TS_GS + i) * TS::VEC, 0, p, uu[i]);
+          ts_for<TS_GS>([&](auto I) {
+            constexpr int i = decltype(I)::value, t = g * TS_GS + i;
+            const float a = ts_lane<t>(a32);
+            ts_for<RL>([&](auto RI) {
+              constexpr int rr = decltype(RI)::value;
+              const float rt = ts_row_bcast<(t & 15)>(rc[rr][t >> 4]);
+#pragma unroll
+              for (int j = 0; j < KQ; ++j) S[rr][j] = fmaf(rt, uu[i][j], S[rr][j] * a);
+            });
+          });
+        }
+      });
+    }
+    auto flush = [&](int g, int pb) {  // the group's row sums, from LDS slots of parity pb, four columns at a time
+      constexpr int KV = K / 4, NF = 3 * TS_GS * KV;
+#pragma unroll
+      for (int m = 0; m < (NF + THREADS - 1) / THREADS; ++m) {
+        const int o = tid + m * THREADS;
+        if (o < NF) {
+          const int vec = o / (TS_GS * KV), rem = o - vec * TS_GS * KV, i = rem / KV, cc = 4 * (rem - i * KV);
           const int64_t tk = tok_in(g, i);
-          if (tk >= 0) gout[vec][tk * K + cc] = sums.col_sum(pb, vec, i, cc);
+          if (tk >= 0) {
+            float* dst = vec == 0 ? gout[0] : vec == 1 ? gout[1] : gout[2];
+            *reinterpret_cast<f32x4*>(dst + tk * K + cc) = sums.col_sum4(pb, vec, i, cc);
+          }
         }
       }
       if (tid < TS_GS) {
@@ -371,106 +509,167 @@ __global__ __launch_bounds__(TS_THREADS) void token_scan_bwd_kernel(
         if (tk >= 0) gl_b[tk] = sums.sca_sum(pb, tid);
       }
     };
-    load_grp([&](int i) { return tok_in(ng - 1, i); }, true);
-    stage_grp(par & 1, true);
-    if (ng > 1) load_grp([&](int i) { return tok_in(ng - 2, i); }, true);
+    // groups last to first: TS_GS forward steps (tokens 0 .. TS_GS - 1 of the group), then TS_GS backward steps
+    load_grp([&](int i) { return tok_in(ng - 1, i); });
+    stage_grp(par & 1);
+    if (ng > 1) load_grp([&](int i) { return tok_in(ng - 2, i); });
     ts_barrier();
     for (int g = ng - 1; g >= 0; --g, ++par) {
-      const int p = par & 1;
-      if (g < ng - 1) {
-        flush(g + 1, p ^ 1);
-        if (g == 0) {
-#pragma unroll
-          for (int j = 0; j < KQ; ++j) S[j] = on ? stb[((int64_t)c * K + j) * V] : 0.f;
-        } else {
-#pragma unroll
-          for (int j = 0; j < KQ; ++j) S[j] = scw[((int64_t)g * KQ + j) * TS_THREADS];
-        }
-      }
-      float Sd[TS_GS][KQ];  // e^{la} S_{t-1} of the group's tokens
-#pragma unroll
-      for (int s = 0; s < 2 * TS_GS; ++s) {
-        const int i = s < TS_GS ? s : 2 * TS_GS - 1 - s;
-        const float a = expf(cla[i]), rc = cr[i], gyc = cgy[i];
-        const float* sb = sv[p][i] + qd * TS::LD;
+      const int pb = par & 1;
+      // the state entering the group before this one, loaded while this one computes
+      float Sn[RL][KQ];
+      if (g > 1) get_state(g - 1, Sn);
+      else load_state(Sn);  // the checkpoint (after the chunk's first group it is not used)
+      if (g < ng - 1) flush(g + 1, pb ^ 1);
+      float Sd[TS_GS][RL][KQ];  // e^{la} S_{t-1} of the group's tokens
+      ts_for<TS_GS>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        const float a = ts_lane<i>(ac);
         float uu[KQ], t[KQ];
-        ts_read<KQ>(sb + TS::VEC, uu);
-        if (s < TS_GS) {
+        TS::read(sv[pb][i], 1, p, uu);
+        ts_for<RL>([&](auto RI) {
+          constexpr int rr = decltype(RI)::value;
+          const float rc = ts_row_bcast<4 * rr + i>(xc), gyc = ts_row_bcast<4 * RL + 4 * rr + i>(xc);
 #pragma unroll
           for (int j = 0; j < KQ; ++j) {
-            S[j] *= a;
-            Sd[i][j] = S[j];
-            S[j] = fmaf(rc, uu[j], S[j]);
-            t[j] = S[j] * gyc;
+            Sd[i][rr][j] = S[rr][j] * a;
+            S[rr][j] = fmaf(rc, uu[j], Sd[i][rr][j]);
+            t[j] = rr == 0 ? S[rr][j] * gyc : fmaf(S[rr][j], gyc, t[j]);
           }
-          ts_rows_rs<KQ>(t, l);
-          sums.put(p, 0, i, t, l);
-        } else {
-          float qq[KQ], kk[KQ];
-          ts_read<KQ>(sb + 2 * TS::VEC, qq);
-          float d[4] = {0.f, 0.f, 0.f, 0.f};
+        });
+        ts_rows_rs(t);
+        sums.put(pb, 0, i, t, l);
+      });
+      float out = 0.f, e4[TS_GS];  // lane p < 4 RL: dv of token p & 3, row p >> 2; the tokens' dla partials
+      ts_for<TS_GS>([&](auto I) {
+        constexpr int i = TS_GS - 1 - decltype(I)::value;
+        const float a = ts_lane<i>(ac);
+        float uu[KQ], kk[KQ], qq[KQ], t[KQ], t2[KQ];
+        TS::read(sv[pb][i], 2, p, qq);
+        TS::read(sv[pb][i], 1, p, uu);
+        TS::read(sv[pb][i], 0, p, kk);
+        float d[RL], rc[RL];
+        ts_for<RL>([&](auto RI) {
+          constexpr int rr = decltype(RI)::value;
+          rc[rr] = ts_row_bcast<4 * rr + i>(xc);
+          const float gyc = ts_row_bcast<4 * RL + 4 * rr + i>(xc);
+#pragma unroll
+          for (int j = 0; j < KQ; ++j) G[rr][j] = fmaf(gyc, qq[j], G[rr][j]);
+          d[rr] = ts_dot(G[rr], uu);
+        });
+        ts_row_sums<RL, KQ>(d, [&](int j) {
+          t[j] = G[0][j] * rc[0];
+          if constexpr (RL == 2) t[j] = fmaf(G[RL - 1][j], rc[RL - 1], t[j]);
+        });
+        e4[i] = 0.f;
+#pragma unroll
+        for (int rr = 0; rr < RL; ++rr) {
+          const float gr = d[rr];
+          out = p == 4 * rr + i ? gr : out;
 #pragma unroll
           for (int j = 0; j < KQ; ++j) {
-            G[j] = fmaf(gyc, qq[j], G[j]);
-            d[j & 3] = fmaf(G[j], uu[j], d[j & 3]);
+            G[rr][j] = fmaf(-gr, kk[j], G[rr][j]);
+            t2[j] = rr == 0 ? -Sd[i][rr][j] * gr : fmaf(-Sd[i][rr][j], gr, t2[j]);
           }
-          const float gr = ts_row_sum((d[0] + d[1]) + (d[2] + d[3]));
-          const int64_t tok = tok_in(g, i);
-          if (on && qd == 0 && tok >= 0) gv[tok * V + vi] = gr;
+          e4[i] += ts_dot(G[rr], Sd[i][rr]);
 #pragma unroll
-          for (int j = 0; j < KQ; ++j) t[j] = G[j] * rc;
-          ts_rows_rs<KQ>(t, l);
-          sums.put(p, 1, i, t, l);
-          ts_read<KQ>(sb, kk);
-#pragma unroll
-          for (int j = 0; j < KQ; ++j) {
-            G[j] = fmaf(-gr, kk[j], G[j]);
-            t[j] = -Sd[i][j] * gr;
-          }
-          ts_rows_rs<KQ>(t, l);
-          sums.put(p, 2, i, t, l);
-          float e[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int j = 0; j < KQ; ++j) e[j & 3] = fmaf(G[j], Sd[i][j], e[j & 3]);
-          const float gl = wave_sum64((e[0] + e[1]) + (e[2] + e[3]));
-          if (l == 0) sums.sca[p][i][wave_id()] = gl;
-#pragma unroll
-          for (int j = 0; j < KQ; ++j) G[j] *= a;
+          for (int j = 0; j < KQ; ++j) G[rr][j] *= a;
         }
+        ts_rows_rs(t);
+        sums.put(pb, 1, i, t, l);
+        ts_rows_rs(t2);
+        sums.put(pb, 2, i, t2, l);
+      });
+      ts_rows_rs(e4);  // lane group l >> 4: token l >> 4's partials
+      e4[0] = sum16(e4[0]);
+      if (p == 0) sums.sca[pb][wave_id()][l >> 4] = e4[0];
+      if (g > 0) stage_grp((par + 1) & 1);  // the group before, loaded a group ago; ahead of the store, as in the forward
+      {
+        const int64_t tk = tok_in(g, ti);
+        if (p < 4 * RL && tk >= 0 && srow < V) gv[tk * V + srow] = out;
       }
-      if (g > 0) {  // stage the group before (loaded a group ago), load the one before it
-        stage_grp((par + 1) & 1, true);
-        if (g > 1) load_grp([&](int i) { return tok_in(g - 2, i); }, true);
-      }
+      if (g > 1) load_grp([&](int i) { return tok_in(g - 2, i); });
+#pragma unroll
+      for (int i = 0; i < RL; ++i)
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) S[i][j] = Sn[i][j];
       ts_barrier();  // the group's vectors read and sums written; the group before staged
     }
     flush(0, (par - 1) & 1);
   }
   // G is now the gradient of the state before the first token: the initial state's
-  if (dh0 && on) {
+  if (dh0) {
 #pragma unroll
-    for (int j = 0; j < KQ; ++j) dh0[cb + (int64_t)j * V] = G[j];
+    for (int i = 0; i < RL; ++i)
+      if (v0 + i < V) {
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) dh0[cb + (int64_t)j * V + i] = G[i][j];
+      }
   }
 }
 
 // ---------------------------------------------------------------------------------------------------------
 bool token_scan_supported(int K) { return K == 64 || K == 128; }
 int token_scan_ct() { return TS_CT; }
-size_t token_scan_scratch_floats(int K) { return (size_t)(TS_CT / TS_GS) * K * TS_ROWS; }
 
-template <int K>
-static hipError_t token_scan_k(const TokenScanArgs& a, bool backward) {
-  const int NB = (a.V + TS_ROWS - 1) / TS_ROWS, NCH = (a.T + TS_CT - 1) / TS_CT;
+// Rows per workgroup: 16 (one row per lane, four waves), 32 (eight waves) or, in the backward, 64 (two rows per lane).
+// A lone workgroup's pace is set by its chain from token to token: with at most one workgroup per CU 16 rows are the
+// fastest, and 32 cost less than two rounds of 16 (the token vectors staged once for twice the rows, half the
+// backward's partial rows); two rows per lane share the row sums' reduce-scatter, so once there is more than one round
+// of 32 the backward is bound by its arithmetic and 64 rows cost about three rounds of 16.  Hence the fewest rounds over
+// the CUs in these weights (16: 1, 32: 2, 64: 3, ties to the larger of 16 and 32 and the smaller of 32 and 64).
+// Measured, H4 K128 V256, forward + backward us at 16, 32 and 64 rows (forward: 32): T1024 B4 241 + 908, 311 + 1040,
+// 313 + 1591; T512 B8 166 + 600, 163 + 553, 167 + 829; T512 B12 211 + 1035, 242 + 1086, 240 + 879; T512 B16 259 + 1182,
+// 246 + 1116, 245 + 912; K64 V256 T256 B16 85 + 318, 83 + 333, 81 + 252; B36 T65 V96 42 + 147, 41 + 151, 40 + 234.
+// (Before, with eight lanes per row and 64 rows per workgroup throughout: B4 507 + 1916, B8 257 + 987, B16 266 + 1029.)
+// Fewer rows also mean more partial rows (12 bytes per row block, token and k): the blocks grow while those would take
+// more than TS_PART_BYTES, which 64-row blocks may exceed.
+constexpr int64_t TS_PART_BYTES = (int64_t)4 << 30;
+static int ts_rows(int B, int T, int H, int K, int V, bool backward) {
+  const int64_t cus = device_cu_count(), BH = (int64_t)B * H;
+  auto rounds = [&](int rows) { return (BH * ((V + rows - 1) / rows) + cus - 1) / cus; };
+  if (backward && 3 * rounds(64) < 2 * rounds(32)) return 64;
+  int rows = rounds(16) < 2 * rounds(32) ? 16 : 32;
+  if (backward)
+    while (rows < 64 && BH * T * K * ((V + rows - 1) / rows) * 12 > TS_PART_BYTES) rows *= 2;
+  return rows;
+}
+
+int token_scan_row_blocks(int B, int T, int H, int K, int V) {
+  const int rows = ts_rows(B, T, H, K, V, true);
+  return (V + rows - 1) / rows;
+}
+size_t token_scan_scratch_floats(int B, int T, int H, int K, int V) {
+  const int rows = ts_rows(B, T, H, K, V, true);
+  return (size_t)B * H * ((V + rows - 1) / rows) * (TS_CT / TS_GS) * K * rows;
+}
+
+template <int K, typename SH>
+static hipError_t token_scan_sh(const TokenScanArgs& a, bool backward) {
+  const int NB = (a.V + SH::ROWS - 1) / SH::ROWS, NCH = (a.T + TS_CT - 1) / TS_CT;
   const dim3 grid((unsigned)(a.B * a.H * NB));
   if (!backward) {
-    token_scan_fwd_kernel<K><<<grid, TS_THREADS, 0, a.stream>>>(a.q, a.k, a.u, a.v, a.la, a.h0, a.y, a.r, a.st,
-                                                                a.hT, a.T, a.H, a.V, NCH, NB);
+    if constexpr (SH::RL == 1)
+      token_scan_fwd_kernel<K, SH><<<grid, SH::THREADS, 0, a.stream>>>(a.q, a.k, a.u, a.v, a.la, a.h0, a.y, a.r, a.st,
+                                                                       a.hT, a.T, a.H, a.V, NCH, NB);
+    else
+      return hipErrorInvalidValue;  // ts_rows gives the forward 16 or 32 rows
   } else {
-    token_scan_bwd_kernel<K><<<grid, TS_THREADS, 0, a.stream>>>(
+    token_scan_bwd_kernel<K, SH><<<grid, SH::THREADS, 0, a.stream>>>(
         a.q, a.k, a.u, a.la, a.r, a.st, a.dy, a.dhT, a.dv, a.dq_part, a.du_part, a.dk_part, a.dla_part, a.dh0,
         a.scratch, a.T, a.H, a.V, NCH, NB, (int64_t)a.B * a.T * a.H);
   }
   return hipGetLastError();
+}
+
+template <int K>
+static hipError_t token_scan_k(const TokenScanArgs& a, bool backward) {
+  switch (ts_rows(a.B, a.T, a.H, K, a.V, backward)) {
+    case 16: return token_scan_sh<K, TsShape<1, 4>>(a, backward);
+    case 32: return token_scan_sh<K, TsShape<1, 8>>(a, backward);
+    default: return token_scan_sh<K, TsShape<2, 8>>(a, backward);
+  }
 }
 
 hipError_t launch_token_scan(const TokenScanArgs& a, bool backward) {

@@ -489,6 +489,19 @@ def _state_arg(t: Optional[Tensor], B: int, H: int, K: int, V: int, what: str) -
     return _arg(t, torch.float32)
 
 
+def _sum_rows(p: Tensor) -> Tensor:
+    """The sum of p's rows in order (the backward's partial rows)."""
+    nb, n = p.shape[0], p.shape[1:].numel()
+    if nb == 1:
+        return p[0]
+    if nb == 0 or n == 0 or n % 8:
+        return p.sum(0)
+    out = torch.empty_like(p[0])
+    _lib.check(_lib.load().gdn_sum_parts(_lib.ptr(p), p.shape[0], _lib.ptr(out), n, _lib.DTYPE_F32,
+                                         _lib.stream_ptr(p.device)), "gdn_sum_parts")
+    return out
+
+
 @torch.library.custom_op("archbench_amd::nsgdn_token_fwd", mutates_args=())
 def nsgdn_token_fwd(q: Tensor, k: Tensor, u: Tensor, v: Tensor, la: Tensor, h0: Optional[Tensor],
                     output_final_state: bool) -> tuple[Tensor, Tensor, Tensor, Tensor]:
@@ -555,8 +568,8 @@ def nsgdn_token_bwd(q: Tensor, k: Tensor, u: Tensor, la: Tensor, r: Tensor, st: 
                                 _lib.ptr(dh0) if need_dh0 else None, _lib.ptr(sc), sc.numel() * 4, B, T, H, K, V,
                                 _lib.stream_ptr(dev))
     _lib.check(rc, "gdn_token_scan_bwd")
-    dq, du, dk = (p[0] if nb == 1 else p.sum(0) for p in parts)
-    return dq, dk, du, dv, (dla_p[0] if nb == 1 else dla_p.sum(0)), dh0
+    dq, du, dk = (_sum_rows(p) for p in parts)
+    return dq, dk, du, dv, _sum_rows(dla_p), dh0
 
 
 @nsgdn_token_bwd.register_fake

@@ -118,3 +118,31 @@ def test_token_scan_is_deterministic():
     torch.cuda.synchronize()
     for a, b in zip(*runs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,T,H,V,rows", [(1, 3, 1, 1, 16), (2, 70, 3, 17, 16), (1, 36, 2, 49, 16), (64, 9, 2, 56, 32),
+                                          (85, 33, 1, 96, 32), (86, 33, 1, 96, 64), (128, 3, 2, 64, 64),
+                                          (64, 37, 1, 256, 64), (64, 8, 4, 124, 64)])
+@pytest.mark.parametrize("K", [64, 128])
+def test_token_scan_row_blocks(B, T, H, V, rows, K):
+    """16, 32 and 64 rows per workgroup (by the rounds over 256 CUs): full and partial row blocks, tokens
+    that end inside a group, a block and a checkpoint chunk, with initial and final states and their gradients.  The
+    bound is test_token_scan_matches_recurrence's, 1e-6: fp32 sums of at most 128 products of operands of order 1 (2^-24
+    per step, decayed over the tokens)."""
+    banner(f"token scan rows {rows}: B={B} T={T} H={H} K={K} V={V}")
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        nb = ops._token_sizes(ops._lib.load(), B, T, H, K, V)[2]
+        assert nb == -(-V // rows), nb
+    q, k, u, v, la, dy = _inputs(B, T, H, K, V, seed=B + T + K + V)
+    g = torch.Generator().manual_seed(7)
+    h0, dhT = (0.1 * torch.randn(B, H, K, V, generator=g) for _ in range(2))
+    d = [t.cuda() for t in (q, k, u, v, la, dy, h0, dhT)]
+    y, r, st, hT = ops.nsgdn_token_fwd(*d[:5], d[6], True)
+    dq, dk, du, dv, dla, dh0 = ops.nsgdn_token_bwd(d[0], d[1], d[2], d[4], r, st, d[5], d[7], True)
+    y_ref, hT_ref = NS.recurrent_fwd(q, k, u, v, la, h0=h0)
+    ref = NS.recurrent_bwd(q, k, u, v, la, dy, h0=h0, dhT=dhT)
+    errs = {n: rel_l2(a, b) for n, a, b in zip(("y", "hT", "dq", "dk", "du", "dv", "dla", "dh0"),
+                                               (y, hT, dq, dk, du, dv, dla, dh0), (y_ref, hT_ref) + tuple(ref))}
+    print("[rel-L2] " + ", ".join(f"{n} {e:.1e}" for n, e in errs.items()), flush=True)
+    for n, e in errs.items():
+        assert e <= 1e-6, (n, e)
