@@ -144,7 +144,10 @@ int device_cu_count() {
 }
 
 bool narrow_sweep_blocks(const ChunkArgs& a, int blocks_per_head) {
-  // only when the narrow workgroups all run at once, one per CU (two per CU were measured slower than one wide)
+  // only when the narrow workgroups all run at once, one per CU (two per CU were measured slower than one wide).  fp32's
+  // products fill a CU's matrix cores, so half the columns per CU is nearly half the time; separate write keys gain a
+  // bf16 sweep's part.  Forward + reverse sweep, wide and narrow, us: fp32 K64 V64 B2 T512 H4 55 + 60, 39 + 40; V128
+  // B16 (256 narrow) 60 + 64, 44 + 44; write keys K128 V256 T1024 B4 H4 58 + 53, 50 + 48; B8 H4 64 + 62, 58 + 55.
   return (int64_t)blocks_per_head * a.B * a.ns * a.H <= (int64_t)device_cu_count();
 }
 

@@ -759,9 +759,7 @@ static hipError_t bwd_state_bv(const ChunkArgs& a, bool local) {
 
 template <typename T, int K, bool SEPU>
 static hipError_t bwd_state_k(const ChunkArgs& a, bool local) {
-  if constexpr (sizeof(T) == 2 && !SEPU) {
-    if (narrow_sweep_blocks(a, a.V / 32)) return bwd_state_bv<T, K, SEPU, 32>(a, local);
-  }
+  if (narrow_sweep_blocks(a, a.V / 32)) return bwd_state_bv<T, K, SEPU, 32>(a, local);
   return bwd_state_bv<T, K, SEPU, 64>(a, local);
 }
 

@@ -312,9 +312,7 @@ static hipError_t fwd_sweep_bv(const ChunkArgs& a) {
 
 template <typename T, int K, int MODE, bool SEPU>
 static hipError_t fwd_sweep_k(const ChunkArgs& a) {
-  if constexpr (sizeof(T) == 2 && !SEPU) {
-    if (narrow_sweep_blocks(a, (a.V + (MODE == 3 ? K : 0)) / 32)) return fwd_sweep_bv<T, K, MODE, SEPU, 32>(a);
-  }
+  if (narrow_sweep_blocks(a, (a.V + (MODE == 3 ? K : 0)) / 32)) return fwd_sweep_bv<T, K, MODE, SEPU, 32>(a);
   return fwd_sweep_bv<T, K, MODE, SEPU, 64>(a);
 }
 

@@ -155,3 +155,33 @@ def test_segments_of_any_length(B, T, H, K, V, dtype):
     errs.update({n: rel_l2(a, b) for n, a, b in zip(NAMES, got, ref)})
     print("[segments of any length] rel-L2 " + ", ".join(f"{n} {e:.2e}" for n, e in errs.items()), flush=True)
     assert all(e <= 1e-2 for e in errs.values()), errs
+
+
+@pytest.mark.parametrize("K,V,sep", [(64, 64, False), (64, 128, False), (64, 64, True), (64, 256, True),
+                                     (128, 128, True), (128, 256, True)])
+def test_narrow_sweep_blocks_equal_wide(K, V, sep):
+    """fp32 and separate-write-key sweeps in 32-column blocks (a grid that fits the 256 CUs) and in 64-column ones (one
+    that does not): a column's arithmetic is the same in both, so a sequence alone equals itself in the batch bit for
+    bit.  (Their agreement with the oracle: the tests above and those of each op.)"""
+    T, H = 100, 2
+    B = 256 * 32 // (V * H) + 1  # one sequence past the narrow grid's limit
+    banner(f"narrow and wide sweep blocks B={B} T={T} H={H} K={K} V={V} separate write keys {sep}")
+    dt = torch.bfloat16 if sep else torch.float32
+    _, d = device_inputs(B, T, H, K, V, dt, seed=61, h0_std=0.1, with_do=True)
+    dhT = 0.1 * torch.randn(B, H, K, V, generator=torch.Generator().manual_seed(62)).cuda()
+    u = (d.k.float() * d.beta.float()[..., None]).to(dt)
+
+    def run(n):
+        q, k, v, g, beta, h0, do, dh, uu = (t[:n].contiguous() for t in (d.q, d.k, d.v, d.g, d.beta, d.h0, d.do, dhT, u))
+        if sep:
+            o, hT, stash = ops.nsgdn_chunk_fwd(q, k, uu, v, g, h0, 0.5)
+            return (o, hT) + tuple(ops.nsgdn_chunk_bwd(q, k, uu, v, g, h0, do, dh, stash, 0.5))
+        o, hT = ops.chunk_fwd(q, k, v, g, beta, h0, 0.5)
+        _, _, stash = ops.chunk_fwd_stash(q, k, v, g, beta, h0, 0.5)
+        return (o, hT) + tuple(ops.chunk_bwd(q, k, v, g, beta, h0, do, dh, 0.5)) + tuple(
+            ops.chunk_bwd_stashed(q, k, v, g, beta, h0, do, dh, stash, 0.5))
+
+    wide, narrow = run(B), run(1)
+    torch.cuda.synchronize()
+    for a, b in zip(wide, narrow):
+        assert torch.isfinite(b.float()).all() and torch.equal(a[:1], b)
