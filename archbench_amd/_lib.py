@@ -68,11 +68,25 @@ SIGNATURES = {
     "gdn_token_scan_fwd": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _p, _i, _i, _i, _i, _i, _p]),
     "gdn_token_scan_bwd": (_i, [_p, _p, _p, _p, _p, _p, _sz, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i,
                                 _i, _i, _p]),
+    "gdn_decode_proj_supported": (_i, [_i, _i]),
+    "gdn_mixer_decode_stage": (_i, [_p, _p]),
     "gdn_profile_enable": (_i, [_i]),
     "gdn_profile_read": (_i, [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_i), _i]),
     "gdn_profile_stage_name": (ctypes.c_char_p, [_i]),
 }
-PROFILE_STAGES = 23
+PROFILE_STAGES = 24
+
+
+class DecodeStageArgs(ctypes.Structure):
+    """gdn_decode_stage_args of the C header."""
+    _fields_ = ([("x", _p)] + [("w_" + n, _p) for n in ("q", "k", "v", "g", "a", "b")]
+                + [(n, _p) for n in ("y", "gate", "ab")]
+                + [(n, _p * 3) for n in ("conv_w", "state_in", "state_out", "out")]
+                + [(n, _p) for n in ("A_log", "dt_bias", "g", "beta")]
+                + [(n, _i) for n in ("B", "d", "key_dim", "value_dim", "H", "W", "norm_group", "w_dtype", "conv_w_dtype",
+                                     "gate_dtype")]
+                + [("beta_scale", ctypes.c_float), ("g_min", ctypes.c_float)])
+
 
 _lock = threading.Lock()
 _lib = None

@@ -192,13 +192,13 @@ static hipError_t copy_or_zero(const float* src, float* dst, int64_t n, hipStrea
 enum Stage {
   ST_FWD = 0, ST_BWD_RECOMP, ST_BWD_STATE, ST_BWD_INTRA, ST_STEP, ST_FWD_STASH, ST_FACTORS, ST_CONV_FWD,
   ST_CONV_BWD, ST_NORM_FWD, ST_NORM_BWD, ST_GATES_FWD, ST_GATES_BWD, ST_L2_FWD, ST_L2_BWD, ST_CE, ST_PREFIX,
-  ST_SEGSCAN, ST_BWD_LOCAL, ST_WD_FWD, ST_WD_BWD, ST_TSCAN_FWD, ST_TSCAN_BWD, ST_COUNT
+  ST_SEGSCAN, ST_BWD_LOCAL, ST_WD_FWD, ST_WD_BWD, ST_TSCAN_FWD, ST_TSCAN_BWD, ST_DECODE_IN, ST_COUNT
 };
 static const char* kStageNames[ST_COUNT] = {"fwd", "bwd_recompute", "bwd_state", "bwd_intra", "step", "fwd_stash",
                                             "factors", "conv_fwd", "conv_bwd", "norm_fwd", "norm_bwd", "gates_fwd", "gates_bwd",
                                             "l2norm_fwd", "l2norm_bwd", "cross_entropy", "prefix", "seg_scan",
                                             "bwd_local", "write_dir_fwd", "write_dir_bwd", "token_scan_fwd",
-                                            "token_scan_bwd"};
+                                            "token_scan_bwd", "decode_in"};
 struct ProfRec { int stage; hipEvent_t a, b; };
 struct Prof {
   std::atomic<bool> on{false};
@@ -724,6 +724,64 @@ int gdn_mixer_stage_fwd(const void* y, const float* w, void* q, void* k, void* v
   a.norm_group = norm_group; a.dtype = dtype; a.stream = static_cast<hipStream_t>(stream);
   const hipError_t e = timed(ST_CONV_FWD, a.stream, [&] { return launch_conv(a, false); });
   if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "mixer input stage forward launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
+int gdn_decode_proj_supported(int B, int d) { return decode_proj_supported(B, d) ? 1 : 0; }
+
+int gdn_mixer_decode_stage(const gdn_decode_stage_args* s, void* stream) {
+  g_err[0] = 0;
+  if (!s) return fail(GDN_ERR_ARG, "args is NULL");
+  if (int e = stage_check(s->B, 1, s->key_dim, s->value_dim, s->W, s->norm_group, DT_BF16)) return e;
+  if (s->norm_group == 0) return fail(GDN_ERR_SHAPE, "norm_group must be 64, 128 or 256");
+  for (int dt : {s->w_dtype, s->conv_w_dtype, s->gate_dtype})
+    if (dt != DT_F32 && dt != DT_BF16) return fail(GDN_ERR_ARG, "dtype code %d is not GDN_DTYPE_F32/BF16", dt);
+  if (s->H <= 0 || (int64_t)s->B * s->H > INT32_MAX / 2) return fail(GDN_ERR_ARG, "invalid B=%d H=%d", s->B, s->H);
+  const int D = 2 * s->key_dim + s->value_dim;
+  if ((int64_t)s->B * (D / 64 + 3) > INT32_MAX) return fail(GDN_ERR_ARG, "grid too large");
+  if (s->B == 0) return GDN_OK;
+  if (!s->y || !s->ab || !s->A_log || !s->dt_bias || !s->g || !s->beta)
+    return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(s->x, s->w_q, s->w_k, s->w_v, s->w_g, s->w_a, s->w_b, s->y, s->gate, s->ab))
+    return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  DecodeStageArgs a{};
+  for (int i = 0; i < 3; ++i) {
+    if (!s->conv_w[i] || !s->state_in[i] || !s->state_out[i] || !s->out[i])
+      return fail(GDN_ERR_ARG, "null input/output pointer");
+    if (misaligned(s->conv_w[i], s->state_in[i], s->state_out[i], s->out[i]))
+      return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+    if (s->state_out[i] == s->state_in[i]) return fail(GDN_ERR_ARG, "state_out must not alias state_in");
+    a.w[i] = s->conv_w[i], a.state_in[i] = s->state_in[i], a.state_out[i] = s->state_out[i], a.out[i] = s->out[i];
+    a.n[i] = i < 2 ? s->key_dim : s->value_dim;
+  }
+  a.y = s->y, a.ab = s->ab, a.A_log = s->A_log, a.dt_bias = s->dt_bias, a.g = s->g, a.beta = s->beta;
+  a.B = s->B, a.H = s->H, a.norm_group = s->norm_group, a.w_dtype = s->conv_w_dtype, a.gate_dtype = s->gate_dtype;
+  a.beta_scale = s->beta_scale, a.g_min = s->g_min, a.stream = static_cast<hipStream_t>(stream);
+  DecodeProjArgs p{};
+  if (s->x) {
+    if (!decode_proj_supported(s->B, s->d))
+      return fail(GDN_ERR_SHAPE, "decode projections take 1 to %d tokens and d a multiple of 32, got %d and d=%d",
+                  DECODE_MAX_TOKENS, s->B, s->d);
+    if (!s->w_q || !s->w_k || !s->w_v || !s->w_a || !s->w_b || !s->w_g != !s->gate)
+      return fail(GDN_ERR_ARG, "null input/output pointer");
+    auto y = [](void* base, int col) -> void* { return static_cast<uint16_t*>(base) + col; };  // bf16 columns
+    auto add = [&](const void* w, void* out, int rows, int ld) {
+      p.w[p.n] = w, p.y[p.n] = out, p.rows[p.n] = rows, p.ld[p.n] = ld;
+      ++p.n;
+    };
+    add(s->w_q, y(s->y, 0), s->key_dim, D);
+    add(s->w_k, y(s->y, s->key_dim), s->key_dim, D);
+    add(s->w_v, y(s->y, 2 * s->key_dim), s->value_dim, D);
+    if (s->w_g) add(s->w_g, s->gate, s->value_dim, s->value_dim);
+    add(s->w_a, y(s->ab, 0), s->H, 2 * s->H);
+    add(s->w_b, y(s->ab, s->H), s->H, 2 * s->H);
+    p.x = s->x, p.M = s->B, p.d = s->d, p.w_dtype = s->w_dtype, p.stream = a.stream;
+  }
+  const hipError_t e = timed(ST_DECODE_IN, a.stream, [&] {
+    const hipError_t r = p.n ? launch_decode_proj(p) : hipSuccess;
+    return r == hipSuccess ? launch_decode_stage(a) : r;
+  });
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "decode input stage launch: %s", hipGetErrorString(e));
   return GDN_OK;
 }
 

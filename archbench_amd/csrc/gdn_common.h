@@ -41,6 +41,14 @@ __device__ __forceinline__ float to_f(bf16 x) { return static_cast<float>(x); }
 template <typename T> __device__ __forceinline__ T from_f(float x);
 template <> __device__ __forceinline__ float from_f<float>(float x) { return x; }
 template <> __device__ __forceinline__ bf16 from_f<bf16>(float x) { return static_cast<bf16>(x); }
+// The gates of a gated DeltaNet head: log-retention g = -exp(A_log) softplus(xa) (torch's softplus threshold), at least
+// g_min, and write strength beta = beta_scale sigmoid(xb)
+__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+__device__ __forceinline__ float gate_g(float xa, float A_log, float g_min) {
+  return fmaxf(-expf(A_log) * softplus_f(xa), g_min);
+}
+__device__ __forceinline__ float gate_beta(float xb, float beta_scale) { return beta_scale * (1.f / (1.f + expf(-xb))); }
+
 // a0 b0 + a1 b1 + c: for bf16 one v_dot2c_f32_bf16 (exact bf16 products, fp32 sum) in place of four conversions
 // and two FMAs
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));

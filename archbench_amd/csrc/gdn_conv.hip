@@ -168,9 +168,9 @@ struct ConvItem {
 // Forward: grid ceil(B * nchunk * blocks / CONV_WAVES), CONV_WAVES waves.  Rows are loaded in batches of CONV_UF with
 // the next batch in flight while the current one is computed; the prefetch of the last batch re-reads it (start clamped
 // to t1 - CONV_UF) so every load stays inside the chunk.  D: all channels (those of w and the states).
-template <typename T, int W, int NG>
+template <typename T, int W, int NG, typename WT>
 __device__ __forceinline__ void conv_fwd_wave(const ConvItem<T>& it, const T* __restrict__ x,
-                                              const float* __restrict__ w, const float* __restrict__ bias,
+                                              const WT* __restrict__ w, const float* __restrict__ bias,
                                               const T* __restrict__ state_in, T* __restrict__ state_out, int Tn, int D,
                                               int ldx) {
   constexpr int CPL = CONV_CPL, U = CONV_UF;
@@ -187,7 +187,7 @@ __device__ __forceinline__ void conv_fwd_wave(const ConvItem<T>& it, const T* __
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
 #pragma unroll
-    for (int i = 0; i < W; ++i) wk[j][i] = act_round<T>(w[(cc + j) * W + i]);
+    for (int i = 0; i < W; ++i) wk[j][i] = act_round<T>(to_f(w[(cc + j) * W + i]));
     bk[j] = bias ? bias[cc + j] : 0.f;
   }
   float win[W - 1][CPL];
@@ -266,6 +266,52 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void conv_silu_fwd_kernel(const T*
     if (it.norm) return conv_fwd_wave<T, W, NG>(it, x, w, bias, state_in, state_out, Tn, D, ldx);
   }
   conv_fwd_wave<T, W, 0>(it, x, w, bias, state_in, state_out, Tn, D, ldx);
+}
+
+// One decoded token per sequence: a wave per (b, 256-channel block of q, k or v), each convolution with its own taps and
+// states, then the workgroups of the gates, an element per thread.  Latency-bound: 4.0 us at B8 H8, where three
+// convolutions, the gates and the copies and casts in front of them took 25 us in eleven launches.
+struct DecodeParam {
+  const void* p;
+  bool half;
+  __device__ __forceinline__ float operator[](int i) const {
+    return half ? to_f(static_cast<const bf16*>(p)[i]) : static_cast<const float*>(p)[i];
+  }
+};
+template <typename WT, int NG>
+__global__ __launch_bounds__(64 * CONV_WAVES) void decode_stage_kernel(DecodeStageArgs a, int conv_wgs) {
+  if ((int)blockIdx.x >= conv_wgs) {
+    const int e = ((int)blockIdx.x - conv_wgs) * 64 * CONV_WAVES + threadIdx.x;
+    if (e < a.B * a.H) {
+      const int b = e / a.H, h = e - b * a.H;
+      const bf16* ab = static_cast<const bf16*>(a.ab) + (int64_t)b * 2 * a.H;
+      const bool half = a.gate_dtype == DT_BF16;
+      a.g[e] = gate_g(to_f(ab[h]) + DecodeParam{a.dt_bias, half}[h], DecodeParam{a.A_log, half}[h], a.g_min);
+      a.beta[e] = gate_beta(to_f(ab[a.H + h]), a.beta_scale);
+    }
+    return;
+  }
+  const int nb0 = (a.n[0] + CONV_CW - 1) / CONV_CW, nb1 = nb0 + (a.n[1] + CONV_CW - 1) / CONV_CW;
+  const int ncb = nb1 + (a.n[2] + CONV_CW - 1) / CONV_CW;
+  const int item = (int)blockIdx.x * CONV_WAVES + __builtin_amdgcn_readfirstlane(wave_id());
+  if (item >= a.B * ncb) return;
+  auto pick = [&](int gi, auto x0, auto x1, auto x2) { return gi == 0 ? x0 : gi == 1 ? x1 : x2; };
+  ConvItem<bf16> it;
+  it.part = it.b = item / ncb;
+  const int blk = item - it.b * ncb, gi = (blk >= nb0) + (blk >= nb1);
+  it.t0 = 0, it.t1 = 1;
+  it.cw0 = (blk - pick(gi, 0, nb0, nb1)) * CONV_CW;
+  it.xc0 = 0;
+  it.n = pick(gi, a.n[0], a.n[1], a.n[2]);
+  it.norm = gi < 2;
+  it.p = static_cast<bf16*>(pick(gi, a.out[0], a.out[1], a.out[2]));
+  const bf16* y = static_cast<const bf16*>(a.y) + pick(gi, 0, a.n[0], a.n[0] + a.n[1]);
+  const WT* w = static_cast<const WT*>(pick(gi, a.w[0], a.w[1], a.w[2]));
+  const bf16* sin = static_cast<const bf16*>(pick(gi, a.state_in[0], a.state_in[1], a.state_in[2]));
+  bf16* sout = static_cast<bf16*>(pick(gi, a.state_out[0], a.state_out[1], a.state_out[2]));
+  const int ldx = a.n[0] + a.n[1] + a.n[2];
+  if (it.norm) return conv_fwd_wave<bf16, 4, NG>(it, y, w, nullptr, sin, sout, 1, it.n, ldx);
+  conv_fwd_wave<bf16, 4, 0>(it, y, w, nullptr, sin, sout, 1, it.n, ldx);
 }
 
 // grid and waves as in the forward; partial sums of dw and dbias per (b, chunk) = part.
@@ -546,6 +592,22 @@ static hipError_t conv_dispatch(const ConvArgs& a, bool backward) {
     case 256: return conv_k<T, 256>(a, backward);
   }
   return hipErrorInvalidValue;
+}
+
+template <typename WT>
+static hipError_t decode_stage_w(const DecodeStageArgs& a) {
+  const int wgs = (int)conv_grid(conv_blocks(a.n), a.B).x, gate_wgs = (a.B * a.H + 64 * CONV_WAVES - 1) / (64 * CONV_WAVES);
+  const dim3 grid(wgs + gate_wgs), block(64 * CONV_WAVES);
+  switch (a.norm_group) {
+    case 64: decode_stage_kernel<WT, 64><<<grid, block, 0, a.stream>>>(a, wgs); break;
+    case 128: decode_stage_kernel<WT, 128><<<grid, block, 0, a.stream>>>(a, wgs); break;
+    case 256: decode_stage_kernel<WT, 256><<<grid, block, 0, a.stream>>>(a, wgs); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+hipError_t launch_decode_stage(const DecodeStageArgs& a) {
+  return a.w_dtype == DT_BF16 ? decode_stage_w<bf16>(a) : decode_stage_w<float>(a);
 }
 
 hipError_t launch_conv(const ConvArgs& a, bool backward) {

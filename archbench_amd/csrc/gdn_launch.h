@@ -126,6 +126,37 @@ size_t conv_ws_bytes(int B, int T, const int (&n)[3], int W);
 bool conv_shape_supported(int D, int W, int norm_group);
 hipError_t launch_conv(const ConvArgs& a, bool backward);
 
+// One decoded token per sequence (M of them): y_i [M] rows of rows_i outputs, ld_i elements apart, = x [M, d] W_i^T,
+// bf16 activations.
+constexpr int DECODE_MAX_WEIGHTS = 6, DECODE_MAX_TOKENS = 128;
+struct DecodeProjArgs {
+  const void* x;
+  const void* w[DECODE_MAX_WEIGHTS];  // [rows, d] in w_dtype
+  void* y[DECODE_MAX_WEIGHTS];
+  int rows[DECODE_MAX_WEIGHTS], ld[DECODE_MAX_WEIGHTS];
+  int n, M, d, w_dtype;
+  hipStream_t stream;
+};
+bool decode_proj_supported(int M, int d);
+hipError_t launch_decode_proj(const DecodeProjArgs& a);
+
+// The rest of the mixer's input stage for one decoded token in bf16: the three short convolutions from their states
+// (q and k normalised) and the gates.
+struct DecodeStageArgs {
+  const void* y;            // [B, n[0] + n[1] + n[2]]: q's, k's and v's channels
+  const void* w[3];         // [n[i], 4] in w_dtype
+  const void* state_in[3];  // [B, n[i], 3]
+  void* state_out[3];
+  void* out[3];             // [B, n[i]]
+  const void* ab;           // [B, 2 H]
+  const void *A_log, *dt_bias;  // [H] in gate_dtype
+  float *g, *beta;          // [B, H]
+  int B, n[3], H, norm_group, w_dtype, gate_dtype;
+  float beta_scale, g_min;
+  hipStream_t stream;
+};
+hipError_t launch_decode_stage(const DecodeStageArgs& a);
+
 // Destinations of consecutive column ranges: columns [0, n[0]) go to p[0], the next n[1] to p[1], the next n[2]
 // to p[2]; a null p drops its range.
 struct ColumnOut {

@@ -178,8 +178,6 @@ __global__ __launch_bounds__(64 * NORM_WAVES) void row_norm_bwd_kernel(
 }
 
 // ------------------------------------------------------------------------------------------------ gates
-__device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(expf(x)); }  // torch threshold
-
 template <typename T>
 __global__ __launch_bounds__(256) void gates_fwd_kernel(const T* __restrict__ a, const T* __restrict__ b,
                                                         const float* __restrict__ A_log,
@@ -191,9 +189,9 @@ __global__ __launch_bounds__(256) void gates_fwd_kernel(const T* __restrict__ a,
     const int64_t t = e / H;
     const int h = (int)(e - t * H);
     const float xa = to_f(a[t * lda + h]) + (dt_bias ? dt_bias[h] : 0.f);
-    g[e] = fmaxf(-expf(A_log[h]) * softplus_f(xa), g_min);
+    g[e] = gate_g(xa, A_log[h], g_min);
     const float xb = to_f(b[t * lda + h]) + (b_bias ? b_bias[h] : 0.f);
-    beta[e] = beta_scale * (1.f / (1.f + expf(-xb)));
+    beta[e] = gate_beta(xb, beta_scale);
   }
 }
 

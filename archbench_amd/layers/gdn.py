@@ -170,15 +170,36 @@ class GatedDeltaNet(nn.Module):
         self.o_norm = GatedRMSNorm(self.head_v_dim, norm_eps)
         self.o_proj = nn.Linear(self.value_dim, hidden_size, bias=False)
 
+    def _input_linears(self) -> list[nn.Module]:
+        gate = [self.g_proj] if self.use_gate else []
+        return [self.q_proj, self.k_proj, self.v_proj, *gate, self.a_proj, self.b_proj]
+
+    def _decode_stage_applies(self, x: torch.Tensor, convs, conv_in) -> bool:
+        """One cached token per sequence in bf16 without grad, plain convolutions with the states they would take: the
+        projections, convolutions and gates then run as one op (ops.mixer_decode_stage) instead of seven.  Anything
+        else, hooks on the convolutions included, takes the separate ops."""
+        if torch.is_grad_enabled() or not x.is_cuda or x.dtype != torch.bfloat16 or x.shape[1] != 1 or not convs:
+            return False
+        if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
+            return False
+        if self.head_k_dim not in (64, 128, 256) or len(conv_in) != 3:
+            return False
+        kd, vd, dk = self.key_dim, self.value_dim, self.head_k_dim
+        for c, s, n, norm in zip(convs, conv_in, (kd, kd, vd), (dk, dk, 0)):
+            if (type(c) is not ShortConvolution or c._forward_hooks or c._forward_pre_hooks or c.bias is not None
+                    or c.size != 4 or c.norm_group != norm or n % 4):
+                return False
+            if not isinstance(s, torch.Tensor) or s.shape != (x.shape[0], n, 3):
+                return False
+        return True
+
     def _grouped_projections(self, hidden_states: torch.Tensor):
         """([q | k | v], gate or None, [a | b]): the six input linears against their concatenated weights, one GEMM
         per group."""
-        mods = [self.q_proj, self.k_proj, self.v_proj] + ([self.g_proj] if self.use_gate else [])
-        mods += [self.a_proj, self.b_proj]
         n_qkv = 2 * self.key_dim + self.value_dim
         bounds = [0, n_qkv] + ([n_qkv + self.value_dim] if self.use_gate else [])
         bounds.append(bounds[-1] + self.a_proj.out_features + self.b_proj.out_features)
-        outs = _grouped_linear(hidden_states, torch.cat([m.weight for m in mods], 0), bounds)
+        outs = _grouped_linear(hidden_states, torch.cat([m.weight for m in self._input_linears()], 0), bounds)
         return outs[0], (outs[1] if self.use_gate else None), outs[-1]
 
     def input_projections(self, hidden_states: torch.Tensor) -> tuple[torch.Tensor, ...]:
@@ -208,6 +229,7 @@ class GatedDeltaNet(nn.Module):
         entry = None if past_key_values is None else past_key_values.get(self.layer_idx)
         conv_in = entry["conv_state"] if entry is not None else (None, None, None)
         conv_out = (None, None, None)
+        ab, gates_done = None, False
         convs = (self.q_conv1d, self.k_conv1d, self.v_conv1d) if self.use_short_conv else ()
         if convs and entry is None and not use_cache and all(c.bias is None for c in convs):
             # training / prefill without a cache: the convolutions read q, k, v straight out of the projection's
@@ -216,8 +238,13 @@ class GatedDeltaNet(nn.Module):
             w = torch.cat([c.weight.squeeze(1) for c in convs], 0)
             q, k, v = ops.mixer_input_stage(y, w, self.key_dim, self.value_dim, DK)
             gp = [gate] if self.use_gate else []
+        elif self._decode_stage_applies(hidden_states, convs, conv_in):
+            w_in = [m.weight for m in self._input_linears()]
+            q, k, v, g, beta, cq, ck, cv, *gp = ops.mixer_decode_stage(
+                hidden_states, w_in, [c.weight for c in convs], list(conv_in), self.A_log, self.dt_bias, DK,
+                2.0 if self.allow_neg_eigval else 1.0, float("-inf"))
+            conv_out, gates_done = (cq, ck, cv), True
         else:
-            ab = None
             q, k, v, a, b, *gp = self.input_projections(hidden_states)
             if convs:
                 (q, cq), (k, ck), (v, cv) = (self.q_conv1d(q, conv_in[0]), self.k_conv1d(k, conv_in[1]),
@@ -229,7 +256,9 @@ class GatedDeltaNet(nn.Module):
         # g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b) (x2 with negative eigenvalues), one HIP pass;
         # from the [a | b] projection output in place when there is one
         scale_b = 2.0 if self.allow_neg_eigval else 1.0
-        if ab is not None:
+        if gates_done:
+            pass
+        elif ab is not None:
             g, beta = ops.gdn_gates_ab(ab, self.A_log, self.dt_bias, None, scale_b, float("-inf"))
         else:
             g, beta = ops.gdn_gates(a, b, self.A_log, self.dt_bias, None, scale_b, float("-inf"))

@@ -727,6 +727,87 @@ def _conv_backward(ctx, dy, dstate_out):
 short_conv.register_autograd(_conv_backward, setup_context=_conv_setup)
 
 
+# The mixer's input stage for one decoded token per sequence: projections, convolutions from their states and gates in
+# one op of two launches.  No autograd: decoding only.
+def _uniform(ts: list[Tensor]) -> int | None:
+    """The kernels' code of the tensors' one dtype if they can be read in place (bf16 or fp32, contiguous, aligned)."""
+    dt = ts[0].dtype
+    if dt not in (torch.bfloat16, torch.float32):
+        return None
+    if any(t.dtype != dt or not t.is_contiguous() or t.data_ptr() % 16 for t in ts):
+        return None
+    return _lib.dtype_code(dt)
+
+
+@torch.library.custom_op("archbench_amd::mixer_decode_stage", mutates_args=())
+def mixer_decode_stage(x: Tensor, w_in: list[Tensor], conv_w: list[Tensor], conv_state: list[Tensor], A_log: Tensor,
+                       dt_bias: Tensor, norm_group: int, beta_scale: float, g_min: float) -> list[Tensor]:
+    """[q, k, v, g, beta, new q state, new k state, new v state(, gate)] of x [B, 1, d] bf16: the linears w_in = [q, k,
+    v(, gate), a, b] ([rows, d]), the convolutions conv_w ([D, 1, W], no bias) from conv_state ([B, D, W-1]) with q and k
+    normalised per norm_group channels, and the gates.  The same values as the separate ops, the projections' fp32
+    sums in another order."""
+    if any(t.device != x.device for t in (*w_in, *conv_w, *conv_state, A_log, dt_bias)):
+        raise RuntimeError(f"expected every tensor on {x.device}, the device of x")
+    _require_gpu(x)
+    if x.dim() != 3 or x.shape[1] != 1 or x.dtype != torch.bfloat16:
+        raise ValueError(f"x must be [B, 1, d] bf16, got {tuple(x.shape)} {x.dtype}")
+    if len(w_in) not in (5, 6) or len(conv_w) != 3 or len(conv_state) != 3:
+        raise ValueError("w_in must be [q, k, v(, gate), a, b], conv_w and conv_state [q, k, v]")
+    B, _, d = x.shape
+    rows = [w.shape[0] for w in w_in]
+    if any(w.dim() != 2 or w.shape[1] != d for w in w_in):
+        raise ValueError(f"w_in must be [rows, {d}], got {[tuple(w.shape) for w in w_in]}")
+    kd, vd, H, W = rows[0], rows[2], rows[-1], conv_w[0].shape[-1]
+    if rows != [kd, kd, vd] + [vd] * (len(rows) - 5) + [H, H] or A_log.shape != (H,) or dt_bias.shape != (H,):
+        raise ValueError(f"projections of {rows} rows with {tuple(A_log.shape)} gates")
+    for w, s, n in zip(conv_w, conv_state, (kd, kd, vd)):
+        if w.numel() != n * W or w.shape[0] != n or s.shape != (B, n, W - 1):
+            raise ValueError(f"conv weight {tuple(w.shape)} and state {tuple(s.shape)} for {B} x {n} channels")
+    lib, dev, bf = _lib.load(), x.device, torch.bfloat16
+    x = _arg(x)
+    y, ab = x.new_empty(B, 2 * kd + vd), x.new_empty(B, 2 * H)
+    gate = x.new_empty(B, 1, vd) if len(w_in) == 6 else None
+    a = _lib.DecodeStageArgs()
+    # the weights where they lie; otherwise concatenated in front of three GEMMs
+    code = _uniform(w_in) if lib.gdn_decode_proj_supported(B, d) else None
+    if code is not None:
+        a.x, a.w_dtype = x.data_ptr(), code
+        for n, w in zip(("q", "k", "v", "g", "a", "b") if len(w_in) == 6 else ("q", "k", "v", "a", "b"), w_in):
+            setattr(a, "w_" + n, w.data_ptr())
+    elif B > 0:
+        wc, x2 = torch.cat(w_in, 0).to(bf), x.view(B, d)
+        n_qkv = 2 * kd + vd
+        torch.mm(x2, wc[:n_qkv].t(), out=y)
+        torch.mm(x2, wc[-2 * H:].t(), out=ab)
+        if gate is not None:
+            torch.mm(x2, wc[n_qkv:-2 * H].t(), out=gate.view(B, vd))
+    cw = conv_w if _uniform(conv_w) is not None else [_arg(w, torch.float32) for w in conv_w]
+    gp = [A_log, dt_bias] if _uniform([A_log, dt_bias]) is not None else [_arg(t, torch.float32) for t in (A_log, dt_bias)]
+    state = [_arg(s, bf) for s in conv_state]
+    out = [x.new_empty(B, 1, n) for n in (kd, kd, vd)]
+    new_state = [x.new_empty(B, n, W - 1) for n in (kd, kd, vd)]
+    g, beta = torch.empty(B, 1, H, dtype=torch.float32, device=dev), torch.empty(B, 1, H, dtype=torch.float32, device=dev)
+    a.y, a.ab, a.gate = y.data_ptr(), ab.data_ptr(), None if gate is None else gate.data_ptr()
+    for i in range(3):
+        a.conv_w[i], a.state_in[i] = cw[i].data_ptr(), state[i].data_ptr()
+        a.state_out[i], a.out[i] = new_state[i].data_ptr(), out[i].data_ptr()
+    a.A_log, a.dt_bias, a.g, a.beta = gp[0].data_ptr(), gp[1].data_ptr(), g.data_ptr(), beta.data_ptr()
+    a.B, a.d, a.key_dim, a.value_dim, a.H, a.W, a.norm_group = B, d, kd, vd, H, W, int(norm_group)
+    a.conv_w_dtype, a.gate_dtype = _lib.dtype_code(cw[0].dtype), _lib.dtype_code(gp[0].dtype)
+    a.beta_scale, a.g_min = float(beta_scale), float(g_min)
+    _lib.check(lib.gdn_mixer_decode_stage(ctypes.byref(a), _lib.stream_ptr(dev)), "gdn_mixer_decode_stage")
+    return [*out, g, beta, *new_state] + ([] if gate is None else [gate])
+
+
+@mixer_decode_stage.register_fake
+def _(x, w_in, conv_w, conv_state, A_log, dt_bias, norm_group, beta_scale, g_min):
+    B, H = x.shape[0], w_in[-1].shape[0]
+    dims = [w.shape[0] for w in w_in[:3]]
+    r = [x.new_empty(B, 1, n) for n in dims] + [x.new_empty(B, 1, H, dtype=torch.float32) for _ in range(2)]
+    r += [x.new_empty(B, n, w.shape[-1] - 1) for n, w in zip(dims, conv_w)]
+    return r + ([x.new_empty(B, 1, dims[2])] if len(w_in) == 6 else [])
+
+
 # The mixer's input stage in one op: q, k and v convolved straight out of the q/k/v input projection's output y
 # [B, T, 2 key_dim + value_dim] (its column groups, read in place), with one weight [2 key_dim + value_dim, W] for
 # the three convolutions (q's rows, then k's, then v's), in one launch.  The backward, one launch and the sum of its

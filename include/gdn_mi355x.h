@@ -168,6 +168,28 @@ int gdn_mixer_stage_bwd(const void* y, const float* w, const void* dq, const voi
                         float* dw, void* ws, size_t ws_bytes, int B, int T, int key_dim, int value_dim, int W,
                         int norm_group, int dtype, void* stream);
 
+/* The mixer's input stage for one decoded token per sequence (T = 1, bf16 activations): the input projections, the three
+ * short convolutions from their states (no bias; q and k normalised per norm_group in {64, 128, 256} channels; W = 4)
+ * and the gates (as gdn_gates_fwd), in two launches.  With x NULL the projections are left out and y and ab read. */
+typedef struct {
+  const void* x;    /* [B, d], or NULL */
+  const void *w_q, *w_k, *w_v, *w_g, *w_a, *w_b; /* [rows, d] in w_dtype (rounded to bf16); w_g NULL: no gate */
+  void* y;          /* [B, 2 key_dim + value_dim]: the projections to q, k and v */
+  void* gate;       /* [B, value_dim] (with w_g) */
+  void* ab;         /* [B, 2 H]: the projections to a and b */
+  const void* conv_w[3];    /* [key_dim | key_dim | value_dim, 4] in conv_w_dtype */
+  const void* state_in[3];  /* [B, key_dim | key_dim | value_dim, 3] bf16 */
+  void* state_out[3];       /* the states after this token; not the same buffers */
+  void* out[3];             /* q, k [B, key_dim], v [B, value_dim] bf16 */
+  const void *A_log, *dt_bias; /* [H] in gate_dtype */
+  float *g, *beta;             /* [B, H] */
+  int B, d, key_dim, value_dim, H, W, norm_group, w_dtype, conv_w_dtype, gate_dtype;
+  float beta_scale, g_min;
+} gdn_decode_stage_args;
+/* 1 if the projections take B tokens of d channels (B <= 128, d a multiple of 32), else 0. */
+int gdn_decode_proj_supported(int B, int d);
+int gdn_mixer_decode_stage(const gdn_decode_stage_args* args, void* stream);
+
 /* Gated RMSNorm of the op's output, per row of `dim` channels (one head of one token):
  *   y = x * rsqrt(mean(x^2) + eps) * weight * silu(gate)
  * Replaces the output normalisation of the mixer: fla's FusedRMSNormGated in GatedDeltaNet and the reference's

@@ -385,3 +385,73 @@ def test_gdn_layer_matches_restatement(use_gate):
     for n, p in m.named_parameters():
         noise = rel_l2(gr_exact[n], gr[n])
         assert rel_l2(p.grad, gr[n]) <= 3e-2 + 4 * noise, (n, rel_l2(p.grad, gr[n]), noise)
+
+
+@pytest.mark.parametrize("B,d,H,dk,dv,gate,w_dtype", [
+    (1, 32, 1, 64, 64, True, torch.bfloat16), (5, 96, 3, 64, 128, False, torch.float32),
+    (16, 1024, 2, 128, 256, True, torch.float32), (17, 768, 3, 128, 256, True, torch.bfloat16),
+    (33, 288, 2, 256, 64, True, torch.bfloat16), (64, 320, 5, 64, 64, False, torch.bfloat16),
+    (65, 96, 2, 64, 64, True, torch.float32), (128, 64, 1, 64, 64, True, torch.bfloat16),
+    (129, 96, 2, 64, 64, True, torch.float32), (3, 80, 2, 64, 64, True, torch.bfloat16)])
+def test_decode_stage_matches_separate_ops(B, d, H, dk, dv, gate, w_dtype):
+    """One token's projections, convolutions and gates in one op: token tiles of 16 (1, 16, 17, 33, 64, 65, 128 tokens), partial
+    row blocks (a and b of 1 to 5 rows), steps of d that do not fill four waves, and the GEMM route (129 tokens; d not a
+    multiple of 32), against the same in fp64 from the projections rounded to bf16.  Bound: the projections' and the
+    outputs' bf16 roundings, 2^-9 each of a value, through a convolution of four taps: 1e-2 (rel-L2)."""
+    banner(f"decode stage B={B} d={d} H={H} K={dk} V={dv} gate={gate} {w_dtype}")
+    gen = torch.Generator().manual_seed(B + d)
+    r = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    rows = [H * dk, H * dk, H * dv] + ([H * dv] if gate else []) + [H, H]
+    x = r(B, 1, d).bfloat16()
+    w_in = [(r(n, d) * d ** -0.5).to(w_dtype) for n in rows]
+    conv_w = [(r(n, 1, 4) * 0.5).to(w_dtype) for n in rows[:3]]
+    state = [r(B, n, 3).bfloat16() for n in rows[:3]]
+    A_log, dt = r(H).to(w_dtype), r(H).to(w_dtype)
+    dev = lambda ts: [t.cuda() for t in ts]  # noqa: E731
+    out = ops.mixer_decode_stage(x.cuda(), dev(w_in), dev(conv_w), dev(state), A_log.cuda(), dt.cuda(), dk, 2.0, -4.0)
+    torch.cuda.synchronize()
+    assert len(out) == (9 if gate else 8)
+    y = [(x.double()[:, 0] @ w.bfloat16().double().t()).bfloat16().double() for w in w_in]
+    for i in range(3):
+        win = torch.cat([state[i].double(), y[i][..., None]], -1)
+        z = (win * conv_w[i].bfloat16().double()[:, 0]).sum(-1)
+        o = z * torch.sigmoid(z)
+        if i < 2:
+            o = torch.nn.functional.normalize(o.view(B, H, dk), dim=-1).view(B, -1)
+        assert out[i].dtype == torch.bfloat16 and rel_l2(out[i][:, 0].double().cpu(), o) <= 1e-2
+        st = out[5 + i].cpu()
+        assert torch.equal(st[..., :2], state[i][..., 1:]) and rel_l2(st.double(), win[..., 1:]) <= 1e-2
+    a, b = y[-2], y[-1]
+    g = (-A_log.double().exp() * torch.nn.functional.softplus(a + dt.double())).clamp_min(-4.0)
+    assert rel_l2(out[3][:, 0].double().cpu(), g) <= 1e-2
+    assert rel_l2(out[4][:, 0].double().cpu(), 2.0 * torch.sigmoid(b)) <= 1e-2
+    if gate:
+        assert rel_l2(out[8][:, 0].double().cpu(), y[3]) <= 1e-2
+
+
+def test_decode_stage_route_equals_separate_ops():
+    """A cached bf16 decode step takes the one-op input stage; a hook on a convolution takes the separate ops, and runs.
+    The two steps agree to the rounding of the projections (1e-2), their caches have the same form."""
+    banner("decode stage route")
+    m = _layer(4).eval()
+    x = torch.randn(3, 66, 256, device="cuda", generator=torch.Generator("cuda").manual_seed(8))
+    fired, res = [], []
+    for hooked in (False, True):
+        handle = m.layer.k_conv1d.register_forward_hook(lambda *_: fired.append(1)) if hooked else None
+        n0 = len(fired)
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16), _lib.StageTimer() as st:
+            _, _, cache = m.layer(x[:, :64], use_cache=True, past_key_values={})
+            for t in (64, 65):
+                y, _, cache = m.layer(x[:, t:t + 1], use_cache=True, past_key_values=cache)
+        assert ("decode_in" in st.result) == (not hooked) and len(fired) - n0 == (3 if hooked else 0)
+        if handle:
+            handle.remove()
+        res.append([y, cache[0]["recurrent_state"], *cache[0]["conv_state"]])
+    for a, b in zip(*res):
+        assert a.dtype == b.dtype and a.shape == b.shape and rel_l2(a.float(), b.float()) <= 1e-2
+    torch.library.opcheck(
+        torch.ops.archbench_amd.mixer_decode_stage.default,
+        (x[:, :1].bfloat16(), [w.weight.detach() for w in m.layer._input_linears()],
+         [c.weight.detach() for c in (m.layer.q_conv1d, m.layer.k_conv1d, m.layer.v_conv1d)],
+         [c.clone() for c in cache[0]["conv_state"]], m.layer.A_log.detach(), m.layer.dt_bias.detach(),
+         m.layer.head_k_dim, 1.0, float("-inf")), test_utils=("test_schema", "test_faketensor"))
