@@ -62,6 +62,8 @@ SIGNATURES = {
     "gdn_cross_entropy_fwd_bwd": (_i, [_p, _p, _p, _p, _p, _i64, _i, _i64, _i64, _i, _p]),
     "gdn_scale": (_i, [_p, _p, _p, _i64, _i, _p]),
     "gdn_sum_parts": (_i, [_p, _i, _p, _i64, _i, _p]),
+    "gdn_sum_parts_t": (_i, [_p, _i, _p, _i, _i, _i, _p]),
+    "gdn_narrow_dx": (_i, [_p, _p, _p, _p, _i64, _i, _i, _i, _p]),
     "gdn_write_direction_fwd": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p]),
     "gdn_write_direction_bwd": (_i, [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p]),
     "gdn_token_scan_sizes": (_i, [_i, _i, _i, _i, _i, ctypes.POINTER(_sz), ctypes.POINTER(_sz), ctypes.POINTER(_i)]),

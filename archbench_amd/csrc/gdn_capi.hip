@@ -967,6 +967,36 @@ int gdn_sum_parts(const float* part, int nparts, void* out, int64_t n, int dtype
   return GDN_OK;
 }
 
+int gdn_sum_parts_t(const float* part, int nparts, void* out, int N, int K, int dtype, void* stream) {
+  g_err[0] = 0;
+  if (dtype != DT_F32 && dtype != DT_BF16) return fail(GDN_ERR_ARG, "dtype code %d is not GDN_DTYPE_F32/BF16", dtype);
+  if (nparts < 1 || N < 0 || K < 0 || N % 4 || K % 4)
+    return fail(GDN_ERR_ARG, "nparts=%d must be >= 1, N=%d and K=%d multiples of 4", nparts, N, K);
+  if ((int64_t)(N / 64 + 1) * (K / 64 + 1) > INT32_MAX) return fail(GDN_ERR_ARG, "grid too large");
+  if (N == 0 || K == 0) return GDN_OK;
+  if (!part || !out) return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(part, out)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  const hipError_t e = launch_sum_parts_t(part, nparts, out, N, K, dtype, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "transposed sum of parts launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
+int gdn_narrow_dx(const void* dx, const void* a, const void* w, void* out, int64_t M, int C, int J, int out_dtype,
+                  void* stream) {
+  g_err[0] = 0;
+  if (out_dtype != DT_F32 && out_dtype != DT_BF16)
+    return fail(GDN_ERR_ARG, "dtype code %d is not GDN_DTYPE_F32/BF16", out_dtype);
+  if (M < 0 || C <= 0 || C % 4 || J < 2 || J > NARROW_MAX_J || J % 2)
+    return fail(GDN_ERR_ARG, "C=%d must be a multiple of 4, J=%d even and 2 to %d", C, J, NARROW_MAX_J);
+  if ((M / 32 + 1) * ((C + 255) / 256) > INT32_MAX) return fail(GDN_ERR_ARG, "grid too large");
+  if (M == 0) return GDN_OK;
+  if (!dx || !a || !w || !out) return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(dx, a, w, out)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
+  const hipError_t e = launch_narrow_dx(dx, a, w, out, M, C, J, out_dtype, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "narrow input gradient launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
 static int write_dir_check(int B, int T, int H, int K, int n_steps, int dtype) {
   if (dtype != DT_F32 && dtype != DT_BF16) return fail(GDN_ERR_ARG, "dtype code %d is not GDN_DTYPE_F32/BF16", dtype);
   if (B < 0 || T < 0 || H <= 0 || K <= 0) return fail(GDN_ERR_ARG, "invalid sizes B=%d T=%d H=%d K=%d", B, T, H, K);

@@ -227,6 +227,12 @@ hipError_t launch_ce(const CeArgs& a);
 // y = *s x over n elements; out = sum over nparts of part[p][n] (n a multiple of 8), rounded to dtype
 hipError_t launch_scale(const void* x, const float* s, void* y, int64_t n, int dtype, hipStream_t st);
 hipError_t launch_sum_parts(const float* part, int nparts, void* out, int64_t n, int dtype, hipStream_t st);
+// out [N, K] = sum over p of part[p] [K, N], transposed; N and K multiples of 4
+hipError_t launch_sum_parts_t(const float* part, int nparts, void* out, int N, int K, int dtype, hipStream_t st);
+// out [M, C] (bf16 or fp32) = dx [M, C] + a [M, J] w [J, C], bf16 operands; J even, at most 32; C a multiple of 4
+constexpr int NARROW_MAX_J = 32;
+hipError_t launch_narrow_dx(const void* dx, const void* a, const void* w, void* out, int64_t M, int C, int J,
+                            int out_dtype, hipStream_t st);
 
 // Write direction of the n-step family (gdn_writedir.hip): k [B,T,H,K] -> u, and the backward.
 struct WriteDirArgs {

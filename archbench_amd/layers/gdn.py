@@ -38,28 +38,47 @@ def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     N = 3072, K = 512), split 8 or 16 ways 27, 77 and 211 us.  The smaller operand's chunks enter the batched
     product as the transposed left operand (a layout the GEMM reads directly; copying them transposed first cost
     140 us at these sizes); the right operand is always contiguous."""
+    dw = torch.empty(dy.shape[1], x.shape[1], dtype=torch.float32, device=dy.device)
+    _weight_grad_(dw, dy, x)
+    return dw
+
+
+def _weight_grad_(dw: torch.Tensor, dy: torch.Tensor, x: torch.Tensor) -> None:
+    """_weight_grad into dw (contiguous rows of a larger gradient): a single product writes there itself, the chunk
+    products are summed there by one HIP pass, transposed where they were taken as x^T dy (a sum and a
+    transposing copy took 26 us for N = 2048, K = 512, the pass 12)."""
     M, N = dy.shape
     K = x.shape[1]
     C = 16 if N * K <= 1 << 20 else 8
+    own = dy.is_cuda and not torch.is_grad_enabled() and dw.is_contiguous() and dw.data_ptr() % 16 == 0
     if dy.dtype == torch.float32:
-        return dy.t() @ x
-    if M % C or M // C < 1024:
-        return torch.mm(dy.t(), x, out_dtype=torch.float32)
-    if N <= K:
-        return torch.bmm(dy.view(C, M // C, N).transpose(1, 2), x.view(C, M // C, K), out_dtype=torch.float32).sum(0)
-    return torch.bmm(x.view(C, M // C, K).transpose(1, 2), dy.view(C, M // C, N), out_dtype=torch.float32).sum(0).t()
+        dw.copy_(dy.t() @ x)
+    elif M % C or M // C < 1024:
+        if own:
+            torch.mm(dy.t(), x, out_dtype=torch.float32, out=dw)
+        else:
+            dw.copy_(torch.mm(dy.t(), x, out_dtype=torch.float32))
+    elif N <= K:
+        parts = torch.bmm(dy.view(C, M // C, N).transpose(1, 2), x.view(C, M // C, K), out_dtype=torch.float32)
+        ops.sum_parts_(parts, dw) if own and N * K % 8 == 0 else dw.copy_(parts.sum(0))
+    else:
+        parts = torch.bmm(x.view(C, M // C, K).transpose(1, 2), dy.view(C, M // C, N), out_dtype=torch.float32)
+        ops.sum_parts_t_(parts, dw) if own and N % 4 == 0 and K % 4 == 0 else dw.copy_(parts.sum(0).t())
 
 
 class _GroupedLinear(torch.autograd.Function):
     """y_g = x W[r_g:r_{g+1}]^T for consecutive row groups of one weight: one GEMM per group, each output its own
-    contiguous tensor, W cast to x's dtype once (as autocast casts it).  Backward: the groups' input gradients
-    accumulated in place into the first (dx += dy_g W_g in the GEMM, no separate sum), and each group's weight
-    gradient split over the tokens (_weight_grad) written into its rows of one fp32 gradient (rows outside every
-    group: zero), returned in W's dtype."""
+    contiguous tensor, x and W cast to ``dtype`` once (as autocast casts them).  Backward: the groups' input gradients
+    accumulated in place into the first (dx += dy_g W_g in the GEMM, no separate sum), the last group's, when it has a
+    few columns only (a and b), together with the cast to x's dtype (ops.narrow_dx), and each group's weight gradient
+    split over the tokens (_weight_grad_) written into its rows of one fp32 gradient (rows outside every group: zero),
+    returned in W's dtype."""
 
     @staticmethod
-    def forward(ctx, x: torch.Tensor, w: torch.Tensor, bounds: tuple):
-        wc = w.to(x.dtype)
+    def forward(ctx, x: torch.Tensor, w: torch.Tensor, bounds: tuple, dtype: torch.dtype):
+        ctx.x_dtype = x.dtype
+        x = x.to(dtype)
+        wc = w.to(dtype)
         ctx.save_for_backward(x, wc)
         ctx.bounds, ctx.w_dtype = bounds, w.dtype
         return tuple(F.linear(x, wc[r0:r1]) for r0, r1 in zip(bounds[:-1], bounds[1:]))
@@ -72,27 +91,43 @@ class _GroupedLinear(torch.autograd.Function):
         x2 = x.reshape(-1, x.shape[-1])
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            for r0, r1, dy in groups:
-                if dy is not None:
-                    dx = dy @ wc[r0:r1] if dx is None else dx.addmm_(dy, wc[r0:r1])
-            dx = torch.zeros_like(x) if dx is None else dx.view(x.shape)
+            for i, (r0, r1, dy) in enumerate(groups):
+                if dy is None:
+                    continue
+                if dx is None:
+                    dx = dy @ wc[r0:r1]
+                elif i == len(groups) - 1 and _narrow_dx_applies(dx, dy, ctx.x_dtype):
+                    dx = ops.narrow_dx(dx, dy, wc[r0:r1], ctx.x_dtype == torch.float32)
+                else:
+                    dx.addmm_(dy, wc[r0:r1])
+            dx = torch.zeros_like(x, dtype=ctx.x_dtype) if dx is None else dx.to(ctx.x_dtype).view(x.shape)
         if ctx.needs_input_grad[1]:
-            whole = ctx.bounds[0] == 0 and ctx.bounds[-1] == wc.shape[0] and all(g[2] is not None for g in groups)
-            dw = (torch.empty if whole else torch.zeros)(wc.shape, dtype=torch.float32, device=wc.device)
-            for r0, r1, dy in groups:
+            dw = torch.empty(wc.shape, dtype=torch.float32, device=wc.device)
+            for r0, r1, dy in [(0, ctx.bounds[0], None), *groups, (ctx.bounds[-1], wc.shape[0], None)]:
                 if dy is not None:
-                    dw[r0:r1] = _weight_grad(dy, x2)
+                    _weight_grad_(dw[r0:r1], dy, x2)
+                elif r1 > r0:
+                    dw[r0:r1].zero_()
             dw = dw.to(ctx.w_dtype)
-        return dx, dw, None
+        return dx, dw, None, None
 
 
-def _grouped_linear(x: torch.Tensor, w: torch.Tensor, bounds) -> tuple[torch.Tensor, ...]:
-    """(x W[r_0:r_1]^T, x W[r_1:r_2]^T, ...) for row bounds r_0 < r_1 < ...; on GPUs one GEMM per group with the
-    backward of _GroupedLinear."""
+def _narrow_dx_applies(dx: torch.Tensor, dy: torch.Tensor, x_dtype: torch.dtype) -> bool:
+    """Whether the last group's dy W joins the cast of dx in one HIP pass: 2 to 32 columns (at 32 the pass still costs
+    less than a GEMM that reads and writes dx).  With create_graph the GEMM stays, which autograd differentiates."""
+    J, C = dy.shape[1], dx.shape[1]
+    return (dx.is_cuda and not torch.is_grad_enabled() and dx.dtype == torch.bfloat16 and dy.dtype == torch.bfloat16
+            and x_dtype in (torch.bfloat16, torch.float32) and J % 2 == 0 and 2 <= J <= 32 and C % 8 == 0)
+
+
+def _grouped_linear(x: torch.Tensor, w: torch.Tensor, bounds, dtype: torch.dtype | None = None):
+    """(x W[r_0:r_1]^T, x W[r_1:r_2]^T, ...) for row bounds r_0 < r_1 < ..., computed in ``dtype`` (x's own by default);
+    on GPUs one GEMM per group with the backward of _GroupedLinear."""
     bounds = tuple(int(r) for r in bounds)
+    dtype = x.dtype if dtype is None else dtype
     if x.is_cuda:
-        return _GroupedLinear.apply(x, w, bounds)
-    wc = w.to(x.dtype)
+        return _GroupedLinear.apply(x, w, bounds, dtype)
+    x, wc = x.to(dtype), w.to(dtype)
     return tuple(F.linear(x, wc[r0:r1]) for r0, r1 in zip(bounds[:-1], bounds[1:]))
 
 
@@ -174,11 +209,11 @@ class GatedDeltaNet(nn.Module):
         gate = [self.g_proj] if self.use_gate else []
         return [self.q_proj, self.k_proj, self.v_proj, *gate, self.a_proj, self.b_proj]
 
-    def _decode_stage_applies(self, x: torch.Tensor, convs, conv_in) -> bool:
+    def _decode_stage_applies(self, x: torch.Tensor, dtype: torch.dtype, convs, conv_in) -> bool:
         """One cached token per sequence in bf16 without grad, plain convolutions with the states they would take: the
         projections, convolutions and gates then run as one op (ops.mixer_decode_stage) instead of seven.  Anything
         else, hooks on the convolutions included, takes the separate ops."""
-        if torch.is_grad_enabled() or not x.is_cuda or x.dtype != torch.bfloat16 or x.shape[1] != 1 or not convs:
+        if torch.is_grad_enabled() or not x.is_cuda or dtype != torch.bfloat16 or x.shape[1] != 1 or not convs:
             return False
         if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
             return False
@@ -193,13 +228,14 @@ class GatedDeltaNet(nn.Module):
                 return False
         return True
 
-    def _grouped_projections(self, hidden_states: torch.Tensor):
+    def _grouped_projections(self, hidden_states: torch.Tensor, dtype: torch.dtype | None = None):
         """([q | k | v], gate or None, [a | b]): the six input linears against their concatenated weights, one GEMM
         per group."""
         n_qkv = 2 * self.key_dim + self.value_dim
         bounds = [0, n_qkv] + ([n_qkv + self.value_dim] if self.use_gate else [])
         bounds.append(bounds[-1] + self.a_proj.out_features + self.b_proj.out_features)
-        outs = _grouped_linear(hidden_states, torch.cat([m.weight for m in self._input_linears()], 0), bounds)
+        outs = _grouped_linear(hidden_states, torch.cat([m.weight for m in self._input_linears()], 0), bounds,
+                               dtype)
         return outs[0], (outs[1] if self.use_gate else None), outs[-1]
 
     def input_projections(self, hidden_states: torch.Tensor) -> tuple[torch.Tensor, ...]:
@@ -222,10 +258,11 @@ class GatedDeltaNet(nn.Module):
         B, T, _ = hidden_states.shape
         H, DK, DV = self.num_heads, self.head_k_dim, self.head_v_dim
         dev_type = hidden_states.device.type
-        if torch.is_autocast_enabled(dev_type) and hidden_states.dtype == torch.float32:
-            # the cast autocast would make in front of each projection GEMM, made once for both (and one cast of
-            # the input gradient back in the backward instead of two and their fp32 sum)
-            hidden_states = hidden_states.to(torch.get_autocast_dtype(dev_type))
+        dtype = hidden_states.dtype
+        if torch.is_autocast_enabled(dev_type) and dtype == torch.float32:
+            # the cast autocast would make in front of each projection GEMM, made once for all by _GroupedLinear (and
+            # undone in the pass that finishes the input gradient)
+            dtype = torch.get_autocast_dtype(dev_type)
         entry = None if past_key_values is None else past_key_values.get(self.layer_idx)
         conv_in = entry["conv_state"] if entry is not None else (None, None, None)
         conv_out = (None, None, None)
@@ -234,18 +271,18 @@ class GatedDeltaNet(nn.Module):
         if convs and entry is None and not use_cache and all(c.bias is None for c in convs):
             # training / prefill without a cache: the convolutions read q, k, v straight out of the projection's
             # output and their backward writes into one gradient of it (ops.mixer_input_stage)
-            y, gate, ab = self._grouped_projections(hidden_states)
+            y, gate, ab = self._grouped_projections(hidden_states, dtype)
             w = torch.cat([c.weight.squeeze(1) for c in convs], 0)
             q, k, v = ops.mixer_input_stage(y, w, self.key_dim, self.value_dim, DK)
             gp = [gate] if self.use_gate else []
-        elif self._decode_stage_applies(hidden_states, convs, conv_in):
+        elif self._decode_stage_applies(hidden_states, dtype, convs, conv_in):
             w_in = [m.weight for m in self._input_linears()]
             q, k, v, g, beta, cq, ck, cv, *gp = ops.mixer_decode_stage(
-                hidden_states, w_in, [c.weight for c in convs], list(conv_in), self.A_log, self.dt_bias, DK,
+                hidden_states.to(dtype), w_in, [c.weight for c in convs], list(conv_in), self.A_log, self.dt_bias, DK,
                 2.0 if self.allow_neg_eigval else 1.0, float("-inf"))
             conv_out, gates_done = (cq, ck, cv), True
         else:
-            q, k, v, a, b, *gp = self.input_projections(hidden_states)
+            q, k, v, a, b, *gp = self.input_projections(hidden_states.to(dtype))
             if convs:
                 (q, cq), (k, ck), (v, cv) = (self.q_conv1d(q, conv_in[0]), self.k_conv1d(k, conv_in[1]),
                                              self.v_conv1d(v, conv_in[2]))

@@ -78,13 +78,13 @@ class NStepGDN(nn.Module):
         n_qkv = 2 * self.qk_dim + self.v_dim
         n_main = n_qkv + self.n_gate
         dev_type = x.device.type
-        xp = x
-        if torch.is_autocast_enabled(dev_type) and x.dtype == torch.float32:
-            xp = x.to(torch.get_autocast_dtype(dev_type))  # autocast's cast, made once for both GEMMs below
+        dtype = x.dtype
+        if torch.is_autocast_enabled(dev_type) and dtype == torch.float32:
+            dtype = torch.get_autocast_dtype(dev_type)  # autocast's cast, made once for the GEMMs below
         # in_proj's rows [q k v], [gate] and [a b] as one GEMM each (the first a multiple of 256 wide at the
         # reference shapes); the rows past them pad the projection and are not computed (their gradient is zero)
         bounds = [0, n_qkv] + ([n_main] if self.n_gate else []) + [n_main + 2 * H]
-        y, *g, ab = _grouped_linear(xp, self.in_proj.weight, bounds)
+        y, *g, ab = _grouped_linear(x, self.in_proj.weight, bounds, dtype)
         g = g[0] if g else None
         # the exact token scan takes fp32 q and k normalised after the conv, as the reference normalises the fp32
         # copies of the conv output (nsgdn.py:525-528); the chunk path gets them normalised inside the conv
@@ -113,12 +113,12 @@ class NStepGDN(nn.Module):
             u = ops.write_direction(kf, beta, lam, self.n_steps)
             y = ops.nsgdn_scan(qf, kf, u, v.float(), la)
             y = ops.gated_rmsnorm(y, None if gate is None else gate.float(), self.norm.weight, eps)
-            return _linear(y.reshape(B, T, -1).to(xp.dtype), self.o_proj.weight)
+            return _linear(y.reshape(B, T, -1).to(dtype), self.o_proj.weight)
         # u from k, the previous token's k and beta in one HIP pass (fp32 arithmetic, written in k's dtype, which
         # the scan takes u in)
         u = ops.write_direction(k, beta, lam, self.n_steps)
         y = ops.nsgdn_scan_chunk(q, k, u, v, la, scale=DK ** -0.5)
-        y = ops.gated_rmsnorm(y.to(xp.dtype), gate, self.norm.weight, eps)
+        y = ops.gated_rmsnorm(y.to(dtype), gate, self.norm.weight, eps)
         return _linear(y.reshape(B, T, -1), self.o_proj.weight)
 
 

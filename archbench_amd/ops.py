@@ -1266,6 +1266,48 @@ def _(parts, out):
     return None
 
 
+@torch.library.custom_op("archbench_amd::sum_parts_t_", mutates_args=("out",))
+def sum_parts_t_(parts: Tensor, out: Tensor) -> None:
+    """out [N, K] (contiguous, bf16 or fp32) <- the sum over parts [S, K, N] (fp32, contiguous), transposed; N and K
+    multiples of 4."""
+    _require_gpu(parts, out)
+    if parts.dtype != torch.float32 or parts.dim() != 3 or (parts.shape[2], parts.shape[1]) != tuple(out.shape) or not (
+            parts.is_contiguous() and out.is_contiguous()):
+        raise ValueError(f"parts must be contiguous fp32 [S, K, N], got {parts.dtype} {tuple(parts.shape)} for out "
+                         f"{tuple(out.shape)}")
+    rc = _lib.load().gdn_sum_parts_t(_lib.ptr(parts), parts.shape[0], _lib.ptr(out), out.shape[0], out.shape[1],
+                                     _lib.dtype_code(out.dtype), _lib.stream_ptr(out.device))
+    _lib.check(rc, "gdn_sum_parts_t")
+
+
+@sum_parts_t_.register_fake
+def _(parts, out):
+    return None
+
+
+@torch.library.custom_op("archbench_amd::narrow_dx", mutates_args=())
+def narrow_dx(dx: Tensor, a: Tensor, w: Tensor, fp32: bool) -> Tensor:
+    """dx [M, C] + a [M, J] w [J, C] (bf16, fp32 sums) as a new tensor, bf16 or (``fp32``) fp32; J even, at most 32, C a
+    multiple of 8."""
+    _require_gpu(dx, a, w)
+    M, C = dx.shape
+    J = a.shape[1]
+    if a.shape[0] != M or w.shape != (J, C) or C % 8 or any(t.dtype != torch.bfloat16 for t in (dx, a, w)):
+        raise ValueError(f"narrow_dx takes bf16 dx [M, C], a [M, J], w [J, C], C a multiple of 8, got {tuple(dx.shape)}, "
+                         f"{tuple(a.shape)}, {tuple(w.shape)}")
+    dx, a, w = _arg(dx), _arg(a), _arg(w)
+    out = torch.empty(M, C, dtype=torch.float32 if fp32 else torch.bfloat16, device=dx.device)
+    rc = _lib.load().gdn_narrow_dx(_lib.ptr(dx), _lib.ptr(a), _lib.ptr(w), _lib.ptr(out), M, C, J,
+                                   _lib.dtype_code(out.dtype), _lib.stream_ptr(dx.device))
+    _lib.check(rc, "gdn_narrow_dx")
+    return out
+
+
+@narrow_dx.register_fake
+def _(dx, a, w, fp32):
+    return dx.new_empty(dx.shape, dtype=torch.float32 if fp32 else torch.bfloat16)
+
+
 # ------------------------------------------------------------------------------------------------- decode step
 @torch.library.custom_op("archbench_amd::gdn_recurrent_step", mutates_args=("state",))
 def _recurrent_step(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, state: Tensor,

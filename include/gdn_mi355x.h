@@ -248,6 +248,12 @@ int gdn_cross_entropy_fwd_bwd(void* logits, const int64_t* target, float* loss, 
  * and out = sum over p < nparts of part[p * n + i] (fp32, p ascending), rounded once to dtype (n a multiple of 8). */
 int gdn_scale(const void* x, const float* s, void* y, int64_t n, int dtype, void* stream);
 int gdn_sum_parts(const float* part, int nparts, void* out, int64_t n, int dtype, void* stream);
+/* The same for parts [K, N] written transposed, out [N, K]; N and K multiples of 4. */
+int gdn_sum_parts_t(const float* part, int nparts, void* out, int N, int K, int dtype, void* stream);
+/* out [M, C] (out_dtype) = dx [M, C] + a [M, J] w [J, C]: bf16 operands, fp32 sums; J even and at most 32, C a multiple
+ * of 4. */
+int gdn_narrow_dx(const void* dx, const void* a, const void* w, void* out, int64_t M, int C, int J, int out_dtype,
+                  void* stream);
 
 /* Write direction of the n-step family: per token row of K channels (one head of one token), with p the previous
  * token's key in the same sequence (zero at t = 0),

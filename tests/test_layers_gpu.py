@@ -455,3 +455,30 @@ def test_decode_stage_route_equals_separate_ops():
          [c.weight.detach() for c in (m.layer.q_conv1d, m.layer.k_conv1d, m.layer.v_conv1d)],
          [c.clone() for c in cache[0]["conv_state"]], m.layer.A_log.detach(), m.layer.dt_bias.detach(),
          m.layer.head_k_dim, 1.0, float("-inf")), test_utils=("test_schema", "test_faketensor"))
+
+
+@pytest.mark.parametrize("S,N,K,dtype", [(1, 4, 4, torch.float32), (8, 132, 68, torch.float32), (16, 64, 200, torch.bfloat16),
+                                         (11, 2048, 512, torch.float32)])
+def test_sum_parts_transposed(S, N, K, dtype):
+    """The transposed sum of parts at whole and partial 64 x 64 tiles, with part counts around the eight in flight.
+    Bound: S - 1 fp32 additions (2^-24 each of a partial sum), and one rounding to the output's dtype (2^-9 in bf16)."""
+    banner(f"sum of parts, transposed S={S} N={N} K={K} {dtype}")
+    parts = torch.randn(S, K, N, device="cuda", generator=torch.Generator("cuda").manual_seed(S))
+    out = torch.empty(N, K, device="cuda", dtype=dtype)
+    ops.sum_parts_t_(parts, out)
+    ref = parts.double().sum(0).t()
+    assert rel_l2(out.double(), ref) <= (1e-6 if dtype == torch.float32 else 4e-3)
+
+
+@pytest.mark.parametrize("M,C,J,fp32", [(1, 8, 2, True), (33, 264, 8, True), (100, 512, 16, False), (1000, 768, 12, True),
+                                        (65, 1024, 32, True)])
+def test_narrow_dx(M, C, J, fp32):
+    """dx + a W for a few columns: rows and columns that do not fill a wave's, J below and at each compiled width.  Bound:
+    J + 1 fp32 additions and, in bf16, one rounding."""
+    banner(f"narrow dx M={M} C={C} J={J} fp32={fp32}")
+    gen = torch.Generator("cuda").manual_seed(M)
+    dx, a, w = (torch.randn(*s, device="cuda", generator=gen).bfloat16() for s in ((M, C), (M, J), (J, C)))
+    out = ops.narrow_dx(dx, a, w, fp32)
+    ref = dx.double() + a.double() @ w.double()
+    assert out.dtype == (torch.float32 if fp32 else torch.bfloat16)
+    assert rel_l2(out.double(), ref) <= (1e-6 if fp32 else 4e-3)
