@@ -1,0 +1,75 @@
+"""Registration of the package's functional GPU ops (no argument mutated, tensors and not lists of them returned).
+
+``gpu_op`` registers what ``torch.library.custom_op`` would -- a schema inferred from the signature, one implementation
+for every device, a fake kernel, an autograd kernel -- on the dispatcher directly, and returns a callable with the same
+``register_fake`` and ``register_autograd``.  Tracing, fake tensors, dispatch modes, functorch transforms and saved-tensor
+hooks therefore see the ops as before; what is left out is Python work per call (schema-driven flattening of the
+arguments, the search for outputs that alias inputs, which these ops never return).  One op with five arguments costs
+14.5 us instead of 26 in a forward that records a gradient, 48 instead of 72 with its backward, 8 instead of 11 without
+a gradient (the op itself empty); a layer of a small model is bound by these calls, not by its kernels."""
+
+from __future__ import annotations
+
+import functools
+
+import torch
+from torch import Tensor
+
+_BelowAutograd = torch._C._AutoDispatchBelowAutograd
+_libs: dict[str, torch.library.Library] = {}  # owner of each op's registrations (dropped when an op is defined again)
+
+
+def _autograd_kernel(op, name: str, backward, setup_context):
+    def forward(ctx, *args):
+        with _BelowAutograd():
+            out = op(*args)
+        if setup_context is not None:
+            setup_context(ctx, args, out)
+        return out
+
+    def no_formula(ctx, *grads):
+        raise RuntimeError(f"Trying to backward through {op} but no autograd formula was registered.")
+
+    fn = type(f"GeneratedBackwardFor_{name.replace('::', '_')}", (torch.autograd.Function,),
+              {"forward": staticmethod(forward), "backward": staticmethod(backward or no_formula)})
+
+    def kernel(*args):
+        if torch.is_grad_enabled():
+            for a in args:
+                if isinstance(a, Tensor) and a.requires_grad:
+                    return fn.apply(*args)
+        with _BelowAutograd():
+            return op(*args)
+
+    return kernel
+
+
+def gpu_op(name: str):
+    """Decorator: registers the function as the op ``name`` ("namespace::op")."""
+    ns, opname = name.split("::")
+
+    def wrap(impl):
+        _libs.pop(name, None)
+        lib = _libs[name] = torch.library.Library(ns, "FRAGMENT")
+        lib.define(opname + torch.library.infer_schema(impl, mutates_args=()), tags=(torch.Tag.pt2_compliant_tag,))
+        # not traced into where a compiled program calls the op between two graphs
+        lib.impl(opname, torch._disable_dynamo(impl), "CompositeExplicitAutograd")
+        op = getattr(getattr(torch.ops, ns), opname).default
+        kernel = [_autograd_kernel(op, name, None, None)]  # replaced once a formula is registered
+        lib.impl(opname, lambda *args: kernel[0](*args), "Autograd")
+
+        @functools.wraps(impl)
+        def call(*args, **kwargs):
+            return op(*args, **kwargs)
+
+        def register_fake(fn):
+            torch.library.register_fake(name, fn, lib=lib)
+            return fn
+
+        def register_autograd(backward, /, *, setup_context=None):
+            kernel[0] = _autograd_kernel(op, name, backward, setup_context)
+
+        call.register_fake, call.register_autograd, call._opoverload = register_fake, register_autograd, op
+        return call
+
+    return wrap

@@ -41,6 +41,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from ._op import gpu_op
 
 __all__ = ["chunk_gated_delta_rule", "fused_recurrent_gated_delta_rule", "recurrent_step", "chunk_fwd",
            "chunk_bwd", "chunk_fwd_stash", "chunk_bwd_stashed", "nsgdn_scan", "nsgdn_scan_chunk", "short_conv", "mixer_input_stage", "write_direction",
@@ -113,7 +114,7 @@ def _shapes(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, h0: Option
 
 
 # ------------------------------------------------------------------------------------------------ chunk forward
-@torch.library.custom_op("archbench_amd::gdn_chunk_fwd", mutates_args=())
+@gpu_op("archbench_amd::gdn_chunk_fwd")
 def chunk_fwd(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, h0: Optional[Tensor],
               scale: float) -> tuple[Tensor, Tensor]:
     _require_gpu(q, k, v, g, beta, h0)
@@ -140,7 +141,7 @@ def _(q, k, v, g, beta, h0, scale):
 
 
 # ----------------------------------------------------------------------------------------------- chunk backward
-@torch.library.custom_op("archbench_amd::gdn_chunk_bwd", mutates_args=())
+@gpu_op("archbench_amd::gdn_chunk_bwd")
 def chunk_bwd(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, h0: Optional[Tensor], do: Tensor,
               dhT: Optional[Tensor], scale: float) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     _require_gpu(q, k, v, g, beta, h0, do, dhT)
@@ -204,7 +205,7 @@ def _prep(q, k, v, g, beta, h0):
             _arg(h0, torch.float32))
 
 
-@torch.library.custom_op("archbench_amd::gdn_chunk_fwd_stash", mutates_args=())
+@gpu_op("archbench_amd::gdn_chunk_fwd_stash")
 def chunk_fwd_stash(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, h0: Optional[Tensor],
                     scale: float) -> tuple[Tensor, Tensor, Tensor]:
     _require_gpu(q, k, v, g, beta, h0)
@@ -230,7 +231,7 @@ def _(q, k, v, g, beta, h0, scale):
             q.new_empty(n, dtype=torch.uint8))
 
 
-@torch.library.custom_op("archbench_amd::gdn_chunk_bwd_stashed", mutates_args=())
+@gpu_op("archbench_amd::gdn_chunk_bwd_stashed")
 def chunk_bwd_stashed(q: Tensor, k: Tensor, v: Tensor, g: Tensor, beta: Tensor, h0: Optional[Tensor], do: Tensor,
                       dhT: Optional[Tensor], stash: Tensor,
                       scale: float) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -304,7 +305,7 @@ def _nsgdn_shapes(q, k, u, v, la, h0):
     return _shapes(q, k, v, la, la, h0)
 
 
-@torch.library.custom_op("archbench_amd::nsgdn_chunk_fwd", mutates_args=())
+@gpu_op("archbench_amd::nsgdn_chunk_fwd")
 def nsgdn_chunk_fwd(q: Tensor, k: Tensor, u: Tensor, v: Tensor, la: Tensor, h0: Optional[Tensor],
                     scale: float) -> tuple[Tensor, Tensor, Tensor]:
     """(y, hT, stash)."""
@@ -331,7 +332,7 @@ def _(q, k, u, v, la, h0, scale):
             q.new_empty(n, dtype=torch.uint8))
 
 
-@torch.library.custom_op("archbench_amd::nsgdn_chunk_bwd", mutates_args=())
+@gpu_op("archbench_amd::nsgdn_chunk_bwd")
 def nsgdn_chunk_bwd(q: Tensor, k: Tensor, u: Tensor, v: Tensor, la: Tensor, h0: Optional[Tensor], dy: Tensor,
                     dhT: Optional[Tensor], stash: Tensor,
                     scale: float) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -386,7 +387,7 @@ nsgdn_chunk_fwd.register_autograd(_nsgdn_backward, setup_context=_nsgdn_setup)
 
 # The n-step family's write direction (nsgdn.py:61-75 with the shift of k at :535): u from k (p = the previous
 # token's key of the same sequence), beta and the effective lam, one HIP pass each way (gdn_writedir.hip).
-@torch.library.custom_op("archbench_amd::write_direction", mutates_args=())
+@gpu_op("archbench_amd::write_direction")
 def write_direction(k: Tensor, beta: Tensor, lam: Tensor, n_steps: int) -> Tensor:
     """u [B,T,H,K] in k's dtype: u_1 = beta k, u_{i+1} = u_i - lam beta (p . u_i) (p - (p . k) k), p = k[:, t-1]
     (zero at t = 0).  n_steps <= 1 is u = beta k, as in the reference; any number of steps."""
@@ -416,7 +417,7 @@ def _(k, beta, lam, n_steps):
     return torch.empty_like(k)
 
 
-@torch.library.custom_op("archbench_amd::write_direction_bwd", mutates_args=())
+@gpu_op("archbench_amd::write_direction_bwd")
 def write_direction_bwd(k: Tensor, beta: Tensor, lam: Tensor, du: Tensor,
                         n_steps: int) -> tuple[Tensor, Tensor, Tensor]:
     """(dk in k's dtype, dbeta [B,T,H] fp32, dlam [H] fp32)."""
@@ -502,7 +503,7 @@ def _sum_rows(p: Tensor) -> Tensor:
     return out
 
 
-@torch.library.custom_op("archbench_amd::nsgdn_token_fwd", mutates_args=())
+@gpu_op("archbench_amd::nsgdn_token_fwd")
 def nsgdn_token_fwd(q: Tensor, k: Tensor, u: Tensor, v: Tensor, la: Tensor, h0: Optional[Tensor],
                     output_final_state: bool) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """(y, r, st, hT), fp32: the scan's output, its residuals r = v - (e^la S) k, the state checkpoints and the
@@ -538,7 +539,7 @@ def _(q, k, u, v, la, h0, output_final_state):
             v.new_empty((B, H, K, V) if output_final_state else (0,), **f32))
 
 
-@torch.library.custom_op("archbench_amd::nsgdn_token_bwd", mutates_args=())
+@gpu_op("archbench_amd::nsgdn_token_bwd")
 def nsgdn_token_bwd(q: Tensor, k: Tensor, u: Tensor, la: Tensor, r: Tensor, st: Tensor, dy: Tensor,
                     dhT: Optional[Tensor], need_dh0: bool) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
     """(dq, dk, du, dv, dla, dh0), fp32; dh0 [B, H, K, V] when need_dh0, else empty.  dhT: the final state's
@@ -642,7 +643,7 @@ def _conv_shapes(x: Tensor, w: Tensor, bias: Optional[Tensor], state: Optional[T
     return B, T, D, W
 
 
-@torch.library.custom_op("archbench_amd::short_conv", mutates_args=())
+@gpu_op("archbench_amd::short_conv")
 def short_conv(x: Tensor, w: Tensor, bias: Optional[Tensor], state: Optional[Tensor],
                norm_group: int) -> tuple[Tensor, Tensor]:
     """(y [B,T,D], new_state [B,D,W-1]): y = silu(causal depthwise conv(x)) (+ L2 norm per norm_group channels)."""
@@ -666,7 +667,7 @@ def _(x, w, bias, state, norm_group):
     return x.new_empty(B, T, D), x.new_empty(B, D, w.shape[1] - 1)
 
 
-@torch.library.custom_op("archbench_amd::short_conv_bwd", mutates_args=())
+@gpu_op("archbench_amd::short_conv_bwd")
 def short_conv_bwd(x: Tensor, w: Tensor, bias: Optional[Tensor], state: Optional[Tensor], dy: Tensor,
                    norm_group: int) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """(dx, dw [D,W] fp32, dbias [D] fp32, dstate [B,D,W-1]); dbias / dstate are zeros-shaped if not needed."""
@@ -822,7 +823,7 @@ def _stage_dims(y: Tensor, w: Tensor, key_dim: int, value_dim: int):
     return y.shape[0], y.shape[1], n, w.shape[1]
 
 
-@torch.library.custom_op("archbench_amd::mixer_input_stage", mutates_args=())
+@gpu_op("archbench_amd::mixer_input_stage")
 def mixer_input_stage(y: Tensor, w: Tensor, key_dim: int, value_dim: int,
                       norm_group: int) -> tuple[Tensor, Tensor, Tensor]:
     """(q, k, v): silu(causal conv(.)) of y's q, k and v columns (q and k L2-normalised per norm_group channels;
@@ -844,7 +845,7 @@ def _(y, w, key_dim, value_dim, norm_group):
     return y.new_empty(B, T, key_dim), y.new_empty(B, T, key_dim), y.new_empty(B, T, value_dim)
 
 
-@torch.library.custom_op("archbench_amd::mixer_input_stage_bwd", mutates_args=())
+@gpu_op("archbench_amd::mixer_input_stage_bwd")
 def mixer_input_stage_bwd(y: Tensor, w: Tensor, dq: Tensor, dk: Tensor, dv: Tensor, key_dim: int, value_dim: int,
                           norm_group: int) -> tuple[Tensor, Tensor]:
     """(dy, dw): the three conv backwards written into dy's column slices and dw's row slices (dw fp32)."""
@@ -900,7 +901,7 @@ def _norm_rows(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor]):
     return x.numel() // dim, dim
 
 
-@torch.library.custom_op("archbench_amd::gated_rmsnorm", mutates_args=())
+@gpu_op("archbench_amd::gated_rmsnorm")
 def gated_rmsnorm(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], eps: float) -> Tensor:
     _require_gpu(x, gate, weight)
     rows, dim = _norm_rows(x, gate, weight)
@@ -919,7 +920,7 @@ def _(x, gate, weight, eps):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("archbench_amd::gated_rmsnorm_bwd", mutates_args=())
+@gpu_op("archbench_amd::gated_rmsnorm_bwd")
 def gated_rmsnorm_bwd(x: Tensor, gate: Optional[Tensor], weight: Optional[Tensor], dy: Tensor,
                       eps: float) -> tuple[Tensor, Tensor, Tensor]:
     """(dx, dgate (zeros-shaped [0] without a gate), dweight [dim] fp32)."""
@@ -966,7 +967,7 @@ gated_rmsnorm.register_autograd(_norm_backward, setup_context=_norm_setup)
 # ---------------------------------------------------------------------------------------------------- L2 norm
 # y = scale * x / max(||x||, eps) over the last dimension: the per-head q / k normalisation (nsgdn.py:527-528,
 # F.normalize(.) * DK^-1/2) where it is not fused into the short convolution.
-@torch.library.custom_op("archbench_amd::l2norm", mutates_args=())
+@gpu_op("archbench_amd::l2norm")
 def l2norm(x: Tensor, eps: float, scale: float) -> Tensor:
     _require_gpu(x)
     rows, dim = _norm_rows(x, None, None)
@@ -984,7 +985,7 @@ def _(x, eps, scale):
     return torch.empty_like(x)
 
 
-@torch.library.custom_op("archbench_amd::l2norm_bwd", mutates_args=())
+@gpu_op("archbench_amd::l2norm_bwd")
 def l2norm_bwd(x: Tensor, dy: Tensor, eps: float, scale: float) -> Tensor:
     _require_gpu(x, dy)
     rows, dim = _norm_rows(x, None, None)
@@ -1031,7 +1032,7 @@ def _gate_shapes(a: Tensor, b: Tensor, A_log: Tensor, dt_bias: Optional[Tensor],
     return a.numel() // H, H
 
 
-@torch.library.custom_op("archbench_amd::gdn_gates", mutates_args=())
+@gpu_op("archbench_amd::gdn_gates")
 def gdn_gates(a: Tensor, b: Tensor, A_log: Tensor, dt_bias: Optional[Tensor], b_bias: Optional[Tensor],
               beta_scale: float, g_min: float) -> tuple[Tensor, Tensor]:
     """(g, beta), fp32, shaped like a."""
@@ -1054,7 +1055,7 @@ def _(a, b, A_log, dt_bias, b_bias, beta_scale, g_min):
     return a.new_empty(a.shape, dtype=torch.float32), a.new_empty(a.shape, dtype=torch.float32)
 
 
-@torch.library.custom_op("archbench_amd::gdn_gates_bwd", mutates_args=())
+@gpu_op("archbench_amd::gdn_gates_bwd")
 def gdn_gates_bwd(a: Tensor, b: Tensor, A_log: Tensor, dt_bias: Optional[Tensor], b_bias: Optional[Tensor],
                   dg: Tensor, dbeta: Tensor, beta_scale: float,
                   g_min: float) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -1114,7 +1115,7 @@ def _half_ptr(t: Tensor, H: int):
     return ctypes.c_void_p(t.data_ptr() + H * t.element_size())
 
 
-@torch.library.custom_op("archbench_amd::gdn_gates_ab", mutates_args=())
+@gpu_op("archbench_amd::gdn_gates_ab")
 def gdn_gates_ab(ab: Tensor, A_log: Tensor, dt_bias: Optional[Tensor], b_bias: Optional[Tensor], beta_scale: float,
                  g_min: float) -> tuple[Tensor, Tensor]:
     """(g, beta), fp32 [..., H], from ab [..., 2H] = [a | b]."""
@@ -1140,7 +1141,7 @@ def _(ab, A_log, dt_bias, b_bias, beta_scale, g_min):
     return ab.new_empty(shape, dtype=torch.float32), ab.new_empty(shape, dtype=torch.float32)
 
 
-@torch.library.custom_op("archbench_amd::gdn_gates_ab_bwd", mutates_args=())
+@gpu_op("archbench_amd::gdn_gates_ab_bwd")
 def gdn_gates_ab_bwd(ab: Tensor, A_log: Tensor, dt_bias: Optional[Tensor], b_bias: Optional[Tensor], dg: Tensor,
                      dbeta: Tensor, beta_scale: float, g_min: float) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """(d ab [..., 2H] in ab's dtype, dA_log, ddt_bias, db_bias fp32)."""
@@ -1217,7 +1218,7 @@ def _(logits, target, dloss, ignore_index):
     return logits.new_empty(N, dtype=torch.float32), logits.new_empty(N, dtype=torch.float32)
 
 
-@torch.library.custom_op("archbench_amd::scaled", mutates_args=())
+@gpu_op("archbench_amd::scaled")
 def scaled(x: Tensor, s: Tensor) -> Tensor:
     """s x for a device scalar s (one element), in x's dtype with the product in fp32."""
     _require_gpu(x, s)
@@ -1285,7 +1286,7 @@ def _(parts, out):
     return None
 
 
-@torch.library.custom_op("archbench_amd::narrow_dx", mutates_args=())
+@gpu_op("archbench_amd::narrow_dx")
 def narrow_dx(dx: Tensor, a: Tensor, w: Tensor, fp32: bool) -> Tensor:
     """dx [M, C] + a [M, J] w [J, C] (bf16, fp32 sums) as a new tensor, bf16 or (``fp32``) fp32; J even, at most 32, C a
     multiple of 8."""
