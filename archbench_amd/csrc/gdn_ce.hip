@@ -135,22 +135,40 @@ __global__ __launch_bounds__(256) void scale_kernel(const T* __restrict__ x, con
   }
 }
 
-// out = sum over p of part[p], p ascending, rounded once to T: the fp32 partial products of a GEMM split over its
-// contraction.  n a multiple of 8.
+// out = sum over p of part[p], in 64 bits, rounded once to T: the fp32 partial products of a GEMM split over its
+// contraction, or a scan's partial rows (added in fp32, sixteen of them cost dq 4% more error against 64 bits than four
+// did; the pass is bound by its reads either way).  n a multiple of 8.
 template <typename T>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ part, int nparts, T* __restrict__ out,
                                                         int64_t n) {
   const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
   if (i >= n) return;
-  float a[8] = {};
-  for (int p = 0; p < nparts; ++p) {
+  double s[8] = {};
+  constexpr int PF = 4;  // parts in flight
+  int p = 0;
+  for (; p + PF <= nparts; p += PF) {
+    Row8<float> r[PF];
+#pragma unroll
+    for (int f = 0; f < PF; ++f) r[f].load(part + (int64_t)(p + f) * n + i);
+#pragma unroll
+    for (int f = 0; f < PF; ++f) {
+      float v[8];
+      r[f].get(v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] += v[e];
+    }
+  }
+  for (; p < nparts; ++p) {
     Row8<float> r;
     r.load(part + (int64_t)p * n + i);
     float v[8];
     r.get(v);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) a[e] += v[e];
+    for (int e = 0; e < 8; ++e) s[e] += v[e];
   }
+  float a[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) a[e] = static_cast<float>(s[e]);
   store_row8(out + i, a);
 }
 

@@ -20,12 +20,17 @@
 // Sums over rows are formed over a lane's own rows, then a reduce-scatter over the wave's four row groups (lane swaps,
 // no LDS crossbar), then over the waves through LDS (a fixed order, no atomics), then over a head's workgroups through
 // partial rows that are added afterwards.
-// Bound: the forward by that chain (per token at K = 128 about 0.24 us: two dot products and row sums, the update and
-// the reads between them) until a SIMD holds two waves or more, the backward by its arithmetic (its row sums over
-// the state's rows included) at one or two waves per SIMD.  Against eight lanes per row with the token's loads, stores,
-// expf and LDS row sums in the chain: B4 T1024 H4 K128 V256 forward 507 -> 241 us, backward 1916 -> 908 us.
+// Only G needs the tokens in reverse order one by one: S restarts from any checkpoint.  With few sequences the backward
+// is therefore split (ts_bwd_plan): token_scan_gstate_kernel runs G's recurrence alone, at the forward's pace, leaving dv
+// and G at every chunk's end, and the rest runs with the chunks in parallel.
+// Bound: the forward and G's recurrence by the chain (per token at K = 128 about 0.24 and 0.21 us: a dot product and its
+// row sum, the update and the reads between them) until a SIMD holds two waves or more, the rest of the backward by its
+// arithmetic (its row sums over the state's rows included, about 330 instructions per token and wave) at two waves per
+// SIMD, a 64-row chunk of 32 tokens in 57 us.  B4 T1024 H4 K128 V256: forward 507 -> 235 us (eight lanes per row with the
+// token's loads, stores, expf and LDS row sums in the chain before), backward 1916 -> 908 (as one chain) -> 216 + 459 us.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -350,25 +355,23 @@ struct TokSums {
 // accumulated), and walked backward.  A short last group is padded with identity tokens (la = 0, zero vectors and
 // row values), which change neither S nor G, and whose sums are not stored.  The forward pass has the chunk's u in LDS
 // at once; the groups' vectors are staged (and their row values loaded) a group ahead: one barrier per group.
-template <int K, typename SH>
+// SPLIT: G at each chunk's end (gst, [BH][NCH][K][V]) and dv come from token_scan_gstate_kernel, so that the chunks are
+// independent: nitems = BH NCH NB (bh, chunk, row block) items, walked by the grid's workgroups (scratch per workgroup).
+// Otherwise a workgroup is a (bh, row block) and carries G through its chunks, computing dv and dh0.
+template <int K, typename SH, bool SPLIT>
 __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))) void token_scan_bwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ u, const float* __restrict__ la,
     const float* __restrict__ r, const float* __restrict__ st, const float* __restrict__ gy,
     const float* __restrict__ dhT, float* __restrict__ gv, float* __restrict__ gqp, float* __restrict__ gup,
-    float* __restrict__ gkp, float* __restrict__ glap, float* __restrict__ dh0, float* __restrict__ sc, int T_, int H,
-    int V, int NCH, int NB, int64_t ntok) {
+    float* __restrict__ gkp, float* __restrict__ glap, float* __restrict__ dh0, float* __restrict__ sc,
+    const float* __restrict__ gst, int nitems, int T_, int H, int V, int NCH, int NB, int64_t ntok) {
   using TS = TokStage<K>;
   constexpr int KQ = TS::KQ, RL = SH::RL, THREADS = SH::THREADS, NGS = TS_CT / TS_GS;
   constexpr int NL = (TS_GS * TS::PER + THREADS - 1) / THREADS;
   __shared__ __attribute__((aligned(16))) float sv[2][TS_GS][TS::SIZE];
   __shared__ __attribute__((aligned(16))) TokSums<K, SH> sums;
   const int tid = threadIdx.x, l = lane_id(), p = l & 15;
-  const int pid = blockIdx.x, bh = pid / NB, vb = pid - bh * NB;
-  const int b = bh / H, h = bh - b * H;
-  const int v0 = vb * SH::ROWS + wave_id() * SH::WROWS + (l >> 4) * RL;  // this lane's rows, as in the forward
-  // uniform bases and 32-bit lane offsets: per-lane 64-bit addresses of the unrolled accesses would fill the registers
-  const float* stb = st + (int64_t)bh * NCH * K * V;
-  const int64_t st_off = (int64_t)p * KQ * V + v0;
+  const int pid = blockIdx.x;
   constexpr int SV = RL * KQ / 4;  // 16-byte pieces of this lane's state
   f32x4* scw = reinterpret_cast<f32x4*>(sc + (int64_t)pid * NGS * RL * KQ * THREADS);
   const unsigned sc_off = (unsigned)tid * SV;
@@ -388,14 +391,13 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))
       for (int e = 0; e < 4; ++e) X[i][j + e] = t[e];
     }
   };
-  float* const gout[3] = {gqp + (int64_t)vb * ntok * K, gup + (int64_t)vb * ntok * K, gkp + (int64_t)vb * ntok * K};
-  float* gl_b = glap + (int64_t)vb * ntok;
   f32x4 xr[NL];  // this thread's pieces of the next group's vectors (piece e: token e / PER), loaded a group ahead
   // The group's row scalars, one token per lane: lane p holds r of token p & 3 and row p >> 2 for p < 4 RL, dy likewise
   // for the next 4 RL lanes; and la of token l & 3
-  const int ti = p & 3, si = p >> 2, srow = v0 + (RL == 2 ? si & 1 : 0);
+  const int ti = p & 3, si = p >> 2, srow_off = RL == 2 ? si & 1 : 0;
   const float* sp = (RL == 2 ? si >= 2 : (si & 1)) ? gy : r;
-  float xn, ln, xc, ac;
+  float xn, ln, xc, ac, dn = 0.f, dc = 0.f;  // dn, dc (SPLIT): dv of token p & 3, row p >> 2, for p < 4 RL
+  int v0 = 0, srow = 0;
   auto load_grp = [&](auto&& tok_at) {  // tok_at(i): token i of the group (< 0: an identity token)
 #pragma unroll
     for (int m = 0; m < NL; ++m) {
@@ -409,6 +411,7 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))
     const int64_t tk = tok_at(ti);
     xn = tk >= 0 && srow < V ? sp[tk * V + srow] : 0.f;
     ln = tk >= 0 ? la[tk] : 0.f;
+    if constexpr (SPLIT) dn = tk >= 0 && p < 4 * RL && srow < V ? gv[tk * V + srow] : 0.f;
   };
   auto stage_grp = [&](int buf) {
 #pragma unroll
@@ -418,15 +421,42 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))
     }
     xc = xn;
     ac = expf(ln);
+    dc = dn;
   };
   int par = 0;  // parity of the group: sv[par & 1] holds its vectors, sums[par & 1] takes its row sums
-  const int64_t cb = (int64_t)bh * K * V + (int64_t)p * KQ * V + v0;  // [B, H, K, V] states, as in the forward
   float G[RL][KQ], S[RL][KQ];
+  if constexpr (!SPLIT) {
+    const int bh = pid / NB;
+    v0 = (pid - bh * NB) * SH::ROWS + wave_id() * SH::WROWS + (l >> 4) * RL;  // this lane's rows, as in the forward
+    srow = v0 + srow_off;
+    const int64_t cb = (int64_t)bh * K * V + (int64_t)p * KQ * V + v0;  // [B, H, K, V] states, as in the forward
 #pragma unroll
-  for (int i = 0; i < RL; ++i)
+    for (int i = 0; i < RL; ++i)
 #pragma unroll
-    for (int j = 0; j < KQ; ++j) G[i][j] = dhT && v0 + i < V ? dhT[cb + (int64_t)j * V + i] : 0.f;
-  for (int c = NCH - 1; c >= 0; --c) {
+      for (int j = 0; j < KQ; ++j) G[i][j] = dhT && v0 + i < V ? dhT[cb + (int64_t)j * V + i] : 0.f;
+  }
+  for (int it = SPLIT ? pid : NCH - 1; SPLIT ? it < nitems : it >= 0; it += SPLIT ? (int)gridDim.x : -1) {
+    // uniform, and said so: the divisions leave their results in vector registers
+    const int bc = SPLIT ? __builtin_amdgcn_readfirstlane(it / NB) : 0;  // (bh, chunk)
+    const int bh = SPLIT ? __builtin_amdgcn_readfirstlane(bc / NCH) : pid / NB, c = SPLIT ? bc - bh * NCH : it;
+    const int vb = SPLIT ? it - bc * NB : pid - bh * NB;
+    const int b = bh / H, h = bh - b * H;
+    if constexpr (SPLIT) {
+      v0 = vb * SH::ROWS + wave_id() * SH::WROWS + (l >> 4) * RL;
+      srow = v0 + srow_off;
+    }
+    // uniform bases and 32-bit lane offsets: per-lane 64-bit addresses of the unrolled accesses would fill the registers
+    const float* stb = st + (int64_t)bh * NCH * K * V;
+    const int64_t st_off = (int64_t)p * KQ * V + v0;
+    float* const gout[3] = {gqp + (int64_t)vb * ntok * K, gup + (int64_t)vb * ntok * K, gkp + (int64_t)vb * ntok * K};
+    float* gl_b = glap + (int64_t)vb * ntok;
+    if constexpr (SPLIT) {
+      const float* g0 = gst + ((int64_t)bh * NCH + c) * K * V;
+#pragma unroll
+      for (int i = 0; i < RL; ++i)
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) G[i][j] = v0 + i < V ? g0[(int64_t)j * V + (st_off + i)] : 0.f;
+    }
     const int n = min(TS_CT, T_ - c * TS_CT), ng = (n + TS_GS - 1) / TS_GS;
     const int64_t tok0 = ((int64_t)b * T_ + (int64_t)c * TS_CT) * H + h;
     auto tok_in = [&](int g, int i) -> int64_t {
@@ -516,10 +546,14 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))
     ts_barrier();
     for (int g = ng - 1; g >= 0; --g, ++par) {
       const int pb = par & 1;
-      // the state entering the group before this one, loaded while this one computes
+      // the state entering the group before this one, loaded while this one computes (split: while it walks backward,
+      // S itself being free then)
       float Sn[RL][KQ];
-      if (g > 1) get_state(g - 1, Sn);
-      else load_state(Sn);  // the checkpoint (after the chunk's first group it is not used)
+      auto load_next = [&](float (&X)[RL][KQ]) {
+        if (g > 1) get_state(g - 1, X);
+        else if (!SPLIT || g == 1) load_state(X);  // the checkpoint (after the chunk's first group it is not used)
+      };
+      if constexpr (!SPLIT) load_next(Sn);
       if (g < ng - 1) flush(g + 1, pb ^ 1);
       float Sd[TS_GS][RL][KQ];  // e^{la} S_{t-1} of the group's tokens
       ts_for<TS_GS>([&](auto I) {
@@ -541,13 +575,15 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))
         ts_rows_rs(t);
         sums.put(pb, 0, i, t, l);
       });
+      if constexpr (SPLIT) load_next(S);
       float out = 0.f, e4[TS_GS];  // lane p < 4 RL: dv of token p & 3, row p >> 2; the tokens' dla partials
       ts_for<TS_GS>([&](auto I) {
         constexpr int i = TS_GS - 1 - decltype(I)::value;
+        if constexpr (SPLIT) __builtin_amdgcn_sched_barrier(0);  // one token's reads at a time (registers)
         const float a = ts_lane<i>(ac);
         float uu[KQ], kk[KQ], qq[KQ], t[KQ], t2[KQ];
         TS::read(sv[pb][i], 2, p, qq);
-        TS::read(sv[pb][i], 1, p, uu);
+        if constexpr (!SPLIT) TS::read(sv[pb][i], 1, p, uu);
         TS::read(sv[pb][i], 0, p, kk);
         float d[RL], rc[RL];
         ts_for<RL>([&](auto RI) {
@@ -556,12 +592,19 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))
           const float gyc = ts_row_bcast<4 * RL + 4 * rr + i>(xc);
 #pragma unroll
           for (int j = 0; j < KQ; ++j) G[rr][j] = fmaf(gyc, qq[j], G[rr][j]);
-          d[rr] = ts_dot(G[rr], uu);
+          if constexpr (SPLIT) d[rr] = ts_row_bcast<4 * rr + i>(dc);
+          else d[rr] = ts_dot(G[rr], uu);
         });
-        ts_row_sums<RL, KQ>(d, [&](int j) {
+        auto du_part = [&](int j) {
           t[j] = G[0][j] * rc[0];
           if constexpr (RL == 2) t[j] = fmaf(G[RL - 1][j], rc[RL - 1], t[j]);
-        });
+        };
+        if constexpr (SPLIT) {
+#pragma unroll
+          for (int j = 0; j < KQ; ++j) du_part(j);
+        } else {
+          ts_row_sums<RL, KQ>(d, du_part);
+        }
         e4[i] = 0.f;
 #pragma unroll
         for (int rr = 0; rr < RL; ++rr) {
@@ -585,27 +628,137 @@ __global__ __launch_bounds__(SH::THREADS) __attribute__((amdgpu_waves_per_eu(2))
       e4[0] = sum16(e4[0]);
       if (p == 0) sums.sca[pb][wave_id()][l >> 4] = e4[0];
       if (g > 0) stage_grp((par + 1) & 1);  // the group before, loaded a group ago; ahead of the store, as in the forward
-      {
+      if constexpr (!SPLIT) {
         const int64_t tk = tok_in(g, ti);
         if (p < 4 * RL && tk >= 0 && srow < V) gv[tk * V + srow] = out;
       }
       if (g > 1) load_grp([&](int i) { return tok_in(g - 2, i); });
+      if constexpr (!SPLIT)
 #pragma unroll
-      for (int i = 0; i < RL; ++i)
+        for (int i = 0; i < RL; ++i)
 #pragma unroll
-        for (int j = 0; j < KQ; ++j) S[i][j] = Sn[i][j];
+          for (int j = 0; j < KQ; ++j) S[i][j] = Sn[i][j];
       ts_barrier();  // the group's vectors read and sums written; the group before staged
     }
     flush(0, (par - 1) & 1);
   }
-  // G is now the gradient of the state before the first token: the initial state's
-  if (dh0) {
+  if constexpr (!SPLIT)
+    if (dh0) {  // G is now the gradient of the state before the first token: the initial state's
+      const int64_t cb = (int64_t)(pid / NB) * K * V + (int64_t)p * KQ * V + v0;
 #pragma unroll
-    for (int i = 0; i < RL; ++i)
-      if (v0 + i < V) {
+      for (int i = 0; i < RL; ++i)
+        if (v0 + i < V) {
 #pragma unroll
-        for (int j = 0; j < KQ; ++j) dh0[cb + (int64_t)j * V + i] = G[i][j];
+          for (int j = 0; j < KQ; ++j) dh0[cb + (int64_t)j * V + i] = G[i][j];
+        }
+    }
+}
+
+// The state gradient's own recurrence, in reverse time: dv, dh0 and G before each chunk's last token (gst).  The
+// forward's mapping, blocks and staging with the token order reversed; per token
+//     G = e^{la'} W + dy q^T (la' of the token after);  dv = G u;  W = G - dv k^T,
+// dy q^T formed in the gaps of the row sum before.
+template <int K, typename SH>
+__global__ __launch_bounds__(SH::THREADS) void token_scan_gstate_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ u, const float* __restrict__ la,
+    const float* __restrict__ gy, const float* __restrict__ dhT, float* __restrict__ gv, float* __restrict__ gst,
+    float* __restrict__ dh0, int T_, int H, int V, int NCH, int NB) {
+  using TS = TokStage<K>;
+  static_assert(SH::RL == 1, "one row per lane");
+  constexpr int KQ = TS::KQ, NL = (TS_TB * TS::PER + SH::THREADS - 1) / SH::THREADS;
+  __shared__ __attribute__((aligned(16))) float sv[2][TS_TB][TS::SIZE];
+  const int tid = threadIdx.x, l = lane_id(), p = l & 15;
+  const int pid = blockIdx.x, bh = pid / NB, vb = pid - bh * NB;
+  const int b = bh / H, h = bh - b * H;
+  const int v0 = vb * SH::ROWS + wave_id() * SH::WROWS + (l >> 4);
+  const bool row = v0 < V;
+  const int64_t off = (int64_t)p * KQ * V + v0;  // this lane's entries of a [K][V] state: off + j V
+  float* gb = gst + (int64_t)bh * NCH * K * V;
+  const int64_t tok_first = (int64_t)b * T_ * H + h;
+  const int ti = p >> 1;
+  f32x4 xr[NL];
+  float gn = 0.f, ln = 0.f;
+  auto load_block = [&](int t0) {  // as in the forward, with dy in v's place
+#pragma unroll
+    for (int m = 0; m < NL; ++m) {
+      const int e = tid + m * SH::THREADS, i = e / TS::PER;
+      xr[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (e < TS_TB * TS::PER && t0 + i < T_)
+        xr[m] = TS::load(k, u, q, tok_first + (int64_t)(t0 + i) * H, e - i * TS::PER);
+    }
+    const bool in = t0 + ti < T_;
+    const int64_t tk = tok_first + (int64_t)(t0 + ti) * H;
+    gn = in && row ? gy[tk * V + v0] : 0.f;
+    ln = in ? la[tk] : 0.f;
+  };
+  auto stage_block = [&](float (*dst)[TS::SIZE]) {
+#pragma unroll
+    for (int m = 0; m < NL; ++m) {
+      const int e = tid + m * SH::THREADS, i = e / TS::PER;
+      if (e < TS_TB * TS::PER) TS::stage(dst[i], e - i * TS::PER, xr[m]);
+    }
+  };
+  float G[KQ];
+#pragma unroll
+  for (int j = 0; j < KQ; ++j) G[j] = dhT && row ? dhT[(int64_t)bh * K * V + (int64_t)j * V + off] : 0.f;
+  const int last = (T_ - 1) / TS_TB;  // T_ >= 1 here
+  load_block(last * TS_TB);
+  stage_block(sv[0]);
+  float gc = gn, ac = expf(ln);
+  if (last > 0) load_block((last - 1) * TS_TB);
+  ts_barrier();
+  for (int blk = last, buf = 0; blk >= 0; --blk, buf ^= 1) {
+    const int t0 = blk * TS_TB;
+    if (blk == last || (t0 + TS_TB) % TS_CT == 0) {  // the block ends its chunk
+      const int64_t c = t0 / TS_CT;
+      if (row) {
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) gb[c * K * V + (int64_t)j * V + off] = G[j];
       }
+    }
+    const float(*sb)[TS::SIZE] = sv[buf];
+    float vec[2][3][KQ], gq[KQ], dv = 0.f;  // lane 2 i: dv of token i
+    auto read3 = [&](int i, float (&d)[3][KQ]) {
+      TS::read(sb[i], 0, p, d[0]);
+      TS::read(sb[i], 1, p, d[1]);
+      TS::read(sb[i], 2, p, d[2]);
+    };
+    read3(TS_TB - 1, vec[(TS_TB - 1) & 1]);
+    const float gy_last = ts_row_bcast<2 * (TS_TB - 1)>(gc);
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) gq[j] = gy_last * vec[(TS_TB - 1) & 1][2][j];
+    ts_for<TS_TB>([&](auto I) {
+      constexpr int i = TS_TB - 1 - decltype(I)::value;
+      if constexpr (i > 0) read3(i - 1, vec[(i - 1) & 1]);
+      const auto& kk = vec[i & 1][0];
+      const auto& uu = vec[i & 1][1];
+      const float a = i + 1 < TS_TB ? ts_lane<(2 * i + 2) & 15>(ac) : 1.f;  // the block's last token: G is already decayed
+#pragma unroll
+      for (int j = 0; j < KQ; ++j) G[j] = i + 1 < TS_TB ? fmaf(a, G[j], gq[j]) : G[j] + gq[j];
+      float d[1] = {ts_dot(G, uu)};
+      const float gy_prev = i > 0 ? ts_row_bcast<(2 * i - 2) & 15>(gc) : 0.f;
+      ts_row_sums<1, KQ>(d, [&](int j) {
+        if constexpr (i > 0) gq[j] = gy_prev * vec[(i - 1) & 1][2][j];
+      });
+      dv = p == 2 * i ? d[0] : dv;
+#pragma unroll
+      for (int j = 0; j < KQ; ++j) G[j] = fmaf(-d[0], kk[j], G[j]);
+    });
+    const float a0 = ts_lane<0>(ac);
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) G[j] *= a0;
+    if (blk > 0) {  // stage the block before (loaded a block ago), ahead of the store, as in the forward
+      stage_block(sv[buf ^ 1]);
+      gc = gn;
+      ac = expf(ln);
+    }
+    if (!(p & 1) && t0 + ti < T_ && row) gv[(tok_first + (int64_t)(t0 + ti) * H) * V + v0] = dv;
+    if (blk > 1) load_block(t0 - 2 * TS_TB);
+    ts_barrier();
+  }
+  if (dh0 && row) {
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) dh0[(int64_t)bh * K * V + (int64_t)j * V + off] = G[j];
   }
 }
 
@@ -636,40 +789,96 @@ static int ts_rows(int B, int T, int H, int K, int V, bool backward) {
   return rows;
 }
 
+// The backward's plan.  split: the state gradient's recurrence in a launch of its own (G at every chunk's end into gst),
+// the rest chunk by chunk in parallel, which pays while the whole chain's workgroups leave the chip waiting for it.
+struct TsBwdPlan {
+  bool split;
+  int rows;                           // per workgroup (of the chunk kernel when split)
+  int64_t items, wgs;                 // the chunk kernel's items when split; workgroups
+  size_t gst_floats, scratch_floats;  // gst first, then the workgroups' group-start states
+};
+// Costs in hundredths of a token of a lone 16-row workgroup (0.87 us at K = 128), as measured at H4 K128 V256: the whole
+// chain per token and round over the CUs 100 (16 rows; 135 for each pair of rounds), 125 (32) and 200 (64); split, the
+// state gradient per token 25 (one round of 16 rows) or 35 a round of 32, and the chunk kernel per 32-token chunk and
+// round 150 (16 rows, two workgroups a CU) or 205 (64 rows) times 32, and the second launch 1000.  The call, us, whole
+// chain and split: B4 T1024 1229 and 939; B1 T4096 4381 and 2264; H1 V64 B1 T1500 1495 and 681; B8 T512 767 and 797; B16
+// T512 1202 and 1408; H1 B120 T34 216 and 322 -- the rule takes the faster one in each.  gst is kept under TS_PART_BYTES.
+static TsBwdPlan ts_bwd_plan(int B, int T, int H, int K, int V) {
+  const int64_t cus = device_cu_count(), BH = (int64_t)B * H, NCH = (T + TS_CT - 1) / TS_CT;
+  auto blocks = [&](int rows) { return (int64_t)((V + rows - 1) / rows); };
+  auto rounds = [&](int64_t wgs, int64_t per_cu) { return (wgs + per_cu * cus - 1) / (per_cu * cus); };
+  TsBwdPlan p{};
+  p.rows = ts_rows(B, T, H, K, V, true);
+  const int64_t r = rounds(BH * blocks(p.rows), 1);
+  const int64_t whole = p.rows == 64 ? 200 * r : p.rows == 32 ? 125 * r : r == 1 ? 100 : 135 * ((r + 1) / 2);
+  const int64_t c16 = 150 * rounds(BH * NCH * blocks(16), 2), c64 = 205 * rounds(BH * NCH * blocks(64), 1);
+  const int64_t state = rounds(BH * blocks(16), 1) <= 1 ? 25 : 35 * rounds(BH * blocks(32), 1);
+  const int64_t gst = BH * NCH * K * V;
+  p.split = T * state + TS_CT * std::min(c16, c64) + 1000 < T * whole && gst * 4 <= TS_PART_BYTES;
+  if (p.split) p.rows = c16 < c64 && BH * T * K * blocks(16) * 12 <= TS_PART_BYTES ? 16 : 64;
+  p.items = BH * blocks(p.rows) * (p.split ? NCH : 1);
+  // resident workgroups per CU: two of 16 rows (249 registers, 68 KB of LDS at K = 128), one of 64 (117 KB)
+  p.wgs = p.split ? std::min<int64_t>(p.items, cus * (p.rows == 16 ? 2 : 1)) : p.items;
+  p.gst_floats = p.split ? (size_t)((gst + 3) / 4 * 4) : 0;
+  p.scratch_floats = p.gst_floats + (size_t)p.wgs * (TS_CT / TS_GS) * K * p.rows;
+  return p;
+}
+
 int token_scan_row_blocks(int B, int T, int H, int K, int V) {
-  const int rows = ts_rows(B, T, H, K, V, true);
+  const int rows = ts_bwd_plan(B, T, H, K, V).rows;
   return (V + rows - 1) / rows;
 }
 size_t token_scan_scratch_floats(int B, int T, int H, int K, int V) {
-  const int rows = ts_rows(B, T, H, K, V, true);
-  return (size_t)B * H * ((V + rows - 1) / rows) * (TS_CT / TS_GS) * K * rows;
+  return ts_bwd_plan(B, T, H, K, V).scratch_floats;
 }
 
 template <int K, typename SH>
-static hipError_t token_scan_sh(const TokenScanArgs& a, bool backward) {
+static hipError_t token_scan_fwd_sh(const TokenScanArgs& a) {
   const int NB = (a.V + SH::ROWS - 1) / SH::ROWS, NCH = (a.T + TS_CT - 1) / TS_CT;
-  const dim3 grid((unsigned)(a.B * a.H * NB));
-  if (!backward) {
-    if constexpr (SH::RL == 1)
-      token_scan_fwd_kernel<K, SH><<<grid, SH::THREADS, 0, a.stream>>>(a.q, a.k, a.u, a.v, a.la, a.h0, a.y, a.r, a.st,
-                                                                       a.hT, a.T, a.H, a.V, NCH, NB);
-    else
-      return hipErrorInvalidValue;  // ts_rows gives the forward 16 or 32 rows
-  } else {
-    token_scan_bwd_kernel<K, SH><<<grid, SH::THREADS, 0, a.stream>>>(
-        a.q, a.k, a.u, a.la, a.r, a.st, a.dy, a.dhT, a.dv, a.dq_part, a.du_part, a.dk_part, a.dla_part, a.dh0,
-        a.scratch, a.T, a.H, a.V, NCH, NB, (int64_t)a.B * a.T * a.H);
-  }
+  token_scan_fwd_kernel<K, SH><<<dim3((unsigned)(a.B * a.H * NB)), SH::THREADS, 0, a.stream>>>(
+      a.q, a.k, a.u, a.v, a.la, a.h0, a.y, a.r, a.st, a.hT, a.T, a.H, a.V, NCH, NB);
+  return hipGetLastError();
+}
+
+template <int K, typename SH>
+static hipError_t token_scan_gstate_sh(const TokenScanArgs& a) {
+  const int NB = (a.V + SH::ROWS - 1) / SH::ROWS, NCH = (a.T + TS_CT - 1) / TS_CT;
+  token_scan_gstate_kernel<K, SH><<<dim3((unsigned)(a.B * a.H * NB)), SH::THREADS, 0, a.stream>>>(
+      a.q, a.k, a.u, a.la, a.dy, a.dhT, a.dv, a.scratch, a.dh0, a.T, a.H, a.V, NCH, NB);
+  return hipGetLastError();
+}
+
+template <int K, typename SH, bool SPLIT>
+static hipError_t token_scan_bwd_sh(const TokenScanArgs& a, const TsBwdPlan& p) {
+  const int NB = (a.V + SH::ROWS - 1) / SH::ROWS, NCH = (a.T + TS_CT - 1) / TS_CT;
+  token_scan_bwd_kernel<K, SH, SPLIT><<<dim3((unsigned)p.wgs), SH::THREADS, 0, a.stream>>>(
+      a.q, a.k, a.u, a.la, a.r, a.st, a.dy, a.dhT, a.dv, a.dq_part, a.du_part, a.dk_part, a.dla_part, a.dh0,
+      a.scratch + p.gst_floats, a.scratch, (int)p.items, a.T, a.H, a.V, NCH, NB, (int64_t)a.B * a.T * a.H);
   return hipGetLastError();
 }
 
 template <int K>
-static hipError_t token_scan_k(const TokenScanArgs& a, bool backward) {
-  switch (ts_rows(a.B, a.T, a.H, K, a.V, backward)) {
-    case 16: return token_scan_sh<K, TsShape<1, 4>>(a, backward);
-    case 32: return token_scan_sh<K, TsShape<1, 8>>(a, backward);
-    default: return token_scan_sh<K, TsShape<2, 8>>(a, backward);
+static hipError_t token_scan_bwd_k(const TokenScanArgs& a, const TsBwdPlan& p) {
+  if (p.split)
+    return p.rows == 16 ? token_scan_bwd_sh<K, TsShape<1, 4>, true>(a, p) : token_scan_bwd_sh<K, TsShape<2, 8>, true>(a, p);
+  switch (p.rows) {
+    case 16: return token_scan_bwd_sh<K, TsShape<1, 4>, false>(a, p);
+    case 32: return token_scan_bwd_sh<K, TsShape<1, 8>, false>(a, p);
+    default: return token_scan_bwd_sh<K, TsShape<2, 8>, false>(a, p);
   }
+}
+
+template <int K>
+static hipError_t token_scan_k(const TokenScanArgs& a, bool backward) {
+  const bool narrow = ts_rows(a.B, a.T, a.H, K, a.V, false) == 16;  // one row per lane in 4 or 8 waves
+  if (!backward)
+    return narrow ? token_scan_fwd_sh<K, TsShape<1, 4>>(a) : token_scan_fwd_sh<K, TsShape<1, 8>>(a);
+  const TsBwdPlan p = ts_bwd_plan(a.B, a.T, a.H, K, a.V);
+  if (p.split) {
+    const hipError_t e = narrow ? token_scan_gstate_sh<K, TsShape<1, 4>>(a) : token_scan_gstate_sh<K, TsShape<1, 8>>(a);
+    if (e != hipSuccess) return e;
+  }
+  return token_scan_bwd_k<K>(a, p);
 }
 
 hipError_t launch_token_scan(const TokenScanArgs& a, bool backward) {

@@ -245,10 +245,11 @@ int gdn_cross_entropy_fwd_bwd(void* logits, const int64_t* target, float* loss, 
                               int64_t N, int V, int64_t ld, int64_t ignore_index, int dtype, void* stream);
 
 /* The streaming passes around the fused loss's matrix products: y = *s x (s a device scalar) over n elements of dtype,
- * and out = sum over p < nparts of part[p * n + i] (fp32, p ascending), rounded once to dtype (n a multiple of 8). */
+ * and out = sum over p < nparts of part[p * n + i] (fp32), added in 64 bits and rounded to dtype (n a multiple of
+ * 8). */
 int gdn_scale(const void* x, const float* s, void* y, int64_t n, int dtype, void* stream);
 int gdn_sum_parts(const float* part, int nparts, void* out, int64_t n, int dtype, void* stream);
-/* The same for parts [K, N] written transposed, out [N, K]; N and K multiples of 4. */
+/* The same for parts [K, N] written transposed, out [N, K], added in fp32, p ascending; N and K multiples of 4. */
 int gdn_sum_parts_t(const float* part, int nparts, void* out, int N, int K, int dtype, void* stream);
 /* out [M, C] (out_dtype) = dx [M, C] + a [M, J] w [J, C]: bf16 operands, fp32 sums; J even and at most 32, C a multiple
  * of 4. */

@@ -94,7 +94,8 @@ def test_fused_linear_ce_passes_and_parts(N, H, V, num_chunks):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("n,S", [(1, 1), (8, 3), (1001, 2), (4096, 16)])
 def test_scale_and_sum_of_parts(dtype, n, S):
-    """ops.scaled equals the product in fp32 rounded once, ops.sum_parts_ the ordered fp32 sum rounded once, exactly."""
+    """ops.scaled equals the product in fp32 rounded once, ops.sum_parts_ the ordered 64-bit sum rounded to fp32 and the
+    dtype, exactly."""
     banner(f"scaled / sum of parts n={n} S={S} {dtype}")
     gen = torch.Generator("cuda").manual_seed(n)
     x = torch.randn(n, device="cuda", generator=gen).to(dtype)
@@ -102,9 +103,9 @@ def test_scale_and_sum_of_parts(dtype, n, S):
     assert torch.equal(ops.scaled(x, s), (x.float() * s).to(dtype))
     if n % 8 == 0:
         parts = torch.randn(S, n, device="cuda", generator=gen)
-        ref = torch.zeros(n, device="cuda")
+        ref = torch.zeros(n, device="cuda", dtype=torch.float64)
         for p in parts:
             ref += p
         out = torch.empty(n, device="cuda", dtype=dtype)
         ops.sum_parts_(parts, out)
-        assert torch.equal(out, ref.to(dtype))
+        assert torch.equal(out, ref.float().to(dtype))

@@ -146,3 +146,36 @@ def test_token_scan_row_blocks(B, T, H, V, rows, K):
     print("[rel-L2] " + ", ".join(f"{n} {e:.1e}" for n, e in errs.items()), flush=True)
     for n, e in errs.items():
         assert e <= 1e-6, (n, e)
+
+
+@pytest.mark.parametrize("B,T,H,V,rows", [(1, 256, 2, 17, 16), (2, 257, 2, 1, 16), (3, 290, 1, 100, 16),
+                                          (4, 199, 4, 250, 64), (17, 300, 1, 256, 64)])
+@pytest.mark.parametrize("K", [64, 128])
+def test_token_scan_split_backward(B, T, H, V, rows, K):
+    """The backward with the state gradient's recurrence in its own launch (16 and 32 rows per workgroup) and the chunks
+    in parallel (16 and 64 rows, more chunks than workgroups in the larger ones): whole and partial row blocks, last chunks
+    of 1 to 32 tokens, with and without states.  The bound is test_token_scan_row_blocks's."""
+    banner(f"token scan split backward rows {rows}: B={B} T={T} H={H} K={K} V={V}")
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        st_bytes, sc_bytes, nb = ops._token_sizes(ops._lib.load(), B, T, H, K, V)
+        assert nb == -(-V // rows), nb
+        wgs = min(B * H * nb * -(-T // 32), 512 if rows == 16 else 256)
+        assert sc_bytes == -(-st_bytes // 16) * 16 + wgs * 8 * K * rows * 4
+    q, k, u, v, la, dy = _inputs(B, T, H, K, V, seed=B + T + K + V)
+    g = torch.Generator().manual_seed(7)
+    h0, dhT = (0.1 * torch.randn(B, H, K, V, generator=g) for _ in range(2))
+    d = [t.cuda() for t in (q, k, u, v, la, dy, h0, dhT)]
+    y, r, st, _ = ops.nsgdn_token_fwd(*d[:5], d[6], True)
+    got = ops.nsgdn_token_bwd(d[0], d[1], d[2], d[4], r, st, d[5], d[7], True)
+    assert all(torch.equal(a, b) for a, b in
+               zip(got, ops.nsgdn_token_bwd(d[0], d[1], d[2], d[4], r, st, d[5], d[7], True)))
+    ref = NS.recurrent_bwd(q, k, u, v, la, dy, h0=h0, dhT=dhT)
+    _, r0, st0, _ = ops.nsgdn_token_fwd(*d[:5], None, False)
+    got0 = ops.nsgdn_token_bwd(d[0], d[1], d[2], d[4], r0, st0, d[5], None, False)[:5]
+    ref0 = NS.recurrent_bwd(q, k, u, v, la, dy)[:5]
+    names = ("dq", "dk", "du", "dv", "dla", "dh0")
+    errs = {n: rel_l2(a, b) for n, a, b in zip(names, got, ref)}
+    errs.update({n + " (no states)": rel_l2(a, b) for n, a, b in zip(names, got0, ref0)})
+    print("[rel-L2] " + ", ".join(f"{n} {e:.1e}" for n, e in errs.items()), flush=True)
+    for n, e in errs.items():
+        assert e <= 1e-6, (n, e)
