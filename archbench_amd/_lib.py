@@ -66,6 +66,7 @@ SIGNATURES = {
     "gdn_narrow_dx": (_i, [_p, _p, _p, _p, _i64, _i, _i, _i, _p]),
     "gdn_write_direction_fwd": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p]),
     "gdn_write_direction_bwd": (_i, [_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p]),
+    "gdn_sum_heads": (_i, [_p, _i64, _i, _p, _sz, _p, _p]),
     "gdn_token_scan_sizes": (_i, [_i, _i, _i, _i, _i, ctypes.POINTER(_sz), ctypes.POINTER(_sz), ctypes.POINTER(_i)]),
     "gdn_token_scan_fwd": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _p, _i, _i, _i, _i, _i, _p]),
     "gdn_token_scan_bwd": (_i, [_p, _p, _p, _p, _p, _p, _sz, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i,

@@ -1039,6 +1039,18 @@ int gdn_write_direction_bwd(const void* k, const float* beta, const float* lam, 
   return GDN_OK;
 }
 
+int gdn_sum_heads(const float* x, int64_t n, int H, void* ws, size_t ws_bytes, float* out, void* stream) {
+  g_err[0] = 0;
+  if (n <= 0 || H <= 0 || H > 256) return fail(GDN_ERR_ARG, "invalid sizes n=%lld H=%d", (long long)n, H);
+  const size_t need = (size_t)head_sum_groups(n, H) * H * 8;
+  if (ws_bytes < need) return fail(GDN_ERR_WORKSPACE, "workspace %zu bytes, need %zu", ws_bytes, need);
+  if (!x || !ws || !out) return fail(GDN_ERR_ARG, "null input/output pointer");
+  if (misaligned(ws)) return fail(GDN_ERR_ARG, "workspace not 16-byte aligned");
+  const hipError_t e = launch_head_sum(x, n, H, static_cast<double*>(ws), out, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "head sum launch: %s", hipGetErrorString(e));
+  return GDN_OK;
+}
+
 static int token_scan_check(int B, int T, int H, int K, int V) {
   if (B < 0 || T < 0 || H <= 0 || V <= 0) return fail(GDN_ERR_ARG, "invalid sizes B=%d T=%d H=%d V=%d", B, T, H, V);
   if (!token_scan_supported(K)) return fail(GDN_ERR_SHAPE, "token scan not compiled for K=%d (K in {64, 128})", K);

@@ -417,6 +417,18 @@ def _(k, beta, lam, n_steps):
     return torch.empty_like(k)
 
 
+def _sum_heads(x: Tensor) -> Tensor:
+    """x [B, T, H] fp32 (contiguous) summed over B and T."""
+    H = x.shape[-1]
+    if x.numel() == 0 or H > 256:
+        return x.sum((0, 1))
+    out = torch.empty(H, dtype=torch.float32, device=x.device)
+    ws = _lib.workspace(x.device, 256 * H * 8)
+    _lib.check(_lib.load().gdn_sum_heads(_lib.ptr(x), x.numel() // H, H, _lib.ptr(ws), ws.numel(), _lib.ptr(out),
+                                         _lib.stream_ptr(x.device)), "gdn_sum_heads")
+    return out
+
+
 @gpu_op("archbench_amd::write_direction_bwd")
 def write_direction_bwd(k: Tensor, beta: Tensor, lam: Tensor, du: Tensor,
                         n_steps: int) -> tuple[Tensor, Tensor, Tensor]:
@@ -432,7 +444,7 @@ def write_direction_bwd(k: Tensor, beta: Tensor, lam: Tensor, du: Tensor,
                                      _lib.ptr(dbeta), _lib.ptr(dlam_rows), B, T, H, K, max(int(n_steps), 1),
                                      _lib.dtype_code(k.dtype), _lib.stream_ptr(k.device))
     _lib.check(rc, "gdn_write_direction_bwd")
-    return dk, dbeta, dlam_rows.sum((0, 1))
+    return dk, dbeta, _sum_heads(dlam_rows)
 
 
 @write_direction_bwd.register_fake

@@ -268,6 +268,9 @@ int gdn_write_direction_fwd(const void* k, const float* beta, const float* lam, 
 int gdn_write_direction_bwd(const void* k, const float* beta, const float* lam, const void* du, void* dk,
                             float* dbeta, float* dlam, int B, int T, int H, int K, int n_steps, int dtype,
                             void* stream);
+/* out [H] = the sum over n >= 1 rows of x [n, H] (fp32, H <= 256), added in 64 bits in a fixed order: dlam's.  ws: up to
+ * 256 * H * 8 bytes, 16-byte aligned. */
+int gdn_sum_heads(const float* x, int64_t n, int H, void* ws, size_t ws_bytes, float* out, void* stream);
 
 /* Exact fp32 token scan of the n-step family: the reference's "triton" / "ref" scan, archbench::nsgdn_fwd and
  * archbench::nsgdn_bwd (archbench/layers/nsgdn.py:80-154, ops :162-216, the recurrence of nsgdn_ref :408-417).

@@ -94,3 +94,18 @@ def test_write_direction_one_step_and_edges():
         ops.write_direction(torch.randn(1, 4, 2, 96, device="cuda"), beta[:1, :4].cuda(), lam.cuda(), 2)
     with pytest.raises(ValueError, match="beta must be"):
         ops.write_direction(k.cuda(), beta[:, :3].cuda(), lam.cuda(), 2)
+
+
+@pytest.mark.parametrize("B,T,H", [(1, 1, 1), (2, 77, 3), (1, 2048, 1), (4, 513, 6), (3, 1000, 8), (1, 2500, 256), (1, 2, 100),
+                                   (1, 300, 257)])
+def test_sum_heads(B, T, H):
+    """dlam's sum over the tokens: one workgroup and several, heads that do not divide its 256 threads, and more heads than
+    it takes (torch's sum there).  In 64 bits with one rounding: 2^-24 of the result, and 2^-52 of the sum of magnitudes per
+    addition; torch's fp32 tree 2^-20 of that sum."""
+    banner(f"sum over tokens B={B} T={T} H={H}")
+    x = torch.randn(B, T, H, device="cuda", generator=torch.Generator("cuda").manual_seed(T + H))
+    out, ref = ops._sum_heads(x).double(), x.double().sum((0, 1))
+    per = B * T * 2.0 ** -52 if H <= 256 else 2.0 ** -20
+    assert out.shape == (H,)
+    assert ((out - ref).abs() <= 2.0 ** -24 * ref.abs() + per * x.double().abs().sum((0, 1))).all()
+    assert torch.equal(ops._sum_heads(x).double(), out)
