@@ -61,8 +61,10 @@ def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> None:
     """out [rows, d] = dlogits [rows, V] W [V, d]."""
     rows, V = dlogits.shape
     d = weight.shape[1]
-    # 16-byte rows throughout; not under an autocast that would change a dtype
-    split = dlogits.dtype == weight.dtype == out.dtype == torch.bfloat16 and d % 8 == 0 and weight.is_contiguous()
+    # 16-byte rows throughout; not under an autocast that would change a dtype, nor into the gradient of an x laid out
+    # feature by feature (dx has x's strides)
+    split = (dlogits.dtype == weight.dtype == out.dtype == torch.bfloat16 and d % 8 == 0 and weight.is_contiguous()
+             and out.is_contiguous())
     S = _dx_split(rows, d, V) if split else 1
     if S == 1:
         out.copy_(dlogits @ weight)

@@ -91,6 +91,25 @@ def test_fused_linear_ce_passes_and_parts(N, H, V, num_chunks):
     assert rel_l2(wd.grad, 3.0 * dw_r) <= 1e-2
 
 
+@pytest.mark.parametrize("num_chunks", [1, 8])
+def test_fused_linear_ce_feature_major_x(num_chunks):
+    """Hidden states laid out feature by feature (a dense transposed x, whose gradient has its strides), at a size whose
+    dx may be taken in parts: the same result as for the row-major copy to the rounding of dx."""
+    banner(f"fused linear CE feature-major x chunks={num_chunks}")
+    N, H, V = 1100, 128, 8192
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn(1, H, N, generator=gen).bfloat16().cuda().transpose(1, 2)
+    w = (torch.randn(V, H, generator=gen) * 0.05).bfloat16()
+    t = torch.randint(0, V, (1, N), generator=gen)
+    assert fused_ce._dx_split(fused_ce._rows_per_pass(N, num_chunks, H, 2), H, V) > 1 and not x[0].is_contiguous()
+    xd, wd = x.requires_grad_(), w.cuda().requires_grad_()
+    loss = fused_ce.fused_linear_cross_entropy(xd, t.cuda(), wd, num_chunks=num_chunks)
+    loss.backward()
+    l_r, dx_r, dw_r = CE.linear_ce(x.detach().float().cpu().reshape(-1, H), t.reshape(-1), w.float())
+    assert abs(loss.item() - l_r.item()) <= 1e-3 * abs(l_r.item())
+    assert rel_l2(xd.grad.reshape(-1, H), dx_r) <= 1e-2 and rel_l2(wd.grad, dw_r) <= 1e-2
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("n,S", [(1, 1), (8, 3), (1001, 2), (4096, 16)])
 def test_scale_and_sum_of_parts(dtype, n, S):
