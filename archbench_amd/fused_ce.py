@@ -90,10 +90,13 @@ class _FusedLinearCE(torch.autograd.Function):
             logits = c_x @ weight.t()
             loss_rows[s:e] = ops.cross_entropy_fwd_bwd_(logits, target[s:e], dloss, ignore_index)[0]
             _dx(logits, weight, dx[s:e])
-            if C >= N:
+            if C >= N and (num_chunks == 1 or logits.dtype == weight.dtype):
                 # one pass: dW needs no accumulation across passes, so the GEMM writes it in the weight's dtype
                 # directly (fp32 accumulation inside, one rounding -- where several passes round at the end)
                 dw = logits.t() @ c_x
+            elif C >= N:
+                # under autocast an fp32 weight's gradient over several chunks keeps its fp32 sums, also in one pass
+                dw = torch.mm(logits.t(), c_x.to(logits.dtype), out_dtype=torch.float32)
             elif dw is None:
                 dw = torch.mm(logits.t(), c_x, out_dtype=torch.float32)
             else:  # in place

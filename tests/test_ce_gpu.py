@@ -110,6 +110,26 @@ def test_fused_linear_ce_feature_major_x(num_chunks):
     assert rel_l2(xd.grad.reshape(-1, H), dx_r) <= 1e-2 and rel_l2(wd.grad, dw_r) <= 1e-2
 
 
+@pytest.mark.parametrize("N,x_dtype", [(96, torch.bfloat16), (1100, torch.bfloat16), (96, torch.float32)])
+def test_fused_linear_ce_fp32_weight_under_autocast(N, x_dtype):
+    """bf16 (and, in one pass, fp32) hidden states and an fp32 weight under bf16 autocast: over several chunks the weight's gradient holds fp32
+    sums, also where every row fits one pass (a sum rounded to bf16 on the way would be a bf16 number throughout)."""
+    H, V, num_chunks = 128, 4096, 8
+    rows = fused_ce._rows_per_pass(N, num_chunks, H, 2)
+    banner(f"fused linear CE fp32 weight N={N}: {rows} rows per pass")
+    gen = torch.Generator().manual_seed(N)
+    x = torch.randn(1, N, H, generator=gen).bfloat16()
+    w = (torch.randn(V, H, generator=gen) * 0.05).bfloat16().float()
+    t = torch.randint(0, V, (1, N), generator=gen)
+    xd, wd = x.to("cuda", x_dtype).requires_grad_(), w.cuda().requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        loss = fused_ce.fused_linear_cross_entropy(xd, t.cuda(), wd, num_chunks=num_chunks)
+    loss.backward()
+    assert wd.grad.dtype == torch.float32
+    assert (wd.grad != wd.grad.bfloat16().float()).float().mean() > 0.9  # 2^-16 of fp32 values are bf16 ones
+    assert rel_l2(wd.grad, CE.linear_ce(x.float().reshape(-1, H), t.reshape(-1), w)[2]) <= 1e-2
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("n,S", [(1, 1), (8, 3), (1001, 2), (4096, 16)])
 def test_scale_and_sum_of_parts(dtype, n, S):
