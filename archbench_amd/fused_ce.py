@@ -74,6 +74,11 @@ def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> None:
     ops.sum_parts_(parts, out)
 
 
+def _scaled(t: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
+    """s t for a device scalar s; the dtypes that the kernels do not take (an fp16 weight under autocast) in torch."""
+    return ops.scaled(t, s) if t.dtype in (torch.bfloat16, torch.float32) else t * s
+
+
 class _FusedLinearCE(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, target, weight, num_chunks: int, ignore_index: int):
@@ -108,7 +113,7 @@ class _FusedLinearCE(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         dx, dw = ctx.saved_tensors
-        return ops.scaled(dx, dout), None, ops.scaled(dw, dout), None, None
+        return _scaled(dx, dout), None, _scaled(dw, dout), None, None
 
 
 def fused_linear_cross_entropy(x, target, weight, num_chunks: int = 8, ignore_index: int = -100):

@@ -130,6 +130,24 @@ def test_fused_linear_ce_fp32_weight_under_autocast(N, x_dtype):
     assert rel_l2(wd.grad, CE.linear_ce(x.float().reshape(-1, H), t.reshape(-1), w)[2]) <= 1e-2
 
 
+@pytest.mark.parametrize("num_chunks", [1, 8])
+def test_fused_linear_ce_fp16_weight_under_autocast(num_chunks):
+    """An fp16 weight under bf16 autocast: its gradient comes back in fp16."""
+    banner(f"fused linear CE fp16 weight chunks={num_chunks}")
+    N, H, V = 300, 128, 4096
+    gen = torch.Generator().manual_seed(5)
+    x = torch.randn(1, N, H, generator=gen).bfloat16()
+    w = (torch.randn(V, H, generator=gen) * 0.05).bfloat16()
+    t = torch.randint(0, V, (1, N), generator=gen)
+    xd, wd = x.cuda().requires_grad_(), w.to("cuda", torch.float16).requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        loss = fused_ce.fused_linear_cross_entropy(xd, t.cuda(), wd, num_chunks=num_chunks)
+    (1024.0 * loss).backward()  # a gradient scale that keeps fp16's small values normal
+    _, dx_r, dw_r = CE.linear_ce(x.float().reshape(-1, H), t.reshape(-1), w.float())
+    assert wd.grad.dtype == torch.float16 and rel_l2(wd.grad, 1024 * dw_r) <= 1e-2
+    assert rel_l2(xd.grad.reshape(-1, H), 1024 * dx_r) <= 1e-2
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("n,S", [(1, 1), (8, 3), (1001, 2), (4096, 16)])
 def test_scale_and_sum_of_parts(dtype, n, S):
