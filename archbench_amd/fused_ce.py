@@ -27,6 +27,7 @@ def fused_ce_available() -> bool:
     return True
 
 
+_KERNEL_DTYPES = (torch.bfloat16, torch.float32)
 _TILE = 256  # rows and columns of the GEMMs' output tiles
 
 
@@ -57,26 +58,49 @@ def _dx_split(rows: int, d: int, V: int) -> int:
     return max(S, 1)
 
 
-def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor) -> None:
-    """out [rows, d] = dlogits [rows, V] W [V, d]."""
+# Below this a call waits for its launches, not for its kernels: 250 us for about 25 torch and package calls from Python,
+# forward and backward (measured at N 128 to 1024, d 384 to 1024, V 8192).
+_HOST_US = 250
+
+
+def _outlasts_host(N: int, d: int, V: int) -> bool:
+    """Whether a call's kernels take longer than its launches, so that extra calls which shorten them pay.  In us: dx's
+    product in one part (its chain over V alone takes about 3.5 ns a class while the tiles leave CUs idle: V 8192, 32000
+    and 50304 at 128 to 1024 rows 15 to 45, 97 to 175 and 146 to 242; in the parts of _dx_split 13 to 35, 28 to 91 and
+    35 to 118, for 25 us of the host), 6 N d V operations at 0.6 PFLOP/s, and the passes over W's size with torch's
+    scaling of its gradient.  Calls at V 8192, N 128 to 1024 (43 to 146 by this count): 215 to 252 us, with parts and the
+    HIP scaling 341 to 350; N 1024, d 512, V 32000 (345): 350 and 258; N 128, d 1024, V 50304 (448): 420 and 289."""
+    return 3.5e-3 * V + V * d * (1e-8 * N + 4e-6) > _HOST_US
+
+
+def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None, N: int) -> torch.Tensor:
+    """dlogits [rows, V] W [V, d] of a call with N rows, written to ``out`` if given."""
     rows, V = dlogits.shape
     d = weight.shape[1]
     # 16-byte rows throughout; not under an autocast that would change a dtype, nor into the gradient of an x laid out
     # feature by feature (dx has x's strides)
-    split = (dlogits.dtype == weight.dtype == out.dtype == torch.bfloat16 and d % 8 == 0 and weight.is_contiguous()
-             and out.is_contiguous())
+    split = (dlogits.dtype == weight.dtype == torch.bfloat16 and d % 8 == 0 and weight.is_contiguous()
+             and (out is None or (out.dtype == torch.bfloat16 and out.is_contiguous())) and _outlasts_host(N, d, V))
     S = _dx_split(rows, d, V) if split else 1
     if S == 1:
-        out.copy_(dlogits @ weight)
-        return
+        return dlogits @ weight if out is None else out.copy_(dlogits @ weight)
+    if out is None:
+        out = dlogits.new_empty(rows, d)
     parts = torch.bmm(dlogits.view(rows, S, V // S).transpose(0, 1), weight.view(S, V // S, d),
                       out_dtype=torch.float32)
     ops.sum_parts_(parts, out)
+    return out
 
 
-def _scaled(t: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
-    """s t for a device scalar s; the dtypes that the kernels do not take (an fp16 weight under autocast) in torch."""
-    return ops.scaled(t, s) if t.dtype in (torch.bfloat16, torch.float32) else t * s
+def _scaled(t: torch.Tensor, s: torch.Tensor, hip: bool) -> torch.Tensor:
+    """s t for a 0-d s, the product in fp32 and rounded once.  The HIP pass (``hip``) runs at the copy rate, 41 us for 64M
+    bf16 elements where torch's mixed-type loop takes 163, but as an op it costs the host 20 us more in a backward."""
+    if t.dtype not in (torch.bfloat16, torch.float32):  # an fp16 weight under autocast
+        return t * s
+    if hip or torch.is_grad_enabled():
+        return ops.scaled(t, s)
+    # a 1-d s, which takes part in the type promotion: torch rounds a 0-d one to t's dtype first
+    return torch.mul(t, s.reshape(1), out=torch.empty_like(t))
 
 
 class _FusedLinearCE(torch.autograd.Function):
@@ -86,34 +110,38 @@ class _FusedLinearCE(torch.autograd.Function):
         C = _rows_per_pass(N, num_chunks, d, x.element_size())
         total = target.ne(ignore_index).sum().clamp_min(1)
         dloss = total.float().reciprocal().reshape(1)  # device scalar: no host sync
-        loss_rows = torch.empty(N, device=x.device, dtype=torch.float32)
-        dx = torch.empty_like(x)
-        dw = None
-        for s in range(0, max(N, 1), C):
-            e = min(s + C, N)
-            c_x = x[s:e]
-            logits = c_x @ weight.t()
-            loss_rows[s:e] = ops.cross_entropy_fwd_bwd_(logits, target[s:e], dloss, ignore_index)[0]
-            _dx(logits, weight, dx[s:e])
-            if C >= N and (num_chunks == 1 or logits.dtype == weight.dtype):
-                # one pass: dW needs no accumulation across passes, so the GEMM writes it in the weight's dtype
-                # directly (fp32 accumulation inside, one rounding -- where several passes round at the end)
-                dw = logits.t() @ c_x
-            elif C >= N:
-                # under autocast an fp32 weight's gradient over several chunks keeps its fp32 sums, also in one pass
-                dw = torch.mm(logits.t(), c_x.to(logits.dtype), out_dtype=torch.float32)
-            elif dw is None:
-                dw = torch.mm(logits.t(), c_x, out_dtype=torch.float32)
-            else:  # in place
-                torch.addmm(dw, logits.t(), c_x, out_dtype=torch.float32, out=dw)
-            del logits
+        if C >= N:
+            logits = x @ weight.t()
+            loss_rows = ops.cross_entropy_fwd_bwd_(logits, target, dloss, ignore_index)[0]
+            dx = _dx(logits, weight, None, N).to(x.dtype)
+            if num_chunks == 1 or logits.dtype == weight.dtype:
+                # dW needs no accumulation across passes, so the GEMM writes it in the weight's dtype directly (fp32
+                # accumulation inside, one rounding -- where several passes round at the end)
+                dw = logits.t() @ x
+            else:  # under autocast an fp32 weight's gradient over several chunks keeps its fp32 sums, also in one pass
+                dw = torch.mm(logits.t(), x.to(logits.dtype), out_dtype=torch.float32)
+        else:
+            loss_rows = torch.empty(N, device=x.device, dtype=torch.float32)
+            dx, dw = torch.empty_like(x), None
+            for s in range(0, N, C):
+                e = min(s + C, N)
+                c_x = x[s:e]
+                logits = c_x @ weight.t()
+                loss_rows[s:e] = ops.cross_entropy_fwd_bwd_(logits, target[s:e], dloss, ignore_index)[0]
+                _dx(logits, weight, dx[s:e], N)
+                if dw is None:
+                    dw = torch.mm(logits.t(), c_x, out_dtype=torch.float32)
+                else:  # in place
+                    torch.addmm(dw, logits.t(), c_x, out_dtype=torch.float32, out=dw)
+                del logits
         ctx.save_for_backward(dx, dw.to(weight.dtype))
+        ctx.outlasts_host = _outlasts_host(N, d, weight.shape[0])
         return loss_rows.sum() / total
 
     @staticmethod
     def backward(ctx, dout):
-        dx, dw = ctx.saved_tensors
-        return _scaled(dx, dout), None, _scaled(dw, dout), None, None
+        dx, dw = (_scaled(t, dout, ctx.outlasts_host) for t in ctx.saved_tensors)
+        return dx, None, dw, None, None
 
 
 def fused_linear_cross_entropy(x, target, weight, num_chunks: int = 8, ignore_index: int = -100):

@@ -5,6 +5,7 @@ dx, dW) over several chunkings."""
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from archbench_amd import fused_ce, ops
 from oracle import ce_oracle as CE
@@ -73,8 +74,10 @@ def test_fused_linear_ce_matches_oracle(num_chunks, V):
     (257, 64, 1000, 4),    # a vocabulary that allows no parts
     (90, 512, 16384, 1),   # one pass; dx in sixteen parts
 ])
-def test_fused_linear_ce_passes_and_parts(N, H, V, num_chunks):
-    """The rows per pass, the accumulation of dW across passes and the parts of dx against the oracle."""
+def test_fused_linear_ce_passes_and_parts(monkeypatch, N, H, V, num_chunks):
+    """The rows per pass, the accumulation of dW across passes and the parts of dx (which calls this small would not
+    take by themselves) against the oracle."""
+    monkeypatch.setattr(fused_ce, "_outlasts_host", lambda *a: True)
     rows = fused_ce._rows_per_pass(N, num_chunks, H, 2)
     banner(f"fused linear CE N={N} H={H} V={V}: {rows} rows per pass, {fused_ce._dx_split(rows, H, V)} parts")
     gen = torch.Generator().manual_seed(N)
@@ -92,10 +95,11 @@ def test_fused_linear_ce_passes_and_parts(N, H, V, num_chunks):
 
 
 @pytest.mark.parametrize("num_chunks", [1, 8])
-def test_fused_linear_ce_feature_major_x(num_chunks):
+def test_fused_linear_ce_feature_major_x(monkeypatch, num_chunks):
     """Hidden states laid out feature by feature (a dense transposed x, whose gradient has its strides), at a size whose
     dx may be taken in parts: the same result as for the row-major copy to the rounding of dx."""
     banner(f"fused linear CE feature-major x chunks={num_chunks}")
+    monkeypatch.setattr(fused_ce, "_outlasts_host", lambda *a: True)
     N, H, V = 1100, 128, 8192
     gen = torch.Generator().manual_seed(3)
     x = torch.randn(1, H, N, generator=gen).bfloat16().cuda().transpose(1, 2)
@@ -146,6 +150,45 @@ def test_fused_linear_ce_fp16_weight_under_autocast(num_chunks):
     _, dx_r, dw_r = CE.linear_ce(x.float().reshape(-1, H), t.reshape(-1), w.float())
     assert wd.grad.dtype == torch.float16 and rel_l2(wd.grad, 1024 * dw_r) <= 1e-2
     assert rel_l2(xd.grad.reshape(-1, H), 1024 * dx_r) <= 1e-2
+
+
+class _Calls(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("N,H,V,parts", [(128, 384, 8192, False), (1024, 1024, 8192, False), (256, 512, 32000, False),
+                                         (128, 1024, 50304, True), (1024, 512, 32000, True)])
+def test_fused_linear_ce_one_pass_calls(N, H, V, parts):
+    """A call that waits for its launches makes the fewest: three products, the loss and torch's scaling of both
+    gradients; one whose kernels outlast them takes dx in parts and the HIP scaling."""
+    banner(f"fused linear CE one pass N={N} H={H} V={V}")
+    gen = torch.Generator("cuda").manual_seed(N)
+    x = torch.randn(1, N, H, device="cuda", generator=gen).bfloat16().requires_grad_()
+    w = (torch.randn(V, H, device="cuda", generator=gen) * 0.05).bfloat16().requires_grad_()
+    t = torch.randint(0, V, (1, N), device="cuda", generator=gen)
+    with _Calls() as calls:
+        fused_ce.fused_linear_cross_entropy(x, t, w, num_chunks=1).backward()
+    n = [sum(k in c for c in calls.names) for k in ("aten.mm", "aten.bmm", "archbench_amd", "aten.copy_", "aten.mul")]
+    assert n == ([2, 1, 4, 0, 0] if parts else [3, 0, 1, 0, 2]), calls.names
+
+
+@pytest.mark.parametrize("hip", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_scaled_gradients(dtype, hip):
+    """Both ways of scaling a stored gradient give the fp32 product rounded once, and differentiate under create_graph."""
+    banner(f"scaled gradient {dtype} hip={hip}")
+    x = torch.randn(33, 8, device="cuda", generator=torch.Generator("cuda").manual_seed(7)).to(dtype)
+    s = torch.tensor(1 / 3, device="cuda", requires_grad=True)
+    with torch.no_grad():
+        assert torch.equal(fused_ce._scaled(x, s, hip), (x.float() * s).to(dtype))
+    y = fused_ce._scaled(x.requires_grad_(), s, hip)
+    assert all(g is not None for g in torch.autograd.grad(y.float().sum(), (x, s)))
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
