@@ -31,39 +31,35 @@ import torch.nn.functional as F
 from .. import ops
 
 
-def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """dW = dy^T x (dy [M, N], x [M, K]) in fp32, split over the M tokens: a batch of chunk products summed in fp32.
+def _weight_grad_(dw: torch.Tensor, r0: int, dy: torch.Tensor, x: torch.Tensor) -> None:
+    """dW = dy^T x (dy [M, N], x [M, K]) in fp32 into rows r0 .. r0 + N - 1 of dw (a freshly allocated fp32 gradient),
+    split over the M tokens: a batch of chunk products summed in fp32.
     A weight gradient reduces over every token into a small N x K output; as one GEMM it has too few output tiles
     to fill the GPU (hipBLASLt at M = 65536: 131 us for N = 8, K = 512; 248 us for N = 512, K = 1024; 400 us for
     N = 3072, K = 512), split 8 or 16 ways 27, 77 and 211 us.  The smaller operand's chunks enter the batched
     product as the transposed left operand (a layout the GEMM reads directly; copying them transposed first cost
-    140 us at these sizes); the right operand is always contiguous."""
-    dw = torch.empty(dy.shape[1], x.shape[1], dtype=torch.float32, device=dy.device)
-    _weight_grad_(dw, dy, x)
-    return dw
-
-
-def _weight_grad_(dw: torch.Tensor, dy: torch.Tensor, x: torch.Tensor) -> None:
-    """_weight_grad into dw (contiguous rows of a larger gradient): a single product writes there itself, the chunk
-    products are summed there by one HIP pass, transposed where they were taken as x^T dy (a sum and a
-    transposing copy took 26 us for N = 2048, K = 512, the pass 12)."""
+    140 us at these sizes); the right operand is always contiguous.  A single product writes the rows itself; the chunk
+    products are summed there by one HIP pass, transposed where they were taken as x^T dy (a sum and a transposing
+    copy took 26 us for N = 2048, K = 512, the pass 12)."""
     M, N = dy.shape
     K = x.shape[1]
     C = 16 if N * K <= 1 << 20 else 8
-    own = dy.is_cuda and not torch.is_grad_enabled() and dw.is_contiguous() and dw.data_ptr() % 16 == 0
+    rows = dw[r0:r0 + N]
+    # in place where the rows begin 16-byte aligned (by their offset: an address cannot be traced)
+    own = dy.is_cuda and not torch.is_grad_enabled() and r0 * K % 4 == 0
     if dy.dtype == torch.float32:
-        dw.copy_(dy.t() @ x)
+        rows.copy_(dy.t() @ x)
     elif M % C or M // C < 1024:
         if own:
-            torch.mm(dy.t(), x, out_dtype=torch.float32, out=dw)
+            torch.mm(dy.t(), x, out_dtype=torch.float32, out=rows)
         else:
-            dw.copy_(torch.mm(dy.t(), x, out_dtype=torch.float32))
+            rows.copy_(torch.mm(dy.t(), x, out_dtype=torch.float32))
     elif N <= K:
         parts = torch.bmm(dy.view(C, M // C, N).transpose(1, 2), x.view(C, M // C, K), out_dtype=torch.float32)
-        ops.sum_parts_(parts, dw) if own and N * K % 8 == 0 else dw.copy_(parts.sum(0))
+        ops.sum_parts_(parts, rows) if own and N * K % 8 == 0 else rows.copy_(parts.sum(0))
     else:
         parts = torch.bmm(x.view(C, M // C, K).transpose(1, 2), dy.view(C, M // C, N), out_dtype=torch.float32)
-        ops.sum_parts_t_(parts, dw) if own and N % 4 == 0 and K % 4 == 0 else dw.copy_(parts.sum(0).t())
+        ops.sum_parts_t_(parts, rows) if own and N % 4 == 0 and K % 4 == 0 else rows.copy_(parts.sum(0).t())
 
 
 class _GroupedLinear(torch.autograd.Function):
@@ -105,7 +101,7 @@ class _GroupedLinear(torch.autograd.Function):
             dw = torch.empty(wc.shape, dtype=torch.float32, device=wc.device)
             for r0, r1, dy in [(0, ctx.bounds[0], None), *groups, (ctx.bounds[-1], wc.shape[0], None)]:
                 if dy is not None:
-                    _weight_grad_(dw[r0:r1], dy, x2)
+                    _weight_grad_(dw, r0, dy, x2)
                 elif r1 > r0:
                     dw[r0:r1].zero_()
             dw = dw.to(ctx.w_dtype)

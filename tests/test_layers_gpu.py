@@ -274,21 +274,53 @@ def test_layer_under_torch_compile():
         assert rel_l2(gp1[n], gp0[n]) <= 2e-2, n
 
 
-@pytest.mark.parametrize("N,K", [(8, 512), (512, 1024), (3072, 512), (24, 40)])
+@pytest.mark.parametrize("arch,B,T", [("gdn", 2, 100), ("gdn", 16, 1024), ("nsgdn", 2, 100)])
+def test_mixer_compiles_whole(arch, B, T):
+    """A mixer's training step under bf16 autocast is one graph (torch.compile(fullgraph=True)), its projections' backward
+    included, with the gradients products single (T = 100) and split over the tokens (16384 of them): the same bits as
+    eager."""
+    banner(f"{arch} mixer under torch.compile(fullgraph=True) B={B} T={T}")
+    torch.manual_seed(0)
+    kw = dict(n_steps=2, lam=1.0) if arch == "nsgdn" else {}
+    m = layers.build_mixer(arch, 256, 0, 2, num_heads=2, head_dim=128, expand_v=2.0, **kw).cuda()
+    x = torch.randn(B, T, 256, device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+
+    def run(fn):
+        m.zero_grad(set_to_none=True)
+        xi = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = fn(xi)
+        y.float().square().sum().backward()
+        return [y, xi.grad] + [p.grad for p in m.parameters()]
+
+    def fn(x):
+        return m(x)
+
+    ref = run(fn)
+    torch._dynamo.reset()
+    for a, b in zip(run(torch.compile(fn, dynamic=False, fullgraph=True, backend="aot_eager")), ref):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("N,K", [(8, 512), (512, 1024), (3072, 512), (24, 40), (6, 35), (1030, 130)])
 def test_split_weight_gradient(N, K):
     """The layer's weight gradient split over the tokens equals dy^T x to fp32 accumulation (both operand orders,
     and the single-product fallback for short inputs), and the layer's linear backward returns it in the
     weight's dtype."""
-    from archbench_amd.layers.gdn import _linear, _weight_grad
+    from archbench_amd.layers.gdn import _linear, _weight_grad_
     banner(f"split weight gradient N={N} K={K}")
     M = 16384 if N != 24 else 1000
     gen = torch.Generator("cuda").manual_seed(7)
     dy = torch.randn(M, N, device="cuda", generator=gen).to(torch.bfloat16)
     x = torch.randn(M, K, device="cuda", generator=gen).to(torch.bfloat16)
     ref = dy.double().t() @ x.double()
-    got = _weight_grad(dy, x)
-    assert got.dtype == torch.float32 and got.shape == (N, K)
-    assert rel_l2(got.double(), ref) <= 1e-5
+    for r0 in (0, 3, 8):  # rows of a larger gradient, the others untouched; without grad as in training, and with it
+        for grad in (False, True):
+            dw = torch.full((N + 16, K), 7.0, device="cuda")
+            with torch.set_grad_enabled(grad):
+                _weight_grad_(dw, r0, dy, x)
+            assert rel_l2(dw[r0:r0 + N].double(), ref) <= 1e-5, (r0, grad)
+            assert (dw[:r0] == 7).all() and (dw[r0 + N:] == 7).all()
     w = torch.randn(N, K, device="cuda", generator=gen).requires_grad_()
     xa = x.clone().requires_grad_()
     y = _linear(xa, w)
