@@ -44,7 +44,7 @@ def _weight_grad_(dw: torch.Tensor, r0: int, dy: torch.Tensor, x: torch.Tensor) 
     M, N = dy.shape
     K = x.shape[1]
     C = 16 if N * K <= 1 << 20 else 8
-    rows = dw[r0:r0 + N]
+    rows = _rows(dw, r0, r0 + N)
     # in place where the rows begin 16-byte aligned (by their offset: an address cannot be traced)
     own = dy.is_cuda and not torch.is_grad_enabled() and r0 * K % 4 == 0
     if dy.dtype == torch.float32:
@@ -68,22 +68,32 @@ class _GroupedLinear(torch.autograd.Function):
     accumulated in place into the first (dx += dy_g W_g in the GEMM, no separate sum), the last group's, when it has a
     few columns only (a and b), together with the cast to x's dtype (ops.narrow_dx), and each group's weight gradient
     split over the tokens (_weight_grad_) written into its rows of one fp32 gradient (rows outside every group: zero),
-    returned in W's dtype."""
+    returned in W's dtype.  The casts are outputs too, after the groups': saved as such they have a history, so under
+    create_graph the gradients' own dependence on x and W is differentiated (casts recorded outside the function cost the
+    host of a mixer's training step 20 us)."""
 
     @staticmethod
     def forward(ctx, x: torch.Tensor, w: torch.Tensor, bounds: tuple, dtype: torch.dtype):
-        ctx.x_dtype = x.dtype
-        x = x.to(dtype)
-        wc = w.to(dtype)
-        ctx.save_for_backward(x, wc)
-        ctx.bounds, ctx.w_dtype = bounds, w.dtype
-        return tuple(F.linear(x, wc[r0:r1]) for r0, r1 in zip(bounds[:-1], bounds[1:]))
+        xc, wc = x.to(dtype), w.to(dtype)
+        ctx.save_for_backward(xc, wc)
+        ctx.set_materialize_grads(False)
+        ctx.bounds, ctx.x_dtype, ctx.w_dtype = bounds, x.dtype, w.dtype
+        out = [F.linear(xc, _rows(wc, r0, r1)) for r0, r1 in zip(bounds, bounds[1:])]
+        ctx.casts = []
+        if xc is not x:
+            ctx.casts.append(0)
+            out.append(xc)
+        if wc is not w:
+            ctx.casts.append(1)
+            out.append(wc)
+        return tuple(out)
 
     @staticmethod
     def backward(ctx, *dys):
         x, wc = ctx.saved_tensors
+        bounds = ctx.bounds
         groups = [(r0, r1, None if dy is None else dy.reshape(-1, dy.shape[-1]))
-                  for r0, r1, dy in zip(ctx.bounds[:-1], ctx.bounds[1:], dys)]
+                  for r0, r1, dy in zip(bounds, bounds[1:], dys)]
         x2 = x.reshape(-1, x.shape[-1])
         dx = dw = None
         if ctx.needs_input_grad[0]:
@@ -91,7 +101,7 @@ class _GroupedLinear(torch.autograd.Function):
                 if dy is None:
                     continue
                 if dx is None:
-                    dx = dy @ wc[r0:r1]
+                    dx = dy @ _rows(wc, r0, r1)
                 elif i == len(groups) - 1 and _narrow_dx_applies(dx, dy, ctx.x_dtype):
                     dx = ops.narrow_dx(dx, dy, wc[r0:r1], ctx.x_dtype == torch.float32)
                 else:
@@ -99,13 +109,26 @@ class _GroupedLinear(torch.autograd.Function):
             dx = torch.zeros_like(x, dtype=ctx.x_dtype) if dx is None else dx.to(ctx.x_dtype).view(x.shape)
         if ctx.needs_input_grad[1]:
             dw = torch.empty(wc.shape, dtype=torch.float32, device=wc.device)
-            for r0, r1, dy in [(0, ctx.bounds[0], None), *groups, (ctx.bounds[-1], wc.shape[0], None)]:
+            for r0, r1, dy in groups:
                 if dy is not None:
                     _weight_grad_(dw, r0, dy, x2)
-                elif r1 > r0:
+                else:
+                    dw[r0:r1].zero_()
+            for r0, r1 in ((0, bounds[0]), (bounds[-1], wc.shape[0])):
+                if r1 > r0:
                     dw[r0:r1].zero_()
             dw = dw.to(ctx.w_dtype)
+        if len(dys) > len(groups):  # the casts' gradients, under create_graph only
+            grads = [dx, dw]
+            for i, d in zip(ctx.casts, dys[len(groups):]):
+                if d is not None and grads[i] is not None:
+                    grads[i] = grads[i] + d.to(grads[i].dtype)
+            dx, dw = grads
         return dx, dw, None, None
+
+
+def _rows(w: torch.Tensor, r0: int, r1: int) -> torch.Tensor:
+    return w if r0 == 0 and r1 == w.shape[0] else w[r0:r1]
 
 
 def _narrow_dx_applies(dx: torch.Tensor, dy: torch.Tensor, x_dtype: torch.dtype) -> bool:
@@ -122,7 +145,7 @@ def _grouped_linear(x: torch.Tensor, w: torch.Tensor, bounds, dtype: torch.dtype
     bounds = tuple(int(r) for r in bounds)
     dtype = x.dtype if dtype is None else dtype
     if x.is_cuda:
-        return _GroupedLinear.apply(x, w, bounds, dtype)
+        return _GroupedLinear.apply(x, w, bounds, dtype)[:len(bounds) - 1]
     x, wc = x.to(dtype), w.to(dtype)
     return tuple(F.linear(x, wc[r0:r1]) for r0, r1 in zip(bounds[:-1], bounds[1:]))
 

@@ -175,3 +175,26 @@ def test_in_place_row_layouts_of_projection_slices():
     assert (ldg, gpl) == (0, 1)
     g, ldg, gpl = ops._gate_lines(gate.transpose(2, 3).contiguous().transpose(2, 3), dim)  # dim not contiguous
     assert (ldg, gpl) == (0, 1) and g.is_contiguous()
+
+
+@pytest.mark.parametrize("x_dtype,w_dtype,dtype", [(torch.float64, torch.float64, torch.float32),
+                                                   (torch.float32, torch.float64, torch.float32),
+                                                   (torch.float32, torch.float32, torch.float32)])
+def test_grouped_linear_second_derivatives(x_dtype, w_dtype, dtype):
+    """Under create_graph the grouped projections' gradients depend on x and W as a plain linear's do, also where either
+    is cast to the computing dtype (fp32 sums: 1e-5)."""
+    from archbench_amd.layers.gdn import _GroupedLinear
+    gen = torch.Generator().manual_seed(0)
+    x = torch.randn(3, 5, 8, generator=gen, dtype=torch.float64).to(x_dtype).requires_grad_()
+    w = torch.randn(12, 8, generator=gen, dtype=torch.float64).to(w_dtype).requires_grad_()
+    bounds = (0, 4, 8, 10)  # the last two rows in no group
+
+    def second(ys):
+        gx, gw = torch.autograd.grad(sum((y.double() ** 3).sum() for y in ys), (x, w), create_graph=True)
+        return [gx, gw, *torch.autograd.grad((gx.double() ** 2).sum() + 1.5 * (gw.double() ** 2).sum(), (x, w))]
+
+    got = second(_GroupedLinear.apply(x, w, bounds, dtype)[:3])
+    xd, wd = x.double(), w.double()
+    ref = second([xd @ wd[r0:r1].t() for r0, r1 in zip(bounds[:-1], bounds[1:])])
+    for a, b in zip(got, ref):
+        assert a.dtype == b.dtype and (a - b).norm() <= 1e-5 * b.norm()
