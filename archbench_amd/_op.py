@@ -20,11 +20,15 @@ _libs: dict[str, torch.library.Library] = {}  # owner of each op's registrations
 
 
 def _autograd_kernel(op, name: str, backward, setup_context):
+    # the dispatcher drops trailing arguments that equal their defaults; setup_context sees them all
+    n_args = len(op._schema.arguments)
+    defaults = tuple(a.default_value for a in op._schema.arguments)
+
     def forward(ctx, *args):
         with _BelowAutograd():
             out = op(*args)
         if setup_context is not None:
-            setup_context(ctx, args, out)
+            setup_context(ctx, args if len(args) == n_args else args + defaults[len(args):], out)
         return out
 
     def no_formula(ctx, *grads):
@@ -44,14 +48,27 @@ def _autograd_kernel(op, name: str, backward, setup_context):
     return kernel
 
 
+def _check_schema(name: str, schema) -> None:
+    """Refuses what the kernels here do not handle: keyword-only arguments and lists of tensors."""
+    for a in schema.arguments:
+        if a.kwarg_only or ("Tensor" in str(a.type) and str(a.type) not in ("Tensor", "Optional[Tensor]")):
+            raise ValueError(f"{name}: argument {a.name} ({a.type}) is keyword-only or a list of tensors; "
+                             "register it with torch.library.custom_op")
+    for r in schema.returns:
+        if str(r.type) != "Tensor":
+            raise ValueError(f"{name}: returns {r.type}; register it with torch.library.custom_op")
+
+
 def gpu_op(name: str):
     """Decorator: registers the function as the op ``name`` ("namespace::op")."""
     ns, opname = name.split("::")
 
     def wrap(impl):
+        schema = opname + torch.library.infer_schema(impl, mutates_args=())
+        _check_schema(name, torch._C.parse_schema(schema))
         _libs.pop(name, None)
         lib = _libs[name] = torch.library.Library(ns, "FRAGMENT")
-        lib.define(opname + torch.library.infer_schema(impl, mutates_args=()), tags=(torch.Tag.pt2_compliant_tag,))
+        lib.define(schema, tags=(torch.Tag.pt2_compliant_tag,))
         # not traced into where a compiled program calls the op between two graphs
         lib.impl(opname, torch._disable_dynamo(impl), "CompositeExplicitAutograd")
         op = getattr(getattr(torch.ops, ns), opname).default

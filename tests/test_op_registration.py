@@ -2,6 +2,8 @@
 inputs only), no gradient, saved-tensor hooks, dispatch modes, fake tensors, make_fx, vmap, forward mode, functorch's grad,
 a missing autograd formula and a compiled call behave alike."""
 
+from typing import Optional
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fw
@@ -44,6 +46,29 @@ def _make(kind):
     return f, b
 
 
+def _make_default(kind):
+    deco = gpu_op if kind == "gpu_op" else lambda n: torch.library.custom_op(n, mutates_args=())
+
+    @deco(f"archbench_test::{kind}_d")
+    def d(x: Tensor, y: Tensor | None = None, c: float = 3.0, n: int = 2) -> Tensor:
+        return x * c * n if y is None else x * y * c * n
+
+    d.register_fake(lambda x, y=None, c=3.0, n=2: torch.empty_like(x))
+
+    def setup(ctx, inputs, output):
+        x, y, ctx.c, ctx.n = inputs
+        ctx.save_for_backward(x, y)
+
+    def backward(ctx, g):
+        x, y = ctx.saved_tensors
+        f = ctx.c * ctx.n
+        return (g * f if y is None else g * y * f), (None if y is None else g * x * f), None, None
+
+    d.register_autograd(backward, setup_context=setup)
+    return d
+
+
+DEFAULTS = {k: _make_default(k) for k in ("gpu_op", "custom_op")}
 OPS = {k: _make(k) for k in ("gpu_op", "custom_op")}
 
 
@@ -139,3 +164,35 @@ def test_gpu_op_behaves_like_custom_op(check):
     assert len(got) == len(ref)
     for a, r in zip(got, ref):
         assert torch.equal(a, r) if isinstance(r, Tensor) else a == r, (a, r)
+
+
+@pytest.mark.parametrize("args,kw", [((), {}), (("y",), {}), ((None,), {"n": 2}), ((), {"c": 3.0}), ((), {"n": 5}),
+                                     (("y", 4.0, 5), {}), ((None, 3.0), {"n": 7})])
+def test_default_arguments(args, kw):
+    """Arguments left at (or equal to) their defaults, in front of given ones or not, reach setup_context."""
+    out = []
+    for d in DEFAULTS.values():
+        x, y = _leaves()
+        r = d(x, *(y if a == "y" else a for a in args), **kw)
+        r.sum().backward()
+        out.append([r, x.grad] + [y.grad] * ("y" in args))
+    for a, r in zip(*out):
+        assert torch.equal(a, r)
+
+
+def test_unsupported_signatures_are_refused():
+    def kw_only(x: Tensor, *, c: float) -> Tensor:
+        return x * c
+
+    def tensor_list(xs: list[Tensor]) -> Tensor:
+        return xs[0].clone()
+
+    def optional_list(x: Tensor, ys: list[Optional[Tensor]]) -> Tensor:
+        return x.clone()
+
+    def returns_list(x: Tensor) -> list[Tensor]:
+        return [x.clone()]
+
+    for f in (kw_only, tensor_list, optional_list, returns_list):
+        with pytest.raises(ValueError, match="custom_op"):
+            gpu_op(f"archbench_test::{f.__name__}")(f)
