@@ -48,6 +48,8 @@ SIGNATURES = {
     "gdn_short_conv_bwd": (_i, [_p, _i64, _p, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _sz, _i, _i, _i, _i, _i, _i,
                                 _p]),
     "gdn_mixer_stage_fwd": (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
+    "gdn_mixer_stage_fwd_ld": (_i, [_p, _i64, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p]),
+    "gdn_mixer_stage_bwd_ld": (_i, [_p, _i64, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i, _i, _i, _i, _i, _p]),
     "gdn_mixer_stage_bwd_ws_bytes": (_i, [_i, _i, _i, _i, _i, ctypes.POINTER(_sz)]),
     "gdn_mixer_stage_bwd": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i, _i, _i, _i, _i, _p]),
     "gdn_gated_rmsnorm_fwd": (_i, [_p, _p, _i64, _i, _p, _p, _i64, _i, _f, _i, _p]),

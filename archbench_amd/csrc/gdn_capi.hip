@@ -702,25 +702,34 @@ int gdn_short_conv_bwd(const void* x, int64_t ldx, const float* w, const float* 
 }
 
 // The mixer's input stage: key_dim columns for q, key_dim for k (both normalised), value_dim for v
-static int stage_check(int B, int T, int key_dim, int value_dim, int W, int norm_group, int dtype) {
+static int stage_check(int B, int T, int key_dim, int value_dim, int64_t ldy, int W, int norm_group, int dtype) {
   if (key_dim <= 0 || value_dim <= 0)
     return fail(GDN_ERR_ARG, "invalid key_dim=%d value_dim=%d", key_dim, value_dim);
   if ((int64_t)2 * key_dim + value_dim > INT32_MAX / 8) return fail(GDN_ERR_ARG, "too many channels");
   const int D = 2 * key_dim + value_dim;
-  if (int e = conv_check(B, T, key_dim, D, W, norm_group, dtype, "2 key_dim + value_dim")) return e;
-  return conv_check(B, T, value_dim, D, W, 0, dtype, "2 key_dim + value_dim");
+  const char* ld = ldy ? "ldy" : "2 key_dim + value_dim";
+  if (ldy && ldy < D) return fail(GDN_ERR_ARG, "ldy = %lld must be >= 2 key_dim + value_dim = %d", (long long)ldy, D);
+  if (ldy == 0) ldy = D;
+  if (int e = conv_check(B, T, key_dim, ldy, W, norm_group, dtype, ld)) return e;
+  return conv_check(B, T, value_dim, ldy, W, 0, dtype, ld);
 }
 
 int gdn_mixer_stage_fwd(const void* y, const float* w, void* q, void* k, void* v, int B, int T, int key_dim,
                         int value_dim, int W, int norm_group, int dtype, void* stream) {
+  return gdn_mixer_stage_fwd_ld(y, 0, w, q, k, v, B, T, key_dim, value_dim, W, norm_group, dtype, stream);
+}
+
+int gdn_mixer_stage_fwd_ld(const void* y, int64_t ldy, const float* w, void* q, void* k, void* v, int B, int T,
+                           int key_dim, int value_dim, int W, int norm_group, int dtype, void* stream) {
   g_err[0] = 0;
-  if (int e = stage_check(B, T, key_dim, value_dim, W, norm_group, dtype)) return e;
+  if (int e = stage_check(B, T, key_dim, value_dim, ldy, W, norm_group, dtype)) return e;
   if (B == 0 || T == 0) return GDN_OK;
   if (!y || !w || !q || !k || !v) return fail(GDN_ERR_ARG, "null input/output pointer");
   if (misaligned(y, w, q, k, v)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
   ConvArgs a{};
   a.x = y; a.w = w; a.y[0] = q; a.y[1] = k; a.y[2] = v;
-  a.B = B; a.T = T; a.n[0] = a.n[1] = key_dim; a.n[2] = value_dim; a.normed = 2; a.ldx = 2 * key_dim + value_dim;
+  a.B = B; a.T = T; a.n[0] = a.n[1] = key_dim; a.n[2] = value_dim; a.normed = 2;
+  a.ldx = ldy ? ldy : 2 * key_dim + value_dim;
   a.norm_group = norm_group; a.dtype = dtype; a.stream = static_cast<hipStream_t>(stream);
   const hipError_t e = timed(ST_CONV_FWD, a.stream, [&] { return launch_conv(a, false); });
   if (e != hipSuccess) return fail(GDN_ERR_LAUNCH, "mixer input stage forward launch: %s", hipGetErrorString(e));
@@ -732,7 +741,7 @@ int gdn_decode_proj_supported(int B, int d) { return decode_proj_supported(B, d)
 int gdn_mixer_decode_stage(const gdn_decode_stage_args* s, void* stream) {
   g_err[0] = 0;
   if (!s) return fail(GDN_ERR_ARG, "args is NULL");
-  if (int e = stage_check(s->B, 1, s->key_dim, s->value_dim, s->W, s->norm_group, DT_BF16)) return e;
+  if (int e = stage_check(s->B, 1, s->key_dim, s->value_dim, 0, s->W, s->norm_group, DT_BF16)) return e;
   if (s->norm_group == 0) return fail(GDN_ERR_SHAPE, "norm_group must be 64, 128 or 256");
   for (int dt : {s->w_dtype, s->conv_w_dtype, s->gate_dtype})
     if (dt != DT_F32 && dt != DT_BF16) return fail(GDN_ERR_ARG, "dtype code %d is not GDN_DTYPE_F32/BF16", dt);
@@ -797,8 +806,15 @@ int gdn_mixer_stage_bwd_ws_bytes(int B, int T, int key_dim, int value_dim, int W
 int gdn_mixer_stage_bwd(const void* y, const float* w, const void* dq, const void* dk, const void* dv, void* dy,
                         float* dw, void* ws, size_t ws_bytes, int B, int T, int key_dim, int value_dim, int W,
                         int norm_group, int dtype, void* stream) {
+  return gdn_mixer_stage_bwd_ld(y, 0, w, dq, dk, dv, dy, dw, ws, ws_bytes, B, T, key_dim, value_dim, W, norm_group,
+                                dtype, stream);
+}
+
+int gdn_mixer_stage_bwd_ld(const void* y, int64_t ldy, const float* w, const void* dq, const void* dk, const void* dv,
+                           void* dy, float* dw, void* ws, size_t ws_bytes, int B, int T, int key_dim, int value_dim,
+                           int W, int norm_group, int dtype, void* stream) {
   g_err[0] = 0;
-  if (int e = stage_check(B, T, key_dim, value_dim, W, norm_group, dtype)) return e;
+  if (int e = stage_check(B, T, key_dim, value_dim, ldy, W, norm_group, dtype)) return e;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int D = 2 * key_dim + value_dim;
   if (B == 0 || T == 0) {
@@ -810,7 +826,8 @@ int gdn_mixer_stage_bwd(const void* y, const float* w, const void* dq, const voi
   if (misaligned(y, w, dq, dk, dv, dy, dw, ws)) return fail(GDN_ERR_ARG, "array pointer not 16-byte aligned");
   ConvArgs a{};
   a.x = y; a.w = w; a.dy[0] = dq; a.dy[1] = dk; a.dy[2] = dv; a.dx = dy; a.dw = dw; a.ws = ws;
-  a.B = B; a.T = T; a.n[0] = a.n[1] = key_dim; a.n[2] = value_dim; a.normed = 2; a.ldx = a.lddx = D;
+  a.B = B; a.T = T; a.n[0] = a.n[1] = key_dim; a.n[2] = value_dim; a.normed = 2;
+  a.ldx = ldy ? ldy : D; a.lddx = D;
   a.norm_group = norm_group; a.dtype = dtype; a.stream = st;
   const size_t need = conv_ws_bytes(B, T, a.n, W);
   if (!ws || ws_bytes < need)

@@ -822,10 +822,18 @@ def _(x, w_in, conv_w, conv_state, A_log, dt_bias, norm_group, beta_scale, g_min
 
 
 # The mixer's input stage in one op: q, k and v convolved straight out of the q/k/v input projection's output y
-# [B, T, 2 key_dim + value_dim] (its column groups, read in place), with one weight [2 key_dim + value_dim, W] for
+# [B, T, 2 key_dim + value_dim] (its column groups, read in place, also where y is a column slice), with one weight [2 key_dim + value_dim, W] for
 # the three convolutions (q's rows, then k's, then v's), in one launch.  The backward, one launch and the sum of its
 # partial weight gradients, writes the three input gradients into the column groups of one dy and the weight gradients
 # into one dw, so no gradient of a split or of a concatenation costs a pass.
+def _stage_rows(y: Tensor) -> tuple[Tensor, int]:
+    """y as (tensor, row stride); a stride past the kernels' 32-bit row offsets is copied away."""
+    rows, ld = _token_rows(y)
+    if y.shape[1] * ld * y.element_size() >= 1 << 31 and ld > y.shape[2]:
+        return _arg(y), y.shape[2]
+    return rows, ld
+
+
 def _stage_dims(y: Tensor, w: Tensor, key_dim: int, value_dim: int):
     n = 2 * key_dim + value_dim
     if y.dim() != 3 or y.shape[-1] != n:
@@ -843,10 +851,10 @@ def mixer_input_stage(y: Tensor, w: Tensor, key_dim: int, value_dim: int,
     _require_gpu(y, w)
     B, T, _, W = _stage_dims(y, w, key_dim, value_dim)
     lib = _lib.load()
-    y, w = _arg(y), _arg(w, torch.float32)
+    (y, ldy), w = _stage_rows(y), _arg(w, torch.float32)
     q, k, v = y.new_empty(B, T, key_dim), y.new_empty(B, T, key_dim), y.new_empty(B, T, value_dim)
-    rc = lib.gdn_mixer_stage_fwd(_lib.ptr(y), _lib.ptr(w), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, T, key_dim,
-                                 value_dim, W, int(norm_group), _lib.dtype_code(y.dtype), _lib.stream_ptr(y.device))
+    rc = lib.gdn_mixer_stage_fwd_ld(_lib.ptr(y), ldy, _lib.ptr(w), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), B, T, key_dim,
+                                    value_dim, W, int(norm_group), _lib.dtype_code(y.dtype), _lib.stream_ptr(y.device))
     _lib.check(rc, "gdn_mixer_stage_fwd")
     return q, k, v
 
@@ -867,14 +875,14 @@ def mixer_input_stage_bwd(y: Tensor, w: Tensor, dq: Tensor, dk: Tensor, dv: Tens
         if tuple(g.shape) != (B, T, d):
             raise ValueError(f"{n} must be [B, T, {d}] = {(B, T, d)}, got {tuple(g.shape)}")
     lib = _lib.load()
-    y, w = _arg(y), _arg(w, torch.float32)
+    (y, ldy), w = _stage_rows(y), _arg(w, torch.float32)
     dq, dk, dv = _arg(dq, y.dtype), _arg(dk, y.dtype), _arg(dv, y.dtype)
-    dy = torch.empty_like(y)
+    dy = y.new_empty(B, T, D)
     dw = torch.empty(D, W, dtype=torch.float32, device=w.device)
     ws = _lib.workspace(y.device, _lib.stage_ws_bytes(B, T, key_dim, value_dim, W))
-    rc = lib.gdn_mixer_stage_bwd(_lib.ptr(y), _lib.ptr(w), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(dy),
-                                 _lib.ptr(dw), _lib.ptr(ws), ws.numel(), B, T, key_dim, value_dim, W,
-                                 int(norm_group), _lib.dtype_code(y.dtype), _lib.stream_ptr(y.device))
+    rc = lib.gdn_mixer_stage_bwd_ld(_lib.ptr(y), ldy, _lib.ptr(w), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv),
+                                    _lib.ptr(dy), _lib.ptr(dw), _lib.ptr(ws), ws.numel(), B, T, key_dim, value_dim, W,
+                                    int(norm_group), _lib.dtype_code(y.dtype), _lib.stream_ptr(y.device))
     _lib.check(rc, "gdn_mixer_stage_bwd")
     return dy, dw
 

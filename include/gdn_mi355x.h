@@ -167,6 +167,13 @@ int gdn_mixer_stage_bwd_ws_bytes(int B, int T, int key_dim, int value_dim, int W
 int gdn_mixer_stage_bwd(const void* y, const float* w, const void* dq, const void* dk, const void* dv, void* dy,
                         float* dw, void* ws, size_t ws_bytes, int B, int T, int key_dim, int value_dim, int W,
                         int norm_group, int dtype, void* stream);
+/* The same with y's token rows ldy elements apart (0: contiguous; as ldx of gdn_short_conv_fwd), a column slice of a
+ * wider tensor read in place.  dy is contiguous. */
+int gdn_mixer_stage_fwd_ld(const void* y, int64_t ldy, const float* w, void* q, void* k, void* v, int B, int T,
+                           int key_dim, int value_dim, int W, int norm_group, int dtype, void* stream);
+int gdn_mixer_stage_bwd_ld(const void* y, int64_t ldy, const float* w, const void* dq, const void* dk, const void* dv,
+                           void* dy, float* dw, void* ws, size_t ws_bytes, int B, int T, int key_dim, int value_dim,
+                           int W, int norm_group, int dtype, void* stream);
 
 /* The mixer's input stage for one decoded token per sequence (T = 1, bf16 activations): the input projections, the three
  * short convolutions from their states (no bias; q and k normalised per norm_group in {64, 128, 256} channels; W = 4)

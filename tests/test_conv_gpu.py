@@ -205,6 +205,34 @@ def test_mixer_input_stage_equals_separate_convs(dtype):
         ops.mixer_input_stage(y[..., :-4], w, kd, vd, ng)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,off", [(130, 0), (3, 64), (65, 2)])
+def test_mixer_input_stage_reads_a_column_slice_in_place(dtype, T, off):
+    """y as a column slice of a wider projection output: the bits of the contiguous copy, forward and backward, with no
+    copy made of it (except from columns that are not 16-byte aligned)."""
+    banner(f"mixer input stage column slice dtype={dtype} T={T} off={off}")
+    B, kd, vd, ng, wide = 2, 128, 256, 64, 768
+    L = 2 * kd + vd
+    gen = torch.Generator().manual_seed(12)
+    y = torch.randn(B, T, wide, generator=gen).to("cuda", dtype)[..., off:off + L]
+    w = (torch.randn(L, W, generator=gen) * 0.5).cuda()
+    grads = [torch.randn(B, T, d, generator=gen).to("cuda", dtype) for d in (kd, kd, vd)]
+    yc = y.contiguous()
+    ref = [*ops.mixer_input_stage(yc, w, kd, vd, ng), *ops.mixer_input_stage_bwd(yc, w, *grads, kd, vd, ng)]
+    peak = []
+    for t in (yc, y):  # the outputs of both passes, which are as large as y, and what else is taken
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        got = [*ops.mixer_input_stage(t, w, kd, vd, ng), *ops.mixer_input_stage_bwd(t, w, *grads, kd, vd, ng)]
+        peak.append(torch.cuda.max_memory_allocated() - before)
+        for a, b in zip(got, ref):
+            assert torch.equal(a, b) and a.is_contiguous()
+        del got
+    if off % 8 == 0:
+        assert peak[1] == peak[0]
+
+
 def test_conv_taps_rounded_to_activation_dtype():
     """With bf16 activations the kernels use the taps rounded to bf16 (as the reference's conv runs its fp32
     weight under bf16 autocast): an fp32 weight gives bit for bit what its bf16-rounded copy gives, forward and
