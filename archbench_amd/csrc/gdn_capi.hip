@@ -360,7 +360,8 @@ static hipError_t seg_forward_prefix(ChunkArgs& a, const float* h0) {
   hipError_t e = timed(ST_PREFIX, a.stream, [&] { return launch_fwd(p, FWD_PREFIX); });
   if (e == hipSuccess)
     e = timed(ST_SEGSCAN, a.stream, [&] {
-      return launch_seg_scan(a.ws.phi, a.ws.sloc, h0, a.ws.sin, a.B, a.ns, a.H, a.K, a.V, false, a.stream);
+      return launch_seg_scan(a.ws.phi, a.ws.sloc, h0, a.ws.sin, a.B, a.ns, a.H, a.K, a.V, a.dtype, false,
+                             a.stream);
     });
   a.h0 = a.ws.sin;
   return e;
@@ -471,7 +472,7 @@ static int chunk_bwd_impl(const void* q, const void* k, const void* u, const voi
     e = timed(ST_BWD_LOCAL, st, [&] { return launch_bwd_state(l, true); });
     if (e == hipSuccess)
       e = timed(ST_SEGSCAN, st, [&] {
-        return launch_seg_scan(a.ws.phi, a.ws.dsloc, dhT, a.ws.dsend, B, a.ns, H, K, V, true, st);
+        return launch_seg_scan(a.ws.phi, a.ws.dsloc, dhT, a.ws.dsend, B, a.ns, H, K, V, dtype, true, st);
       });
     a.dhT = a.ws.dsend;
   }

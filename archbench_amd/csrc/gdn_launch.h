@@ -99,7 +99,7 @@ struct SegPlan { int ns, cps; };
 SegPlan segment_plan(int B, int T, int H, int K, int V);
 // Carry states (reverse = false) or state gradients (reverse = true) across the segments of every (b, h).
 hipError_t launch_seg_scan(const float* phi, const float* loc, const float* init, float* outs, int B, int NS, int H,
-                           int K, int V, bool reverse, hipStream_t stream);
+                           int K, int V, int dtype, bool reverse, hipStream_t stream);
 bool chunk_shape_supported(int K, int V, int dtype);
 bool step_shape_supported(int K, int V);
 

@@ -157,6 +157,33 @@ def test_segments_of_any_length(B, T, H, K, V, dtype):
     assert all(e <= 1e-2 for e in errs.values()), errs
 
 
+def test_fp32_segments_add_no_error():
+    """In fp32 the scan across segments sums each product as a tree, so cutting a sequence (here into segments of four
+    chunks) puts its results no further from 64 bits than sweeping it whole does, as a batch too large to be cut is
+    (sums in two chains put o, dq and dv 0.7% further; the bound is 0.3%)."""
+    B, n, T, H, K, V = 65, 8, 2048, 1, 64, 64
+    banner(f"segmented fp32 errors B={n} T={T} H={H} K={K} V={V}")
+    host, dev = device_inputs(B, T, H, K, V, torch.float32, seed=63, with_do=True)
+
+    def run(m):
+        q, k, v, g, beta, do = (t[:m].contiguous() for t in (dev.q, dev.k, dev.v, dev.g, dev.beta, dev.do))
+        with _lib.StageTimer() as st:
+            o, _, stash = ops.chunk_fwd_stash(q, k, v, g, beta, None, 1.0)
+            got = ops.chunk_bwd_stashed(q, k, v, g, beta, None, do, None, stash, 1.0)
+        torch.cuda.synchronize()
+        return ("seg_scan" in st.result), [t[:n] for t in (o, *got[:3])]
+
+    (cut, seg), (whole_cut, whole) = run(n), run(B)
+    assert cut and not whole_cut
+    h = [t[:n] for t in (host.q, host.k, host.v, host.g, host.beta)]
+    o_r, _ = O.chunk_fwd(*h, 1.0, None)
+    ref = [o_r, *O.chunk_bwd(*h, host.do[:n], 1.0, None)[:3]]
+    for name, a, b, r in zip(("o", "dq", "dk", "dv"), seg, whole, ref):
+        ea, eb = rel_l2(a.double().cpu(), r.double()), rel_l2(b.double().cpu(), r.double())
+        print(f"[segmented fp32] {name}: {ea:.4e} cut, {eb:.4e} whole", flush=True)
+        assert ea <= 1.003 * eb, name
+
+
 @pytest.mark.parametrize("K,V,sep", [(64, 64, False), (64, 128, False), (64, 64, True), (64, 256, True),
                                      (128, 128, True), (128, 256, True)])
 def test_narrow_sweep_blocks_equal_wide(K, V, sep):
