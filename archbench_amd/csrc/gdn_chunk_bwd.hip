@@ -74,18 +74,28 @@ __global__ __launch_bounds__(state_threads<BV>()) __attribute__((amdgpu_waves_pe
   // per token: exp(G), exp(G_C - G) and -beta exp(G) (formed once per chunk by the first wave)
   __shared__ float sGam[CH], sDte[CH], sBGn[CH];
 
-  int vb, bh;
-  sweep_block(V / BV, gridDim.x * BV / V, vb, bh);
   // sequence b, segment seg, head h; the segment's chunks c_first .. c_end - 1 of the sequence (as in the forward sweep)
-  const int bs = bh / H, h = bh - bs * H;
-  const int b = bs / ns, seg = bs - b * ns;
+  int vb, bh, b, h, seg;
+  if constexpr (STORE) {
+    sweep_block(V / BV, gridDim.x * BV / V, vb, bh);
+    const int bs = bh / H;
+    h = bh - bs * H;
+    b = bs / ns;
+    seg = bs - b * ns;
+  } else {  // the segments but each sequence's first, evenly over the XCDs
+    const int nv = V / BV, rank = xcd_rank(gridDim.x), j = rank / nv, head = j / (ns - 1);
+    vb = rank - j * nv;
+    seg = 1 + j - head * (ns - 1);
+    b = head / H;
+    h = head - b * H;
+    bh = (b * ns + seg) * H + h;
+  }
   const int c_first = seg * cps, c_end = min(NT, c_first + cps);
   const int64_t seq = (int64_t)b * H + h;
-  // The local pass of a segmented sweep (STORE = false) skips each sequence's first segment (its entering-state
+  // The local pass of a segmented sweep (STORE = false) leaves out each sequence's first segment (its entering-state
   // gradient is the main sweep's dh0) and starts the last from the sequence's dhT, so that its result already
   // carries dhT.  dh0: per swept sequence in the local pass; otherwise, when segmented, only from the first
   // segment of each sequence, at the sequence's index.  dhT: per swept sequence in the main pass.
-  if (!STORE && seg == 0) return;  // uniform over the workgroup, before any barrier
   const bool put_dh0 = !STORE || seg == 0;
   const int64_t dh0_base = (!STORE ? (int64_t)bh : seq) * K * V;
   const bool use_dhT = dhT && (STORE || seg == ns - 1);
@@ -745,7 +755,7 @@ __global__ __launch_bounds__(ITH) void bwd_intra_kernel(
 // ---------------------------------------------------------------------------------------------------------
 template <typename T, int K, bool SEPU, int BV>
 static hipError_t bwd_state_bv(const ChunkArgs& a, bool local) {
-  dim3 grid(a.V / BV * a.B * a.ns * a.H);
+  dim3 grid(a.V / BV * a.B * (local ? a.ns - 1 : a.ns) * a.H);
   auto go = [&](auto kern) {
     kern<<<grid, state_threads<BV>(), 0, a.stream>>>(
         static_cast<const T*>(a.q), static_cast<const T*>(a.k), static_cast<const T*>(a.u),

@@ -76,23 +76,33 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
   // per token: beta, exp(G), exp(G_C - G), s exp(G) (formed once per chunk by the first wave)
   __shared__ float sB[CH], sGam[CH], sDte[CH], sGs[CH];
 
-  int vb, bh;
-  const int NVB = (V + (MODE == 3 ? K : 0)) / BV;  // column blocks per head
-  sweep_block(NVB, gridDim.x / NVB, vb, bh);
   // bh counts the segments of every head: sequence b, segment seg (of ns; ns = 1: not segmented), head h.  The
   // segment covers the sequence's chunks c_first .. c_end - 1 (cps each, the last segment possibly fewer); chunk c of
   // the sequence keeps its place in the per-chunk buffers, [B H][NT], whatever the segments
-  const int bs = bh / H, h = bh - bs * H;
-  const int b = bs / ns, seg = bs - b * ns;
+  int vb, bh, b, h, seg;
+  if constexpr (MODE == 3) {
+    // only the workgroups with work, evenly over the XCDs: of each head, the V blocks of the segments but the last and
+    // the K blocks (the transition's) of those between the first and the last
+    const int nv = V / BV, nb = nv + K / BV, rank = xcd_rank(gridDim.x), per = nv + (ns - 2) * nb;
+    const int head = rank / per, i = rank - head * per;
+    seg = i < nv ? 0 : 1 + (i - nv) / nb;
+    vb = i < nv ? i : i - nv - (seg - 1) * nb;
+    b = head / H;
+    h = head - b * H;
+    bh = (b * ns + seg) * H + h;
+  } else {
+    sweep_block(V / BV, gridDim.x / (V / BV), vb, bh);
+    const int bs = bh / H;
+    h = bh - bs * H;
+    b = bs / ns;
+    seg = bs - b * ns;
+  }
   const int c_first = seg * cps, c_end = min(NT, c_first + cps);
   const int64_t seq = (int64_t)b * H + h;
   // identity block (MODE 3): columns iv0 .. iv0 + BV - 1 of the transition; v reads nothing (no valid rows)
   const bool ident = MODE == 3 && vb * BV >= V;
   const int iv0 = vb * BV - V;
   const int v0 = ident ? 0 : vb * BV;
-  if constexpr (MODE == 3) {
-    if (seg == ns - 1 || (ident && seg == 0)) return;  // uniform over the workgroup, before any barrier
-  }
   // hT: per swept sequence in MODE 3 (the segments' local states); otherwise, when segmented, only from the last
   // segment of each sequence, at the sequence's index.  h0: in MODE 3 the sequence's own, for its first segment
   // only; otherwise per swept sequence (the entering state of every segment).
@@ -300,7 +310,8 @@ __global__ __launch_bounds__(fwd_threads<BV>()) __attribute__((amdgpu_waves_per_
 // ---------------------------------------------------------------------------------------------------------
 template <typename T, int K, int MODE, bool SEPU, int BV>
 static hipError_t fwd_sweep_bv(const ChunkArgs& a) {
-  dim3 grid((a.V + (MODE == 3 ? K : 0)) / BV * a.B * a.ns * a.H);
+  const int nv = a.V / BV;  // MODE 3: of ns >= 2 segments those with work
+  dim3 grid((MODE == 3 ? nv + (a.ns - 2) * (nv + K / BV) : nv * a.ns) * a.B * a.H);
   fwd_sweep_kernel<T, K, BV, MODE, SEPU><<<grid, fwd_threads<BV>(), 0, a.stream>>>(
       static_cast<const T*>(a.q), static_cast<const T*>(a.k), static_cast<const T*>(a.u),
       static_cast<const T*>(a.v), a.beta, a.h0,

@@ -223,6 +223,13 @@ __device__ __forceinline__ void sweep_block(int NV, int BH, int& vb, int& bh) {
   }
 }
 
+// Workgroup -> rank, for a 1-D grid of n workgroups of any number: XCD x (linear ids x modulo 8) takes consecutive ranks,
+// n / 8 or one more of them, so that neighbours share an L2 and every XCD has the same work.
+__device__ __forceinline__ int xcd_rank(int n) {
+  const int x = blockIdx.x & 7, s = blockIdx.x >> 3, more = n & 7;
+  return x * (n >> 3) + min(x, more) + s;
+}
+
 // Sum over the 16 lanes of a DPP row (the columns of one accumulator tile row set), left in every lane of the
 // row: butterfly on DPP, no LDS crossbar.  quad_perm [1,0,3,2] and [2,3,0,1] sum each quad, row_half_mirror
 // (lane i <- 7 - i) adds the other quad of the half-row, row_mirror (lane i <- 15 - i) the other half-row.
