@@ -173,8 +173,8 @@ struct TokStage {
 };
 
 // grid B * H * NB (NB = ceil(V / ROWS)) workgroups: workgroup x -> (b h, row block vb).  Tokens past the end of the
-// sequence in the last block are identity tokens (zero vectors, v = 0, la = 0), which leave S as it is; nothing is
-// stored for them.
+// sequence in the last block are identity tokens (zero vectors, v = 0, la = 0), which leave a finite S as it is; nothing
+// is stored for them.
 template <int K, typename SH>
 __global__ __launch_bounds__(SH::THREADS) void token_scan_fwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ u, const float* __restrict__ v,
@@ -303,6 +303,28 @@ __global__ __launch_bounds__(SH::THREADS) void token_scan_fwd_kernel(
     ts_barrier();  // the block's vectors read by every lane; the next block's staged
   }
   if (hT) {
+    // an infinite entry of S has become a NaN at the identity tokens (their S k is inf 0): such a wave steps from the last
+    // checkpoint to the end again with the r it stored
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < RL; ++i)
+#pragma unroll
+      for (int j = 0; j < KQ; ++j) nan |= S[i][j] != S[i][j];
+    if (T_ % TS_TB != 0 && __any(nan)) {
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      const int64_t c = (T_ - 1) / TS_CT;
+      for (int i = 0; i < RL; ++i)
+        if (v0 + i < V)
+          for (int j = 0; j < KQ; ++j) {
+            float s = stb[c * K * V + (int64_t)j * V + (st_off + i)];
+            for (int t = (int)c * TS_CT; t < T_; ++t) {
+              const int64_t tok = tok_first + (int64_t)t * H;
+              s = fmaf(r[tok * V + v0 + i], u[tok * K + p * KQ + j], s * expf(la[tok]));
+            }
+            hT[cb + (int64_t)j * V + i] = s;
+          }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < RL; ++i)
       if (v0 + i < V) {

@@ -179,3 +179,25 @@ def test_token_scan_split_backward(B, T, H, V, rows, K):
     print("[rel-L2] " + ", ".join(f"{n} {e:.1e}" for n, e in errs.items()), flush=True)
     for n, e in errs.items():
         assert e <= 1e-6, (n, e)
+
+
+@pytest.mark.parametrize("T", [1, 9, 12, 31])
+def test_infinite_state_at_a_ragged_end(T):
+    """A state that overflows at the last token is returned as it is, infinite where it overflowed, also where the
+    sequence ends inside a block of tokens (whose padding must not turn it into NaN)."""
+    B, H, K, V = 1, 2, 64, 40
+    banner(f"token scan infinite state T={T}")
+    q, k, u = (torch.zeros(B, T, H, K, device="cuda") for _ in range(3))
+    v, la = torch.zeros(B, T, H, V, device="cuda"), torch.zeros(B, T, H, device="cuda")
+    q[:, -1], u[:, -1, :, 0], v[:, -1] = 1.0, 4.0, 3e38
+    y, r, _, hT = ops.nsgdn_token_fwd(q, k, u, v, la, None, True)
+    assert torch.isinf(hT[:, :, 0]).all() and not hT[:, :, 1:].any()
+    assert torch.isinf(y[:, -1]).all() and (r[:, -1] == v[:, -1]).all()
+    if T > 8:  # beside the infinite rows (the first 16 are one workgroup's), ordinary ones keep their values
+        q, k, u, v0, la, _ = (t.cuda() for t in _inputs(B, T, H, K, V, seed=T))
+        ref = ops.nsgdn_token_fwd(q, k, u, v0, la, None, True)[3]
+        v = v0.clone()
+        v[:, -1, :, 5] = float("inf")
+        hT = ops.nsgdn_token_fwd(q, k, u, v, la, None, True)[3]
+        keep = [i for i in range(V) if i != 5]
+        assert torch.equal(hT[..., keep], ref[..., keep]) and torch.isinf(hT[..., 5]).all()
