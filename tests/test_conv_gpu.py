@@ -256,22 +256,27 @@ def test_conv_taps_rounded_to_activation_dtype():
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 def test_conv_backward_long_chunks_match_oracle(dtype):
-    """A large grid's backward without normalisation, over many chunks per sequence: a ragged last chunk (T = 4000 =
-    62 * 64 + 32 = 31 * 128 + 32), bias and conv state, against the oracle."""
-    B, T, D = 4, 4000, 2048
+    """A large grid's backward, whose waves take 128 tokens (8 of them per CU), over many chunks per sequence: a ragged
+    last chunk (T = 4000 = 31 * 128 + 32), bias and conv state, on the first and last channels (the convolution is
+    depthwise) against the oracle."""
+    B, T, D = 8, 4000, 2048
     waves_long = (D // 256) * B * -(-T // 128)
-    if waves_long < 4 * torch.cuda.get_device_properties(0).multi_processor_count:
+    if waves_long < 8 * torch.cuda.get_device_properties(0).multi_processor_count:
         pytest.skip("device has too many CUs for this grid to take the long-chunk backward")
+    # its partial rows, one per 128 tokens
+    assert _lib.conv_ws_bytes(B, T, D, W) == B * -(-T // 128) * (D * W + D) * 4
     banner(f"short conv backward, 128-token waves: B={B} T={T} D={D} {dtype}")
-    x, w, bias, state, dy = _inputs(B, T, D, dtype, 11, True, True)
-    dx, dw, db, dst = ops.short_conv_bwd(_dev(x, dtype), w.cuda(), _dev(bias, torch.float32), _dev(state, dtype),
-                                         _dev(dy, dtype), 0)
+    gen = torch.Generator("cuda").manual_seed(11)
+    r = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+    x, dy, state = r(B, T, D).to(dtype), r(B, T, D).to(dtype), r(B, D, W - 1).to(dtype)
+    w, bias = (r(D, W) * 0.5).to(dtype).float(), r(D) * 0.1
+    dx, dw, db, dst = ops.short_conv_bwd(x, w, bias, state, dy, 0)
     torch.cuda.synchronize()
-    dx_ref, dw_ref, db_ref, dst_ref = CO.short_conv_bwd(x, w, bias, state, dy, 0)
-    _check(dx, dx_ref, dtype, "dx")
-    _check(dw, dw_ref, dtype, "dw")
-    _check(db, db_ref, dtype, "dbias")
-    _check(dst, dst_ref, dtype, "dstate")
+    for cols in (slice(0, 64), slice(D - 64, D)):
+        ref = CO.short_conv_bwd(*(t.float().cpu() for t in (x[..., cols], w[cols], bias[cols], state[:, cols],
+                                                             dy[..., cols])), 0)
+        for n, a, b in zip(("dx", "dw", "dbias", "dstate"), (dx[..., cols], dw[cols], db[cols], dst[:, cols]), ref):
+            _check(a, b, dtype, n)
 
 
 @pytest.mark.parametrize("B,T,kd,vd,ng", [
