@@ -175,7 +175,8 @@ struct TokStage {
 // grid B * H * NB (NB = ceil(V / ROWS)) workgroups: workgroup x -> (b h, row block vb).  Tokens past the end of the
 // sequence in the last block are identity tokens (zero vectors, v = 0, la = 0), which leave a finite S as it is; nothing
 // is stored for them.
-template <int K, typename SH>
+// FIN: the final state is wanted (its epilogue in the other calls' kernel cost them 1%).
+template <int K, typename SH, bool FIN>
 __global__ __launch_bounds__(SH::THREADS) void token_scan_fwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ u, const float* __restrict__ v,
     const float* __restrict__ la, const float* __restrict__ h0, float* __restrict__ y, float* __restrict__ r,
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(SH::THREADS) void token_scan_fwd_kernel(
     if (t0 + 2 * TS_TB < T_) load_block(t0 + 2 * TS_TB);
     ts_barrier();  // the block's vectors read by every lane; the next block's staged
   }
-  if (hT) {
+  if constexpr (FIN) {
     // an infinite entry of S has become a NaN at the identity tokens (their S k is inf 0): such a wave steps from the last
     // checkpoint to the end again with the r it stored
     bool nan = false;
@@ -857,9 +858,12 @@ size_t token_scan_scratch_floats(int B, int T, int H, int K, int V) {
 template <int K, typename SH>
 static hipError_t token_scan_fwd_sh(const TokenScanArgs& a) {
   const int NB = (a.V + SH::ROWS - 1) / SH::ROWS, NCH = (a.T + TS_CT - 1) / TS_CT;
-  token_scan_fwd_kernel<K, SH><<<dim3((unsigned)(a.B * a.H * NB)), SH::THREADS, 0, a.stream>>>(
-      a.q, a.k, a.u, a.v, a.la, a.h0, a.y, a.r, a.st, a.hT, a.T, a.H, a.V, NCH, NB);
-  return hipGetLastError();
+  auto go = [&](auto kern) {
+    kern<<<dim3((unsigned)(a.B * a.H * NB)), SH::THREADS, 0, a.stream>>>(a.q, a.k, a.u, a.v, a.la, a.h0, a.y, a.r, a.st,
+                                                                        a.hT, a.T, a.H, a.V, NCH, NB);
+    return hipGetLastError();
+  };
+  return a.hT ? go(token_scan_fwd_kernel<K, SH, true>) : go(token_scan_fwd_kernel<K, SH, false>);
 }
 
 template <int K, typename SH>
