@@ -92,7 +92,10 @@ size_t chunk_ws_bytes(int B, int T, int H, int K, int V, int dtype, int parts, C
 // kernels that do not depend on the segments left out.  Measured at K = 128 in bf16, a sweep over c chunks takes about
 // 6 + 2.15 c (forward), 6 + 2.4 c (reverse) and 6 + 2.05 c (local reverse) with at most one 32-column workgroup per CU,
 // 6 + 2.9 c, 6 + 3.2 c and 6 + 2.7 c with one 64-column workgroup per CU, and the prefix pass (neither Q nor O) 6 + 1.65 c;
-// workgroups past one per CU run in further rounds.  A step of the scan takes 2.4 at K = 128 and 0.8 at K = 64.
+// workgroups past one per CU run in further rounds.  A step of the scan: 2.4 at K = 128 and 0.8 at K = 64 (now 1.6 and
+// 0.55; a cut moves by a chunk or none).  fp32 (twice the time a chunk) and K = 64 (two thirds) take the same figures:
+// whole and cut sweeps scale alike.  Over 2615 shapes (fp32 and bf16, K 64 and 128, V 64 to 256, 1 to 64 heads in batches
+// of 1 to 16, 16 to 200 chunks) no cut call is slower than the whole sweep, forward or training pair.
 static float segment_cost(int64_t BH, int NT, int K, int V, int ns, int cps) {
   const int64_t cus = device_cu_count();
   auto sweep = [&](int64_t wide, float narrow_us, float wide_us) {  // wide: workgroups of 64 columns
@@ -114,7 +117,8 @@ SegPlan segment_plan(int B, int T, int H, int K, int V) {
   const int64_t BH = (int64_t)B * H, wide = BH * (V / 64);
   SegPlan best{1, NT};
   // Measured (forward / training pair, us): B1 T6007 H8 K128 V256 206 / 471 unsegmented, 110 / 284 in 6 segments; B1
-  // T4096 H1 K128 V128 140 / 282, 63 / 136 in 11; B1 T2048 H16 K128 V256 78 / 203, 70 / 184 in 4 (86 / 220 in 2).
+  // T4096 H1 K128 V128 140 / 282, 60 / 129 in 11; B1 T2048 H16 K128 V256 80 / 207, 71 / 184 in 4.  fp32
+  // K64 V64 B1 T2048 H1 203 / 438, 48 / 113; bf16 K64 V128 B1 T2048 H1 61 / 126, 30 / 70.
   // at least four segments (with two or three the prefix pass, half or a third of a sweep, costs what the
   // parallelism gains) of at least four chunks, no more than the device sweeps at once; whole pairs of chunks, so
   // that a state kept for every second chunk is one of its segment's own

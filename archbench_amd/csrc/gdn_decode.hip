@@ -6,7 +6,7 @@
 // 7.2 us, 64 tokens 14.2 us, 128 tokens 22.6 us; the concatenation and three GEMMs 28.9 us at 8 and 36.7 us at 128 tokens (past which
 // they take over: two passes over the weights are then three).
 // One workgroup per 16 weight rows, its four waves taking every fourth 32-wide step of d, so that all of a row block's
-// loads are in flight at once (385 row blocks at d 1024 with 8 heads: one or two workgroups per CU, 8 KB in flight per
+// loads are in flight at once (386 row blocks at d 1024 with 8 heads: one or two workgroups per CU, 8 KB in flight per
 // wave); the four partial sums are added through LDS.  W rows are the A operand, tokens the B operand, so a lane ends
 // with four consecutive outputs of one token.
 #include <hip/hip_runtime.h>

@@ -249,11 +249,11 @@ struct WriteDirArgs {
 bool write_dir_supported(int K, int n_steps);
 hipError_t launch_write_dir(const WriteDirArgs& a, bool backward);
 
-// Exact fp32 token scan of the n-step family (gdn_tokenscan.hip)
 // out [H] = the sum over n >= 1 tokens of x [n, H], 1 <= H <= 256; part: head_sum_groups(n, H) * H doubles
 int head_sum_groups(int64_t n, int H);
 hipError_t launch_head_sum(const float* x, int64_t n, int H, double* part, float* out, hipStream_t stream);
 
+// Exact fp32 token scan of the n-step family (gdn_tokenscan.hip)
 struct TokenScanArgs {
   const float *q, *k, *u, *v, *la;  // [B, T, H, K] x3, [B, T, H, V], [B, T, H]
   const float* h0;                  // [B, H, K, V] or NULL (zero)
