@@ -122,8 +122,12 @@ def traffic(args) -> None:
         sums[tag] = per
     names = _keys(set(sums["fetch"]) | set(sums["write"]))
     sums = {tag: {names[k]: v for k, v in per.items()} for tag, per in sums.items()}
-    copy_f = sum(sum(v) for k, v in sums["fetch"].items() if k.split("@")[0] == "copy")
-    copy_w = sum(sum(v) for k, v in sums["write"].items() if k.split("@")[0] == "copy")
+
+    def last_copies(disp, ctr):  # the calibration copies end the run; the workload may make others before them
+        ids = sorted((i for i, (key, vals) in disp.items() if key[0] == "copy" and ctr in vals), key=int)
+        return sum(disp[i][1][ctr] for i in ids[-2:])
+
+    copy_f, copy_w = last_copies(fetch, "FETCH_SIZE"), last_copies(write, "WRITE_SIZE")
     if not copy_f or not copy_w:
         raise SystemExit("no calibration copy in the runs (run bench.py with --calibration-copy)")
     # KiB read / written by the two 256 MiB copies -> bytes per counter unit
