@@ -58,18 +58,18 @@ def _dx_split(rows: int, d: int, V: int) -> int:
     return max(S, 1)
 
 
-# Below this a call waits for its launches, not for its kernels: 250 us for about 25 torch and package calls from Python,
-# forward and backward (measured at N 128 to 1024, d 384 to 1024, V 8192).
-_HOST_US = 250
+# Below this a call that takes dx in parts and scales by the HIP pass waits for its launches, not for its kernels (measured
+# 314 to 330 us, at N 128 to 1024 and V 32000 and 50304; without the two 215 to 263, at V 8192).
+_HOST_US = 320
 
 
 def _outlasts_host(N: int, d: int, V: int) -> bool:
     """Whether a call's kernels take longer than its launches, so that extra calls which shorten them pay.  In us: dx's
     product in one part (its chain over V alone takes about 3.5 ns a class while the tiles leave CUs idle: V 8192, 32000
     and 50304 at 128 to 1024 rows 15 to 45, 97 to 175 and 146 to 242; in the parts of _dx_split 13 to 35, 28 to 91 and
-    35 to 118, for 25 us of the host), 6 N d V operations at 0.6 PFLOP/s, and the passes over W's size with torch's
-    scaling of its gradient.  Calls at V 8192, N 128 to 1024 (43 to 146 by this count): 215 to 252 us, with parts and the
-    HIP scaling 341 to 350; N 1024, d 512, V 32000 (345): 350 and 258; N 128, d 1024, V 50304 (448): 420 and 289."""
+    35 to 118), 6 N d V operations at 0.6 PFLOP/s, and the passes over W's size with torch's scaling of its gradient.
+    By this count and measured, without / with the two: N 128 to 1024 at V 8192 43 to 146, 252 / 345 us; N 210, d 768, V
+    32000 262, 278 / 318; N 1024, d 512, V 32000 345, 350 / 258 to 334; N 128, d 1024, V 50304 448, 420 / 289 to 324."""
     return 3.5e-3 * V + V * d * (1e-8 * N + 4e-6) > _HOST_US
 
 
@@ -94,10 +94,11 @@ def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None, N
 
 def _scaled(t: torch.Tensor, s: torch.Tensor, hip: bool) -> torch.Tensor:
     """s t for a 0-d s, the product in fp32 and rounded once.  The HIP pass (``hip``) runs at the copy rate, 41 us for 64M
-    bf16 elements where torch's mixed-type loop takes 163, but as an op it costs the host 20 us more in a backward."""
+    bf16 elements and 2.9 for 4M where torch's mixed-type loop takes 163 and 13.6, but as an op it costs the host 20 us
+    more in a backward."""
     if t.dtype not in (torch.bfloat16, torch.float32):  # an fp16 weight under autocast
         return t * s
-    if hip or torch.is_grad_enabled():
+    if hip and t.numel() >= 1 << 22 or torch.is_grad_enabled():
         return ops.scaled(t, s)
     # a 1-d s, which takes part in the type promotion: torch rounds a 0-d one to t's dtype first
     return torch.mul(t, s.reshape(1), out=torch.empty_like(t))

@@ -162,11 +162,11 @@ class _Calls(TorchDispatchMode):
         return func(*args, **(kwargs or {}))
 
 
-@pytest.mark.parametrize("N,H,V,parts", [(128, 384, 8192, False), (1024, 1024, 8192, False), (256, 512, 32000, False),
+@pytest.mark.parametrize("N,H,V,parts", [(128, 384, 8192, False), (1024, 1024, 8192, False), (210, 768, 32000, False),
                                          (128, 1024, 50304, True), (1024, 512, 32000, True)])
 def test_fused_linear_ce_one_pass_calls(N, H, V, parts):
     """A call that waits for its launches makes the fewest: three products, the loss and torch's scaling of both
-    gradients; one whose kernels outlast them takes dx in parts and the HIP scaling."""
+    gradients; one whose kernels outlast them takes dx in parts and the HIP scaling of the large gradient."""
     banner(f"fused linear CE one pass N={N} H={H} V={V}")
     gen = torch.Generator("cuda").manual_seed(N)
     x = torch.randn(1, N, H, device="cuda", generator=gen).bfloat16().requires_grad_()
@@ -175,7 +175,7 @@ def test_fused_linear_ce_one_pass_calls(N, H, V, parts):
     with _Calls() as calls:
         fused_ce.fused_linear_cross_entropy(x, t, w, num_chunks=1).backward()
     n = [sum(k in c for c in calls.names) for k in ("aten.mm", "aten.bmm", "archbench_amd", "aten.copy_", "aten.mul")]
-    assert n == ([2, 1, 4, 0, 0] if parts else [3, 0, 1, 0, 2]), calls.names
+    assert n == ([2, 1, 3, 0, 1] if parts else [3, 0, 1, 0, 2]), calls.names
 
 
 @pytest.mark.parametrize("hip", [False, True])
@@ -183,7 +183,7 @@ def test_fused_linear_ce_one_pass_calls(N, H, V, parts):
 def test_scaled_gradients(dtype, hip):
     """Both ways of scaling a stored gradient give the fp32 product rounded once, and differentiate under create_graph."""
     banner(f"scaled gradient {dtype} hip={hip}")
-    x = torch.randn(33, 8, device="cuda", generator=torch.Generator("cuda").manual_seed(7)).to(dtype)
+    x = torch.randn(4097, 1024, device="cuda", generator=torch.Generator("cuda").manual_seed(7)).to(dtype)
     s = torch.tensor(1 / 3, device="cuda", requires_grad=True)
     with torch.no_grad():
         assert torch.equal(fused_ce._scaled(x, s, hip), (x.float() * s).to(dtype))
