@@ -73,35 +73,38 @@ def _outlasts_host(N: int, d: int, V: int) -> bool:
     return 3.5e-3 * V + V * d * (1e-8 * N + 4e-6) > _HOST_US
 
 
-def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None, N: int) -> torch.Tensor:
-    """dlogits [rows, V] W [V, d] of a call with N rows, written to ``out`` if given."""
+def _dx(dlogits: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None, parts: bool) -> torch.Tensor:
+    """dlogits [rows, V] W [V, d], written to ``out`` if given; with ``parts`` in parts where that can be done."""
     rows, V = dlogits.shape
     d = weight.shape[1]
     # 16-byte rows throughout; not under an autocast that would change a dtype, nor into the gradient of an x laid out
     # feature by feature (dx has x's strides)
-    split = (dlogits.dtype == weight.dtype == torch.bfloat16 and d % 8 == 0 and weight.is_contiguous()
-             and (out is None or (out.dtype == torch.bfloat16 and out.is_contiguous())) and _outlasts_host(N, d, V))
-    S = _dx_split(rows, d, V) if split else 1
+    parts = (parts and dlogits.dtype == weight.dtype == torch.bfloat16 and d % 8 == 0 and weight.is_contiguous()
+             and (out is None or (out.dtype == torch.bfloat16 and out.is_contiguous())))
+    S = _dx_split(rows, d, V) if parts else 1
     if S == 1:
         return dlogits @ weight if out is None else out.copy_(dlogits @ weight)
     if out is None:
         out = dlogits.new_empty(rows, d)
-    parts = torch.bmm(dlogits.view(rows, S, V // S).transpose(0, 1), weight.view(S, V // S, d),
-                      out_dtype=torch.float32)
-    ops.sum_parts_(parts, out)
+    products = torch.bmm(dlogits.view(rows, S, V // S).transpose(0, 1), weight.view(S, V // S, d),
+                         out_dtype=torch.float32)
+    ops.sum_parts_(products, out)
     return out
 
 
 def _scaled(t: torch.Tensor, s: torch.Tensor, hip: bool) -> torch.Tensor:
     """s t for a 0-d s, the product in fp32 and rounded once.  The HIP pass (``hip``) runs at the copy rate, 41 us for 64M
-    bf16 elements and 2.9 for 4M where torch's mixed-type loop takes 163 and 13.6, but as an op it costs the host 20 us
-    more in a backward."""
+    bf16 elements and 2.9 for 4M where torch's product with a 0-d tensor takes 163 and 13.6 (with a 1-d one 19 for 25M,
+    HIP 15), but as an op it costs the host 20 us more in a backward."""
     if t.dtype not in (torch.bfloat16, torch.float32):  # an fp16 weight under autocast
         return t * s
     if hip and t.numel() >= 1 << 22 or torch.is_grad_enabled():
         return ops.scaled(t, s)
     # a 1-d s, which takes part in the type promotion: torch rounds a 0-d one to t's dtype first
-    return torch.mul(t, s.reshape(1), out=torch.empty_like(t))
+    try:
+        return torch.mul(t, s.reshape(1), out=torch.empty_like(t))
+    except RuntimeError:  # a batch of factors (is_grads_batched), which out= does not take; a second pass otherwise
+        return (t * s.reshape(1)).to(t.dtype)
 
 
 class _FusedLinearCE(torch.autograd.Function):
@@ -109,12 +112,13 @@ class _FusedLinearCE(torch.autograd.Function):
     def forward(ctx, x, target, weight, num_chunks: int, ignore_index: int):
         N, d = x.shape
         C = _rows_per_pass(N, num_chunks, d, x.element_size())
+        outlasts = ctx.outlasts_host = _outlasts_host(N, d, weight.shape[0])
         total = target.ne(ignore_index).sum().clamp_min(1)
         dloss = total.float().reciprocal().reshape(1)  # device scalar: no host sync
         if C >= N:
             logits = x @ weight.t()
             loss_rows = ops.cross_entropy_fwd_bwd_(logits, target, dloss, ignore_index)[0]
-            dx = _dx(logits, weight, None, N).to(x.dtype)
+            dx = _dx(logits, weight, None, outlasts).to(x.dtype)
             if num_chunks == 1 or logits.dtype == weight.dtype:
                 # dW needs no accumulation across passes, so the GEMM writes it in the weight's dtype directly (fp32
                 # accumulation inside, one rounding -- where several passes round at the end)
@@ -129,20 +133,19 @@ class _FusedLinearCE(torch.autograd.Function):
                 c_x = x[s:e]
                 logits = c_x @ weight.t()
                 loss_rows[s:e] = ops.cross_entropy_fwd_bwd_(logits, target[s:e], dloss, ignore_index)[0]
-                _dx(logits, weight, dx[s:e], N)
+                _dx(logits, weight, dx[s:e], outlasts)
                 if dw is None:
                     dw = torch.mm(logits.t(), c_x, out_dtype=torch.float32)
                 else:  # in place
                     torch.addmm(dw, logits.t(), c_x, out_dtype=torch.float32, out=dw)
                 del logits
         ctx.save_for_backward(dx, dw.to(weight.dtype))
-        ctx.outlasts_host = _outlasts_host(N, d, weight.shape[0])
         return loss_rows.sum() / total
 
     @staticmethod
     def backward(ctx, dout):
-        dx, dw = (_scaled(t, dout, ctx.outlasts_host) for t in ctx.saved_tensors)
-        return dx, None, dw, None, None
+        dx, dw = ctx.saved_tensors
+        return _scaled(dx, dout, ctx.outlasts_host), None, _scaled(dw, dout, ctx.outlasts_host), None, None
 
 
 def fused_linear_cross_entropy(x, target, weight, num_chunks: int = 8, ignore_index: int = -100):

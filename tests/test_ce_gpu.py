@@ -191,6 +191,24 @@ def test_scaled_gradients(dtype, hip):
     assert all(g is not None for g in torch.autograd.grad(y.float().sum(), (x, s)))
 
 
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("outlasts", [False, True])
+def test_fused_linear_ce_batched_gradients(monkeypatch, outlasts):
+    """Several gradients of the loss in one backward (is_grads_batched), however they are scaled."""
+    banner(f"fused linear CE batched gradients outlasts={outlasts}")
+    monkeypatch.setattr(fused_ce, "_outlasts_host", lambda *a: outlasts)
+    gen = torch.Generator("cuda").manual_seed(9)
+    x = torch.randn(1, 64, 512, device="cuda", generator=gen).bfloat16().requires_grad_()
+    w = (torch.randn(8192, 512, device="cuda", generator=gen) * 0.05).bfloat16().requires_grad_()
+    t = torch.randint(0, 8192, (1, 64), device="cuda", generator=gen)
+    loss = fused_ce.fused_linear_cross_entropy(x, t, w, num_chunks=1)
+    gs = torch.tensor([1.0, 0.5, 1 / 3], device="cuda")
+    got = torch.autograd.grad(loss, (x, w), gs, is_grads_batched=True, retain_graph=True)
+    for i, g in enumerate(gs):
+        for a, b in zip(got, torch.autograd.grad(loss, (x, w), g, retain_graph=True)):
+            assert torch.equal(a[i], b)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("n,S", [(1, 1), (8, 3), (1001, 2), (4096, 16)])
 def test_scale_and_sum_of_parts(dtype, n, S):
