@@ -823,14 +823,17 @@ def _(x, w_in, conv_w, conv_state, A_log, dt_bias, norm_group, beta_scale, g_min
 
 # The mixer's input stage in one op: q, k and v convolved straight out of the q/k/v input projection's output y
 # [B, T, 2 key_dim + value_dim] (its column groups, read in place, also where y is a column slice), with one weight
-# [2 key_dim + value_dim, W] for the three convolutions (q's rows, then k's, then v's), in one launch.  The backward, one
-# launch and the sum of its partial weight gradients, writes the three input gradients into the column groups of one dy and the weight gradients
-# into one dw, so no gradient of a split or of a concatenation costs a pass.
+# [2 key_dim + value_dim, W] for the three convolutions (q's rows, then k's, then v's), in one launch.  The backward,
+# one launch and the sum of its partial weight gradients, writes the three input gradients into the column groups of
+# one dy and the weight gradients into one dw, so no gradient of a split or of a concatenation costs a pass.
 def _stage_rows(y: Tensor) -> tuple[Tensor, int]:
     """y as (tensor, row stride); a stride past the kernels' 32-bit row offsets is copied away."""
+    B, T, D = y.shape
+    if y.is_contiguous():
+        return _arg(y), D
     rows, ld = _token_rows(y)
-    if y.shape[1] * ld * y.element_size() >= 1 << 31 and ld > y.shape[2]:
-        return _arg(y), y.shape[2]
+    if ld > D and T * ld * y.element_size() >= 1 << 31:
+        return _arg(y), D
     return rows, ld
 
 
